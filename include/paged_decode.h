@@ -282,6 +282,30 @@ int pd_store_kv_pages(const void* key, int64_t key_stride_b, int64_t key_stride_
                       int32_t table_width, const int64_t* positions, int32_t batch,
                       int32_t num_kv_heads, int32_t steps, int32_t head_dim, pd_stream_t stream);
 
+/* Causal prefill attention: new token t of a sequence attends to keys
+ * 0 .. nk - nq + t of it (nq new tokens, nk keys), in float32 up to the bf16
+ * output.  Strides are host arrays {batch, token, head} in elements,
+ * non-negative multiples of 8, tensors 16-byte aligned with a contiguous head.
+ *   packed   (cu_q, cu_k int32 [num_seqs + 1] on the device): sequence i owns
+ *            rows cu_q[i] .. cu_q[i+1] of q and out, [total_q, Hq, D], and rows
+ *            cu_k[i] .. of k and v, [total_k, Hkv, D]; batch strides unused;
+ *   paged    (packed, with a table): its keys are tokens 0 .. cu_k[i+1]-cu_k[i]
+ *            of pages table[i, t / page_size]; k and v [num_pages, page_size,
+ *            Hkv, D], page_size a multiple of 64 (of 32 at head_dim 256);
+ *   batched  (no cu): num_seqs sequences of seq_len new tokens and no prefix.
+ * Rows past total_q / total_k, pages outside [0, num_pages) and entries past
+ * table_width are never read (their keys and values are zeros).
+ * splits > 1 cuts the keys of every row into that many spans whose partials
+ * (part_o float32 [splits, total_q, Hq, D], part_ml [splits, total_q, Hq, 2])
+ * a second launch merges. */
+int pd_prefill(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+               const void* v, const int64_t* v_strides, void* out, const int64_t* out_strides,
+               const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs, int32_t seq_len,
+               int64_t total_q, int64_t total_k, const int32_t* table, int64_t table_stride_b,
+               int32_t table_width, int32_t page_size, int64_t num_pages, int32_t num_heads,
+               int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
+               float* part_o, float* part_ml, pd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

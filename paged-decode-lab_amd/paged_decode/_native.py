@@ -50,6 +50,8 @@ SIGNATURES = {
     "pd_store_kv": [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _vp],
     "pd_store_kv_pages": [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp, _i64,
                           _i32, _vp, _i32, _i32, _i32, _i32, _vp],
+    "pd_prefill": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp,
+                   _i64, _i32, _i32, _i64, _i32, _i32, _i32, _dbl, _i32, _vp, _vp, _vp],
 }
 
 _lib = None
@@ -239,3 +241,21 @@ def store_kv_pages(key, value, k_pages, v_pages, tables, positions):
                                   tables.shape[1],
                                   positions.data_ptr(), b, hkv, steps, d,
                                   stream_handle(key.device)))
+
+
+_Strides = _i64 * 3
+
+
+def prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu_k, num_seqs,
+            seq_len, total_q, total_k, tables, page_size, num_pages, heads, kv_heads, head_dim,
+            scale, splits, part_o, part_ml):
+    """pd_prefill; strides are (batch, token, head) in elements."""
+    check(lib().pd_prefill(
+        q.data_ptr(), _Strides(*q_strides), k.data_ptr(), _Strides(*k_strides), v.data_ptr(),
+        _Strides(*v_strides), out.data_ptr(), _Strides(*out_strides),
+        None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
+        num_seqs, seq_len, total_q, total_k, None if tables is None else tables.data_ptr(),
+        0 if tables is None else tables.stride(0), 0 if tables is None else tables.shape[1],
+        page_size, num_pages, heads, kv_heads, head_dim, scale, splits,
+        None if part_o is None else part_o.data_ptr(),
+        None if part_ml is None else part_ml.data_ptr(), stream_handle(q.device)))

@@ -10,9 +10,9 @@ ModelRunner.prepare_prefill / prepare_decode set, engine/model_runner.py:136-195
 * a decode step calls ``paged_decode`` on the layer's cache with the engine's block
   tables (-1 padded in eager mode) and context lengths, using the ``decode_backend`` and
   ``decode_resources`` that ``integration.configure_model`` attached;
-* prefill is not part of this operator: it runs a float32 PyTorch causal attention per
-  sequence (the overlay uses flash-attn's varlen kernel there, which does not exist for
-  this GPU), reading the cache through the block tables when a prefix is cached.
+* prefill runs causal attention over the packed sequences (``packed_prefill``, a HIP
+  kernel in the place of the overlay's flash-attn varlen call), reading the cache through
+  the block tables when a prefix is cached.
 
 ``decode_backend == "flash_attn"`` (the overlay's default before ``configure_model``)
 has no kernel on this platform and raises.
@@ -23,6 +23,7 @@ import torch
 from torch import nn
 
 from .kv_write import store_kvcache
+from .prefill import packed_prefill
 from .runtime import paged_decode
 
 
@@ -147,24 +148,7 @@ class Attention(nn.Module):
                             backend=self.decode_backend, scale=self.scale).unsqueeze(1)
 
     def _prefill(self, q, k, v, context):
-        cu_q = context.cu_seqlens_q.tolist()
-        cu_k = context.cu_seqlens_k.tolist()
-        group = self.num_heads // self.num_kv_heads
-        out = torch.empty_like(q)
-        for i in range(len(cu_q) - 1):
-            nq, nk = cu_q[i + 1] - cu_q[i], cu_k[i + 1] - cu_k[i]
-            if context.block_tables is None:
-                keys, vals = k[cu_k[i]:cu_k[i + 1]], v[cu_k[i]:cu_k[i + 1]]
-            else:  # prefix cache: the whole context is in the paged cache already
-                pos = torch.arange(nk, device=q.device)
-                blocks = context.block_tables[i, pos // self.k_cache.shape[1]].long()
-                keys = self.k_cache[blocks, pos % self.k_cache.shape[1]]
-                vals = self.v_cache[blocks, pos % self.k_cache.shape[1]]
-            qf = q[cu_q[i]:cu_q[i + 1]].float().transpose(0, 1)                   # [Hq, nq, D]
-            kf = keys.float().repeat_interleave(group, dim=1).transpose(0, 1)     # [Hq, nk, D]
-            vf = vals.float().repeat_interleave(group, dim=1).transpose(0, 1)
-            scores = torch.matmul(qf, kf.transpose(1, 2).contiguous()) * self.scale
-            qpos = torch.arange(nk - nq, nk, device=q.device)[:, None]
-            scores.masked_fill_(torch.arange(nk, device=q.device)[None, :] > qpos, float("-inf"))
-            out[cu_q[i]:cu_q[i + 1]] = torch.matmul(scores.softmax(-1), vf).transpose(0, 1).to(q.dtype)
-        return out
+        if context.block_tables is not None:  # prefix cache: the whole context is paged
+            k, v = self.k_cache, self.v_cache
+        return packed_prefill(q, k, v, context.cu_seqlens_q, context.cu_seqlens_k, self.scale,
+                              tables=context.block_tables, max_keys=context.max_seqlen_k)

@@ -24,9 +24,8 @@ Structure:
   the fed tokens, per-step logits and per-step timings.
 
 Differences from the reference, all outside the decode path: random weights
-from a config instead of a checkpoint (no tokenizer, so no decoded text);
-float32 PyTorch prefill attention instead of flash-attn (not available for this
-GPU); the float32 ``torch`` backend takes the place of the flash-attn decode peer.
+from a config instead of a checkpoint (no tokenizer, so no decoded text); a HIP
+prefill attention kernel instead of flash-attn's; the float32 ``torch`` backend takes the place of the flash-attn decode peer.
 """
 import dataclasses
 
@@ -38,6 +37,7 @@ from transformers.models.qwen3_5 import Qwen3_5ForCausalLM, Qwen3_5TextConfig
 
 from .kv_write import write_pages
 from .matched_splitkv import allocate_matched_resources, matched_decode
+from .prefill import batched_prefill
 from .runtime import allocate_resources, paged_decode
 from .spec import DecodeSpec
 
@@ -187,20 +187,6 @@ class HybridCache:
             layer.reset()
 
 
-def _prefill_attention(query, key, value, scaling):
-    """Causal GQA attention in float32 with contiguous operands; query [B, Hq, S, D] bf16,
-    returns [B, S, Hq, D]."""
-    s = query.shape[2]
-    group = query.shape[1] // key.shape[1]
-    q = query.float()
-    k = key.float().repeat_interleave(group, dim=1).transpose(-1, -2).contiguous()
-    v = value.float().repeat_interleave(group, dim=1).contiguous()
-    scores = torch.matmul(q, k) * scaling
-    future = torch.ones(s, s, dtype=torch.bool, device=query.device).triu(1)
-    probs = scores.masked_fill(future, float("-inf")).softmax(-1)
-    return torch.matmul(probs, v).transpose(1, 2).to(query.dtype)
-
-
 def _dense_decode(q, k_pages, v_pages, tables, lengths, scaling):
     """float32 decode over the gathered pages (reads lengths on the host)."""
     out = torch.zeros_like(q)
@@ -225,7 +211,7 @@ def _attention(module, query, key, value, attention_mask, scaling, dropout=0.0, 
     runner = module.paged_decode_session
     cache = runner.cache
     if cache.phase == "prefill":
-        return _prefill_attention(query, key, value, scaling), None
+        return batched_prefill(query, key, value, scaling), None
     q = query.squeeze(2)
     pool = cache.pool
     k, v = pool.pages(module.layer_idx)

@@ -1,0 +1,152 @@
+"""GPU parity of the prefill attention kernel (pd_prefill) with attention in 64 bits.
+
+The gate is derived per output: half a bf16 ulp, plus what float32 leaves in the scores
+(a dot product of D terms) and in the sums over the keys (and their three bf16 terms).
+"""
+import numpy as np
+import pytest
+import torch
+
+if not torch.cuda.is_available():
+    pytest.skip("needs an MI355X GPU", allow_module_level=True)
+
+from paged_decode import prefill as PF
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+def rows(gen, *shape):
+    return torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+
+
+def check(out, q, k, v, first, scale, where):
+    """out/q [n, Hq, D] at positions first.. against keys k, v [m, Hkv, D]."""
+    n, hq, d = q.shape
+    m, group = k.shape[0], hq // k.shape[1]
+    q64, k64, v64 = (t.double().cpu().transpose(0, 1) for t in (q, k, v))
+    k64, v64 = k64.repeat_interleave(group, 0), v64.repeat_interleave(group, 0)
+    masked = torch.arange(m)[None, :] > first + torch.arange(n)[:, None]
+    s = (torch.matmul(q64, k64.transpose(1, 2)) * scale).masked_fill(masked, float("-inf"))
+    p = s.softmax(-1)
+    ref = torch.matmul(p, v64)
+    spread = torch.matmul(p, v64.abs())
+    size = torch.matmul(q64.abs(), k64.abs().transpose(1, 2)).amax(-1, keepdim=True) * abs(scale)
+    # half an ulp of 8 significant bits is at most 2^-8 of the value
+    bound = 2.0 ** -8 * ref.abs() + (2 * (d + 4) * size + m + 16) * 2 * EPS * spread
+    diff = (out.double().cpu().transpose(0, 1) - ref).abs()
+    worst = (diff / (bound + 1e-30)).max()
+    assert worst <= 1, (where, float(worst), float(diff.max()))
+
+
+def packed(lens, prefix, hq, hkv, d, page, seed, scale=None, splits=None, monkeypatch=None):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    if splits:
+        monkeypatch.setattr(PF, "_splits", lambda *a: splits)
+    total = [n + prefix for n in lens]
+    cu = lambda ns: torch.tensor(np.cumsum([0] + ns), dtype=torch.int32, device="cuda")  # noqa: E731
+    q = rows(gen, sum(lens), hq, d)
+    # keys and values as slices of one fused row, like a model's projection
+    kv = rows(gen, sum(total), 2 * hkv, d)
+    k, v = kv[:, :hkv], kv[:, hkv:]
+    scale = d ** -0.5 if scale is None else scale
+    if page:
+        width = max(-(-n // page) for n in total)
+        blocks = sum(-(-n // page) for n in total) + 1
+        order = list(np.random.default_rng(seed).permutation(blocks))
+        cache = torch.full((2, blocks, page, hkv, d), float("nan"), device="cuda",
+                           dtype=torch.bfloat16)
+        tables = torch.full((len(lens), width), -1, dtype=torch.int32)
+        at = 0
+        for i, n in enumerate(total):
+            for j in range(0, n, page):
+                b = int(order.pop())
+                tables[i, j // page] = b
+                take = min(page, n - j)
+                cache[0, b, :take], cache[1, b, :take] = k[at + j:at + j + take], v[at + j:at + j + take]
+            at += n
+        args = (q, cache[0], cache[1], cu(lens), cu(total), scale)
+        kwargs = dict(tables=tables.cuda(), max_keys=max(total))
+    else:
+        args, kwargs = (q, k, v, cu(lens), cu(total), scale), dict(max_keys=max(total))
+    assert PF._packed_ok(args[0], args[1], args[2], torch.empty_like(q), args[3], args[4], scale,
+                         kwargs.get("tables"))
+    out = PF.packed_prefill(*args, **kwargs)
+    a = b = 0
+    for n, m in zip(lens, total):
+        if n:
+            check(out[a:a + n], q[a:a + n], k[b:b + m], v[b:b + m], prefix, scale, (n, m))
+        a, b = a + n, b + m
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 256), (8, 2, 128), (4, 4, 64), (6, 2, 128), (16, 1, 64)])
+@pytest.mark.parametrize("lens,prefix", [([1], 0), ([31, 1, 65], 0), ([127, 129, 2], 0), ([300, 33], 0),
+                                         ([1, 70], 64), ([40], 1000)])
+def test_packed_rows(hq, hkv, d, lens, prefix):
+    packed(lens, prefix, hq, hkv, d, None, sum(lens) + d)
+
+
+@pytest.mark.parametrize("hq,hkv,d,page", [(8, 2, 256, 256), (8, 2, 256, 32), (8, 8, 128, 64),
+                                           (4, 1, 64, 256)])
+@pytest.mark.parametrize("lens,prefix", [([1, 5, 257], 0), ([64, 31], 256), ([3], 700)])
+def test_paged_keys_with_nan_beyond_the_live_rows(hq, hkv, d, page, lens, prefix):
+    packed(lens, prefix, hq, hkv, d, page, sum(lens) + page)
+
+
+@pytest.mark.parametrize("splits", [2, 3, 8])
+@pytest.mark.parametrize("d,page", [(256, 256), (128, None), (64, 256)])
+def test_split_keys(monkeypatch, splits, d, page):
+    packed([200, 1, 33], 130, 8, 2, d, page, splits, splits=splits, monkeypatch=monkeypatch)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.09, 1.0, 3.0])
+def test_scales(scale):
+    packed([150], 20, 4, 2, 128, None, 7, scale=scale)
+
+
+def test_more_than_a_wavefront_of_sequences():
+    packed([(5 * i) % 23 for i in range(140)], 3, 4, 2, 64, None, 9)
+
+
+@pytest.mark.parametrize("b,hq,hkv,s,d", [(1, 8, 2, 513, 256), (3, 8, 2, 65, 256), (2, 4, 4, 200, 128)])
+def test_batched(b, hq, hkv, s, d):
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    q = rows(gen, b, s, hq, d).transpose(1, 2)
+    k = rows(gen, b, s, hkv, d).transpose(1, 2)
+    v = rows(gen, b, s, hkv, d).transpose(1, 2)
+    assert PF._batched_ok(q, k, v, d ** -0.5)
+    out = PF.batched_prefill(q, k, v, d ** -0.5)
+    for i in range(b):
+        check(out[i], q[i].transpose(0, 1), k[i].transpose(0, 1), v[i].transpose(0, 1), 0,
+              d ** -0.5, i)
+
+
+@pytest.mark.parametrize("special", ["v_inf", "k_inf", "q_nan"])
+def test_infinities_and_nans_as_in_float32(special):
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = rows(gen, 1, 2, 70, 128), rows(gen, 1, 2, 70, 128), rows(gen, 1, 2, 70, 128)
+    if special == "v_inf":
+        v[0, 0, 0, 5], v[0, 1, 0, 7] = float("inf"), float("-inf")
+    elif special == "k_inf":
+        k[0, 0, 0, 3] = float("inf")
+    else:
+        q[0, 1, 40, 9] = float("nan")
+    out = PF.batched_prefill(q, k, v, 0.1).float()
+    ref = PF._batched_torch(q, k, v, 0.1).float()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    ok = ref.isfinite()
+    assert (out[ok] - ref[ok]).abs().max() < 2.0 ** -6
+    assert torch.equal(out[ref.isinf()], ref[ref.isinf()])
+
+
+def test_general_form_serves_what_the_kernel_does_not():
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    q, k, v = (rows(gen, 37, 4, 80) for _ in range(3))
+    cu = torch.tensor([0, 20, 37], dtype=torch.int64, device="cuda")
+    out = PF.packed_prefill(q, k, v, cu, cu, 0.1)
+    for a, b in ((0, 20), (20, 37)):
+        check(out[a:b], q[a:b], k[a:b], v[a:b], 0, 0.1, a)
+    x = torch.randn(9, 2, 64, requires_grad=True)
+    cu = torch.tensor([0, 9], dtype=torch.int32)
+    PF.packed_prefill(x, x, x, cu, cu, 0.1).sum().backward()
+    assert x.grad.abs().sum() > 0
