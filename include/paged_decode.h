@@ -306,6 +306,57 @@ int pd_prefill(const void* q, const int64_t* q_strides, const void* k, const int
                int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
                float* part_o, float* part_ml, pd_stream_t stream);
 
+/* The decoder layer between its matrix products.  bf16 tensors are contiguous
+ * and 16-byte aligned unless strides are given; arithmetic is float32. */
+
+/* x [rows, dim] += y (y may be null), out = x rms(x)^-1 (1 + weight). */
+int pd_add_rms_norm(void* x, const void* y, const void* weight, void* out, int64_t rows,
+                    int32_t dim, double eps, pd_stream_t stream);
+
+/* out = o rms(o)^-1 weight silu(z) per row of dim (64 or 128); o float32. */
+int pd_gated_norm(const float* o, const void* z, const void* weight, void* out, int64_t rows,
+                  int32_t dim, double eps, pd_stream_t stream);
+
+/* out = silu(gate) up; out may be gate. */
+int pd_silu_mul(const void* gate, const void* up, void* out, int64_t elems, pd_stream_t stream);
+
+/* out = x sigmoid(gate), gate's rows gate_stride elements apart. */
+int pd_sigmoid_gate(const void* x, const void* gate, int64_t gate_stride, void* out, int64_t rows,
+                    int32_t cols, pd_stream_t stream);
+
+/* Gated delta rule inputs of x [batch, steps, C], C = 2 hk dk + hv dv channels
+ * (queries, keys, values): causal convolution with taps [C, 4], silu, unit
+ * query (times dk^-1/2) and key heads -> act float32 [batch, steps, C]; decay
+ * = exp(-exp(a_log) softplus(a + dt_bias)) and sigmoid(b) -> gates float32
+ * [batch, steps, hv, 2].  conv_state [batch, C, 4] receives the last four
+ * inputs; with has_prev (at most 16 steps) it holds the four before them. */
+int pd_conv_gates(const void* x, const void* taps, const void* a, const void* b, const void* a_log,
+                  const void* dt_bias, void* conv_state, float* act, float* gates, int32_t batch,
+                  int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t has_prev,
+                  pd_stream_t stream);
+
+/* S = decay S; S += k (beta (v - S^T k))^T; out = S^T q per value head and
+ * token; state float32 [batch, hv, dk, dv], read with has_prev, written;
+ * out float32 [batch, steps, hv, dv]; lanes per state column 16 or 32. */
+int pd_delta_rule(const float* act, const float* gates, float* state, float* out, int32_t batch,
+                  int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t has_prev,
+                  int32_t lanes, pd_stream_t stream);
+
+/* table float32 [steps, half, 2]: cos and sin of positions x inv_freq. */
+int pd_rope_table(const int64_t* positions, const void* inv_freq, int32_t is_bf16, float* table,
+                  int32_t steps, int32_t half, pd_stream_t stream);
+
+/* Query and key heads normed (weights as 1 + w) and rotated (2 half leading
+ * elements), keys and values written to their page slots as
+ * pd_store_kv_pages does.  q [batch, steps, Hq, 2, D] (query, gate), k and v
+ * [batch, steps, Hkv, D] -> q_out [batch, steps, Hq, D], k_out (may be null). */
+int pd_qk_rope(const void* q, const void* k, const void* v, const void* q_weight,
+               const void* k_weight, const float* rope, void* q_out, void* k_out, void* k_pages,
+               void* v_pages, int64_t num_pages, const int32_t* table, int64_t table_stride_b,
+               int32_t table_width, const int64_t* positions, int32_t batch, int32_t steps,
+               int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t half, double eps,
+               pd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -52,6 +52,16 @@ SIGNATURES = {
                           _i32, _vp, _i32, _i32, _i32, _i32, _vp],
     "pd_prefill": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp,
                    _i64, _i32, _i32, _i64, _i32, _i32, _i32, _dbl, _i32, _vp, _vp, _vp],
+    "pd_add_rms_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
+    "pd_gated_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
+    "pd_silu_mul": [_vp, _vp, _vp, _i64, _vp],
+    "pd_sigmoid_gate": [_vp, _vp, _i64, _vp, _i64, _i32, _vp],
+    "pd_conv_gates": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32,
+                      _i32, _i32, _vp],
+    "pd_delta_rule": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp],
+    "pd_rope_table": [_vp, _vp, _i32, _vp, _i32, _i32, _vp],
+    "pd_qk_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp,
+                   _i32, _i32, _i32, _i32, _i32, _i32, _dbl, _vp],
 }
 
 _lib = None
@@ -259,3 +269,58 @@ def prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu
         page_size, num_pages, heads, kv_heads, head_dim, scale, splits,
         None if part_o is None else part_o.data_ptr(),
         None if part_ml is None else part_ml.data_ptr(), stream_handle(q.device)))
+
+
+def add_rms_norm(x, y, weight, out, eps):
+    """x [N, H] += y (or y None), out = x rms(x)^-1 (1 + weight)."""
+    check(lib().pd_add_rms_norm(x.data_ptr(), None if y is None else y.data_ptr(),
+                                weight.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], eps,
+                                stream_handle(x.device)))
+
+
+def gated_norm(o, z, weight, out, rows, dim, eps):
+    """out = o rms(o)^-1 weight silu(z) over `rows` rows of `dim`; o float32."""
+    check(lib().pd_gated_norm(o.data_ptr(), z.data_ptr(), weight.data_ptr(), out.data_ptr(), rows,
+                              dim, eps, stream_handle(o.device)))
+
+
+def silu_mul(gate, up, out):
+    check(lib().pd_silu_mul(gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.numel(),
+                            stream_handle(gate.device)))
+
+
+def sigmoid_gate(x, gate, out, rows, cols):
+    """out = x sigmoid(gate), x and out [rows, cols], gate's rows gate.stride(0) apart."""
+    check(lib().pd_sigmoid_gate(x.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(), rows,
+                                cols, stream_handle(x.device)))
+
+
+def conv_gates(x, taps, a, b, a_log, dt_bias, conv_state, act, gates, batch, steps, hk, hv, dk, dv,
+               has_prev):
+    check(lib().pd_conv_gates(x.data_ptr(), taps.data_ptr(), a.data_ptr(), b.data_ptr(),
+                              a_log.data_ptr(), dt_bias.data_ptr(), conv_state.data_ptr(),
+                              act.data_ptr(), gates.data_ptr(), batch, steps, hk, hv, dk, dv,
+                              int(has_prev), stream_handle(x.device)))
+
+
+def delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, has_prev, lanes):
+    check(lib().pd_delta_rule(act.data_ptr(), gates.data_ptr(), state.data_ptr(), out.data_ptr(),
+                              batch, steps, hk, hv, dk, dv, int(has_prev), lanes,
+                              stream_handle(act.device)))
+
+
+def rope_table(positions, inv_freq, table):
+    """table float32 [steps, half, 2] = (cos, sin) of positions x inv_freq (bf16 or float32)."""
+    check(lib().pd_rope_table(positions.data_ptr(), inv_freq.data_ptr(),
+                              int(inv_freq.dtype == torch.bfloat16), table.data_ptr(),
+                              table.shape[0], table.shape[1], stream_handle(table.device)))
+
+
+def qk_rope(q, k, v, q_weight, k_weight, rope, q_out, k_out, k_pages, v_pages, tables, positions,
+            batch, steps, hq, hkv, d, half, eps):
+    check(lib().pd_qk_rope(q.data_ptr(), k.data_ptr(), v.data_ptr(), q_weight.data_ptr(),
+                           k_weight.data_ptr(), rope.data_ptr(), q_out.data_ptr(),
+                           None if k_out is None else k_out.data_ptr(), k_pages.data_ptr(),
+                           v_pages.data_ptr(), k_pages.shape[0], tables.data_ptr(),
+                           tables.stride(0), tables.shape[1], positions.data_ptr(), batch, steps,
+                           hq, hkv, d, half, eps, stream_handle(q.device)))

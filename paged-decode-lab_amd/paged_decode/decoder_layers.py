@@ -1,0 +1,283 @@
+"""The decoder's layers on this library's kernels.
+
+``decoder_weights`` reads the model's modules and says whether every one of them is the
+plain form the kernels compute; ``decoder_forward`` is then one forward of the model, with
+the residual stream, the norms, the gated delta rule, rotary embedding, the K/V write and
+the gates in HIP kernels between the matrix products.  A model that was changed (hooks,
+replaced or compiled modules, biases, other dtypes or sizes) keeps transformers' modules:
+the weights are read from the modules on every forward, nothing is kept of them.
+"""
+from dataclasses import dataclass
+
+import torch
+import torch.nn.functional as F
+from torch import nn
+from transformers.activations import SiLUActivation
+from transformers.models.qwen3_5 import modeling_qwen3_5 as qwen
+
+from . import _native
+from .prefill import batched_prefill
+
+MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
+
+
+def _plain_module(module, kind):
+    """`module` runs the forward its class defines and nothing else."""
+    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+            and "forward" not in module.__dict__ and module._compiled_call_impl is None
+            and not module.training)
+
+
+def _tensor(module, name, device, shape):
+    t = module._parameters.get(name)
+    if (t is None or type(t) not in (nn.Parameter, torch.Tensor) or t.dtype != torch.bfloat16
+            or t.device != device or t.shape != shape or not t.is_contiguous()
+            or t.data_ptr() % 16):
+        return None
+    return t
+
+
+class _Reader:
+    """Collects the weights of plain modules; ``ok`` turns false at the first other one."""
+
+    def __init__(self, device):
+        self.device, self.ok = device, True
+
+    def module(self, parent, name, kind):
+        module = parent._modules.get(name)
+        self.ok = self.ok and module is not None and _plain_module(module, kind)
+        return module
+
+    def weight(self, module, shape, name="weight"):
+        t = _tensor(module, name, self.device, shape) if self.ok else None
+        self.ok = self.ok and t is not None
+        return t
+
+    def linear(self, parent, name, rows, cols):
+        module = self.module(parent, name, nn.Linear)
+        if self.ok and module._parameters.get("bias") is not None:
+            self.ok = False
+        return self.weight(module, (rows, cols))
+
+    def norm(self, parent, name, dim, kind=qwen.Qwen3_5RMSNorm):
+        module = self.module(parent, name, kind)
+        if not self.ok:
+            return None, 0.0
+        return self.weight(module, (dim,)), float(
+            module.variance_epsilon if kind is qwen.Qwen3_5RMSNormGated else module.eps)
+
+
+@dataclass
+class LayerWeights:
+    index: int
+    module: object          # the attention module of a full-attention layer, else None
+    mixer: tuple
+    in_norm: tuple
+    post_norm: tuple
+    gate: torch.Tensor
+    up: torch.Tensor
+    down: torch.Tensor
+
+
+@dataclass
+class DecoderWeights:
+    layers: list
+    norm: tuple
+    head: torch.Tensor
+    inv_freq: torch.Tensor
+    half: int               # rotated pairs per head
+    linear: tuple           # (key heads, value heads, key dim, value dim)
+
+
+def _linear_mixer(read, layer, cfg):
+    hk, hv = cfg.linear_num_key_heads, cfg.linear_num_value_heads
+    dk, dv, hid = cfg.linear_key_head_dim, cfg.linear_value_head_dim, cfg.hidden_size
+    m = read.module(layer, "linear_attn", qwen.Qwen3_5GatedDeltaNet)
+    if (not read.ok or (m.num_k_heads, m.num_v_heads, m.head_k_dim, m.head_v_dim) != (hk, hv, dk, dv)
+            or m.conv_kernel_size != 4 or m.activation != "silu"):
+        read.ok = False
+        return None
+    channels = 2 * hk * dk + hv * dv
+    conv = read.module(m, "conv1d", nn.Conv1d)
+    if read.ok and (conv._parameters.get("bias") is not None or conv.groups != channels
+                    or conv.kernel_size != (4,) or conv.stride != (1,) or conv.dilation != (1,)
+                    or conv.padding != (3,) or conv.padding_mode != "zeros"):
+        read.ok = False
+    return (read.linear(m, "in_proj_qkv", channels, hid), read.linear(m, "in_proj_z", hv * dv, hid),
+            read.linear(m, "in_proj_b", hv, hid), read.linear(m, "in_proj_a", hv, hid),
+            read.weight(conv, (channels, 1, 4)), read.weight(m, (hv,), "A_log"),
+            read.weight(m, (hv,), "dt_bias"), read.norm(m, "norm", dv, qwen.Qwen3_5RMSNormGated),
+            read.linear(m, "out_proj", hid, hv * dv))
+
+
+def _full_mixer(read, layer, cfg):
+    hq, hkv, d, hid = (cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim,
+                       cfg.hidden_size)
+    m = read.module(layer, "self_attn", qwen.Qwen3_5Attention)
+    if not read.ok or m.head_dim != d:
+        read.ok = False
+        return None
+    mixer = (read.linear(m, "q_proj", 2 * hq * d, hid), read.linear(m, "k_proj", hkv * d, hid),
+             read.linear(m, "v_proj", hkv * d, hid), read.norm(m, "q_norm", d),
+             read.norm(m, "k_norm", d), read.linear(m, "o_proj", hid, hq * d))
+    if read.ok and mixer[3][1] != mixer[4][1]:
+        read.ok = False
+    return mixer
+
+
+def decoder_weights(model, device):
+    """The model's weights, or None when the kernels do not cover it as it is."""
+    text, cfg = model.model, model.model.config
+    hooks = nn.modules.module
+    read = _Reader(device)
+    if hooks._global_forward_hooks or hooks._global_forward_pre_hooks:
+        return None
+    hk, hv = cfg.linear_num_key_heads, cfg.linear_num_value_heads
+    dk, dv, hid, mid = (cfg.linear_key_head_dim, cfg.linear_value_head_dim, cfg.hidden_size,
+                        cfg.intermediate_size)
+    if (cfg._attn_implementation != "paged_decode_lab_hip" or hid % 8 or hid > MAX_HIDDEN or mid % 8
+            or dk not in (64, 128) or dv not in (64, 128) or hk < 1 or hv % hk
+            or cfg.head_dim not in (64, 128, 256)):
+        return None
+    embed = read.module(text, "embed_tokens", nn.Embedding)
+    rope = read.module(text, "rotary_emb", qwen.Qwen3_5TextRotaryEmbedding)
+    if not read.ok or read.weight(embed, (cfg.vocab_size, hid)) is None:
+        return None
+    inv = rope._buffers.get("inv_freq")
+    if (rope.rope_type != "default" or rope.attention_scaling != 1.0 or inv is None
+            or inv.dtype not in (torch.bfloat16, torch.float32) or inv.device != device
+            or inv.dim() != 1 or not inv.is_contiguous() or not 0 < 2 * inv.shape[0] <= cfg.head_dim):
+        return None
+    layers = []
+    for i, layer in enumerate(text.layers):
+        full = cfg.layer_types[i] == "full_attention"
+        if not _plain_module(layer, qwen.Qwen3_5DecoderLayer):
+            return None
+        mixer = _full_mixer(read, layer, cfg) if full else _linear_mixer(read, layer, cfg)
+        mlp = read.module(layer, "mlp", qwen.Qwen3_5MLP)
+        if not read.ok:
+            return None
+        read.module(mlp, "act_fn", SiLUActivation)
+        layers.append(LayerWeights(
+            i, layer._modules["self_attn"] if full else None, mixer,
+            read.norm(layer, "input_layernorm", hid),
+            read.norm(layer, "post_attention_layernorm", hid), read.linear(mlp, "gate_proj", mid, hid),
+            read.linear(mlp, "up_proj", mid, hid), read.linear(mlp, "down_proj", hid, mid)))
+        if not read.ok:
+            return None
+    weights = DecoderWeights(layers, read.norm(text, "norm", hid),
+                             read.linear(model, "lm_head", cfg.vocab_size, hid), inv, inv.shape[0],
+                             (hk, hv, dk, dv))
+    return weights if read.ok else None
+
+
+def _linear_states(cache, index, batch, weights, device):
+    """(conv state, recurrent state, whether they hold earlier tokens) of one layer, made
+    through the cache's own protocol on first use; None when they have another form."""
+    hk, hv, dk, dv = weights.linear
+    layer, channels = cache.linear[index], 2 * hk * dk + hv * dv
+    held = cache.has_previous_state(index)
+    if layer.conv_states.get(0) is None or layer.recurrent_states.get(0) is None:
+        cache.update_conv_state(torch.zeros((batch, channels, 4), device=device,
+                                            dtype=torch.bfloat16), index)
+        cache.update_recurrent_state(torch.zeros((batch, hv, dk, dv), device=device,
+                                                 dtype=torch.float32), index)
+        held = False
+    conv, state = layer.conv_states[0], layer.recurrent_states[0]
+    if (conv.shape != (batch, channels, 4) or conv.dtype != torch.bfloat16
+            or state.shape != (batch, hv, dk, dv) or state.dtype != torch.float32
+            or not conv.is_contiguous() or not state.is_contiguous()
+            or conv.data_ptr() % 16 or state.data_ptr() % 16):
+        return None
+    return conv, state, held
+
+
+def decoder_states(runner, weights, steps):
+    """The linear-attention states of every layer, or None where the kernels cannot run:
+    several steps on top of earlier tokens, or states of another form."""
+    cache, found = runner.cache, {}
+    for index in cache.linear:
+        states = _linear_states(cache, index, runner.batch, weights, runner.device)
+        if states is None or (states[2] and steps > 1):
+            return None
+        found[index] = states
+    return found
+
+
+def _delta_lanes(columns, dk, device):
+    """Lanes per state column: 32 halve the chain of a token where the columns leave the
+    SIMDs idle, 16 take less work in all."""
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    return 32 if dk == 128 and columns <= 8 * cus else 16
+
+
+def _linear_attention(h, w, weights, states, batch, steps):
+    hk, hv, dk, dv = weights.linear
+    qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
+    conv, state, held = states
+    mixed, gate = F.linear(h, qkv), F.linear(h, z)
+    beta, decay = F.linear(h, b), F.linear(h, a)
+    rows = batch * steps
+    act = torch.empty((rows, mixed.shape[1]), device=h.device, dtype=torch.float32)
+    gates = torch.empty((rows, hv, 2), device=h.device, dtype=torch.float32)
+    _native.conv_gates(mixed, taps, decay, beta, a_log, dt_bias, conv, act, gates, batch, steps,
+                       hk, hv, dk, dv, held)
+    out = torch.empty((rows, hv * dv), device=h.device, dtype=torch.float32)
+    _native.delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, held,
+                       _delta_lanes(batch * hv * dv, dk, h.device))
+    y = torch.empty((rows, hv * dv), device=h.device, dtype=torch.bfloat16)
+    _native.gated_norm(out, gate, norm, y, rows * hv, dv, eps)
+    return F.linear(y, out_proj)
+
+
+def _full_attention(h, w, weights, rope, runner, batch, steps, attend):
+    spec, pool = runner.spec, runner.cache.pool
+    hq, hkv, d = spec.num_heads, spec.num_kv_heads, spec.head_dim
+    q_proj, k_proj, v_proj, (q_norm, eps), (k_norm, _), o_proj = w.mixer
+    q, k, v = F.linear(h, q_proj), F.linear(h, k_proj), F.linear(h, v_proj)
+    fill = runner.cache.phase == "prefill"
+    query = torch.empty((batch, steps, hq, d), device=h.device, dtype=torch.bfloat16)
+    keys = torch.empty((batch, steps, hkv, d), device=h.device, dtype=torch.bfloat16) if fill else None
+    k_pages, v_pages = pool.pages(w.index)
+    _native.qk_rope(q, k, v, q_norm, k_norm, rope, query, keys, k_pages, v_pages, pool.tables,
+                    pool.positions, batch, steps, hq, hkv, d, weights.half, eps)
+    if fill:
+        out = batched_prefill(query.transpose(1, 2), keys.transpose(1, 2),
+                              v.view(batch, steps, hkv, d).transpose(1, 2), w.module.scaling)
+    else:
+        out = attend(runner, w.module, query.view(batch, hq, d), k_pages, v_pages)
+    y = torch.empty((batch * steps, hq * d), device=h.device, dtype=torch.bfloat16)
+    _native.sigmoid_gate(out, q.view(-1, 2 * d)[:, d:], y, batch * steps * hq, d)
+    return F.linear(y, o_proj)
+
+
+def decoder_forward(runner, weights, states, tokens, positions, attend):
+    """Logits of the last token; as HybridRunner._forward, on the kernels.  ``attend`` is
+    the decode attention of one layer over its pages."""
+    model, text = runner.model, runner.text
+    batch, steps = tokens.shape
+    runner.cache.pool.begin_step(positions)
+    x = text.embed_tokens(tokens)
+    rows, hid = batch * steps, x.shape[-1]
+    x = x.view(rows, hid)
+    rope = torch.empty((steps, weights.half, 2), device=x.device, dtype=torch.float32)
+    _native.rope_table(positions, weights.inv_freq, rope)
+    y = None
+    for w in weights.layers:
+        h = torch.empty_like(x)
+        _native.add_rms_norm(x, y, w.in_norm[0], h, w.in_norm[1])
+        if w.module is None:
+            y = _linear_attention(h, w, weights, states[w.index], batch, steps)
+            runner.cache.linear[w.index].has_previous_state[0] = True
+        else:
+            y = _full_attention(h, w, weights, rope, runner, batch, steps, attend)
+        _native.add_rms_norm(x, y, w.post_norm[0], h, w.post_norm[1])
+        gate, up = F.linear(h, w.gate), F.linear(h, w.up)
+        _native.silu_mul(gate, up, gate)
+        y = F.linear(gate, w.down)
+    if steps > 1:
+        x = x.view(batch, steps, hid)[:, -1].contiguous()
+        y = y.view(batch, steps, hid)[:, -1].contiguous()
+    h = torch.empty_like(x)
+    _native.add_rms_norm(x, y, weights.norm[0], h, weights.norm[1])
+    return F.linear(h, weights.head)

@@ -2,9 +2,9 @@
 
 The counterpart of the reference's hybrid runner (src/paged_decode/hybrid.py:15-228):
 the full-attention layers keep their KV in 256-slot NHD pages, written by the HIP
-KV-write kernel and read by ``matched_decode`` / ``paged_decode``; the
-linear-attention (Gated DeltaNet) layers run the installed transformers blocks on
-their PyTorch path.  A decode step (every layer and the lm_head) runs eagerly or as
+KV-write kernel and read by ``matched_decode`` / ``paged_decode``.  The layers run on
+HIP kernels between their matrix products (``decoder_layers``); a model whose modules
+were changed runs the installed transformers blocks instead.  A decode step (every layer and the lm_head) runs eagerly or as
 one replayed hipGraph.
 
 Structure:
@@ -35,6 +35,7 @@ from transformers import AttentionInterface
 from transformers.cache_utils import LinearAttentionLayer
 from transformers.models.qwen3_5 import Qwen3_5ForCausalLM, Qwen3_5TextConfig
 
+from .decoder_layers import decoder_forward, decoder_states, decoder_weights
 from .kv_write import write_pages
 from .matched_splitkv import allocate_matched_resources, matched_decode
 from .prefill import batched_prefill
@@ -205,6 +206,22 @@ def _dense_decode(q, k_pages, v_pages, tables, lengths, scaling):
     return out
 
 
+def _decode_attention(runner, module, q, k, v):
+    """One layer's decode attention of q [B, Hq, D] over its pages, on the runner's backend."""
+    pool = runner.cache.pool
+    if runner.backend == "hip_matched":
+        out = matched_decode(q, k, v, pool.tables, pool.lengths, resources=runner.resources,
+                             scale=module.scaling)
+    elif runner.backend == "torch":
+        out = _dense_decode(q, k, v, pool.tables, pool.lengths, module.scaling)
+    else:
+        out = paged_decode(q, k, v, pool.tables, pool.lengths, resources=runner.resources,
+                           backend=runner.backend, scale=module.scaling)
+    if runner.attention_observer is not None:
+        runner.attention_observer(module, q, k, v, out)
+    return out
+
+
 def _attention(module, query, key, value, attention_mask, scaling, dropout=0.0, **kwargs):
     if attention_mask is not None or dropout:
         raise ValueError("the hybrid runner supports unpadded inference batches only")
@@ -212,20 +229,8 @@ def _attention(module, query, key, value, attention_mask, scaling, dropout=0.0, 
     cache = runner.cache
     if cache.phase == "prefill":
         return batched_prefill(query, key, value, scaling), None
-    q = query.squeeze(2)
-    pool = cache.pool
-    k, v = pool.pages(module.layer_idx)
-    if runner.backend == "hip_matched":
-        out = matched_decode(q, k, v, pool.tables, pool.lengths, resources=runner.resources,
-                             scale=scaling)
-    elif runner.backend == "torch":
-        out = _dense_decode(q, k, v, pool.tables, pool.lengths, scaling)
-    else:
-        out = paged_decode(q, k, v, pool.tables, pool.lengths, resources=runner.resources,
-                           backend=runner.backend, scale=scaling)
-    if runner.attention_observer is not None:
-        runner.attention_observer(module, q, k, v, out)
-    return out.unsqueeze(1), None
+    k, v = cache.pool.pages(module.layer_idx)
+    return _decode_attention(runner, module, query.squeeze(2), k, v).unsqueeze(1), None
 
 
 AttentionInterface.register("paged_decode_lab_hip", _attention)
@@ -308,6 +313,11 @@ class HybridRunner:
     @torch.inference_mode()
     def _forward(self, tokens, positions):
         """Logits of the last token; tokens [B, S] at ``positions`` [S] (device tensors)."""
+        weights = decoder_weights(self.model, self.cache.pool.block.device)
+        if weights is not None:
+            states = decoder_states(self, weights, tokens.shape[1])
+            if states is not None:
+                return decoder_forward(self, weights, states, tokens, positions, _decode_attention)
         # Several runners may share one model: the attention layers serve whichever
         # runner is running (a graph keeps the bindings it was captured with).
         for module in self.attention_modules:

@@ -1,0 +1,182 @@
+"""GPU parity of the decoder-layer kernels with the same formulas in 64 bits.
+
+float32 results are held to a few float32 ulps of the largest terms of their sums, bf16
+results to half a bf16 ulp (2^-8 of the value) more.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+if not torch.cuda.is_available():
+    pytest.skip("needs an MI355X GPU", allow_module_level=True)
+
+from paged_decode import _native
+from paged_decode import decoder_layers as DL
+from paged_decode import hybrid as H
+
+pytestmark = pytest.mark.gpu
+
+
+def bf16(gen, *shape, scale=1.0):
+    return (torch.randn(shape, generator=gen, device="cuda") * scale).to(torch.bfloat16)
+
+
+def close(got, ref, absolute, bf16_out=False):
+    bound = absolute + (2.0 ** -8 * ref.abs() if bf16_out else 0)
+    worst = ((got.double() - ref).abs() / bound).max()
+    assert worst <= 1, float(worst)
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 8), (3, 2040), (5, 2048), (2, 2056), (2, 8192)])
+@pytest.mark.parametrize("add", [False, True])
+def test_add_rms_norm(rows, dim, add):
+    gen = torch.Generator(device="cuda").manual_seed(dim)
+    x, y, w = bf16(gen, rows, dim), bf16(gen, rows, dim), bf16(gen, dim, scale=0.1)
+    out, held = torch.empty_like(x), x.clone()
+    _native.add_rms_norm(x, y if add else None, w, out, 1e-6)
+    total = (held.float() + y.float()).to(torch.bfloat16) if add else held
+    assert torch.equal(x, total)
+    t = total.double()
+    ref = t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * (1 + w.double())
+    close(out, ref, 2.0 ** -18 * ref.abs() + 1e-9, bf16_out=True)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_gates_and_gated_norm(dim):
+    gen = torch.Generator(device="cuda").manual_seed(dim)
+    rows = 9
+    o = torch.randn((rows, dim), generator=gen, device="cuda")
+    z, w, out = bf16(gen, rows, dim, scale=4), bf16(gen, dim), bf16(gen, rows, dim)
+    _native.gated_norm(o, z, w, out, rows, dim, 1e-6)
+    ref = o.double() * torch.rsqrt(o.double().square().mean(-1, keepdim=True) + 1e-6) * w.double()
+    ref = ref * F.silu(z.double())
+    close(out, ref, 2.0 ** -18 * ref.abs() + 1e-9, bf16_out=True)
+    a, b = bf16(gen, rows, dim, scale=30), bf16(gen, rows, 2 * dim, scale=30)
+    _native.sigmoid_gate(a, b[:, dim:], out, rows, dim)
+    ref = a.double() * torch.sigmoid(b[:, dim:].double())
+    close(out, ref, 2.0 ** -18 * ref.abs() + 1e-30, bf16_out=True)
+    ref = F.silu(a.double()) * z.double()
+    _native.silu_mul(a, z, a)
+    close(a, ref, 2.0 ** -18 * ref.abs() + 1e-30, bf16_out=True)
+
+
+def linear_case(batch, steps, hk, hv, dk, dv, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    c = 2 * hk * dk + hv * dv
+    return dict(x=bf16(gen, batch, steps, c), taps=bf16(gen, c, 1, 4, scale=0.3),
+                a=bf16(gen, batch, steps, hv, scale=3), b=bf16(gen, batch, steps, hv),
+                a_log=bf16(gen, hv), dt=bf16(gen, hv, scale=2),
+                conv=bf16(gen, batch, c, 4),
+                state=torch.randn((batch, hv, dk, dv), generator=gen, device="cuda") * 0.1)
+
+
+def linear_exact(t, hk, hv, dk, dv, held):
+    x, taps = t["x"].double(), t["taps"].double()[:, 0]
+    batch, steps, c = x.shape
+    prev = t["conv"].double().transpose(1, 2) if held else torch.zeros(batch, 4, c, device="cuda").double()
+    full = torch.cat([prev, x], 1)
+    act = F.silu(sum(full[:, 1 + j:1 + j + steps] * taps[:, j] for j in range(4)))
+    unit = lambda y: y * torch.rsqrt(y.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    q, k, v = act.split([hk * dk, hk * dk, hv * dv], -1)
+    q, k = unit(q.reshape(batch, steps, hk, dk)) * dk ** -0.5, unit(k.reshape(batch, steps, hk, dk))
+    decay = torch.exp(-t["a_log"].double().exp() * F.softplus(t["a"].double() + t["dt"].double()))
+    return (q, k, v.reshape(batch, steps, hv, dv), decay, torch.sigmoid(t["b"].double()),
+            full[:, -4:].transpose(1, 2))
+
+
+@pytest.mark.parametrize("hk,hv,dk,dv", [(4, 4, 64, 64), (2, 4, 128, 128), (1, 2, 64, 128), (3, 3, 128, 64)])
+@pytest.mark.parametrize("batch,steps,held", [(1, 1, False), (2, 1, True), (2, 3, False), (1, 3, True),
+                                              (1, 16, True), (2, 17, False), (1, 50, False)])
+def test_conv_and_delta_rule(hk, hv, dk, dv, batch, steps, held):
+    t = linear_case(batch, steps, hk, hv, dk, dv, steps + dk)
+    q, k, v, decay, beta, conv = linear_exact(t, hk, hv, dk, dv, held)
+    rows, c = batch * steps, t["x"].shape[-1]
+    act = torch.empty(batch, steps, c, device="cuda")
+    gates = torch.empty(batch, steps, hv, 2, device="cuda")
+    state = t["state"].clone()
+    _native.conv_gates(t["x"], t["taps"], t["a"], t["b"], t["a_log"], t["dt"], t["conv"], act, gates,
+                       batch, steps, hk, hv, dk, dv, held)
+    assert torch.equal(t["conv"].double(), conv)
+    ref = torch.cat([q.flatten(2), k.flatten(2), v.flatten(2)], -1)
+    close(act, ref, 1e-6 * (ref.abs() + 1))
+    close(gates[..., 0], decay, 4e-6 * (decay + 0.01))
+    close(gates[..., 1], beta, 1e-6)
+    ref = state.double() if held else torch.zeros_like(state).double()
+    want = torch.empty(batch, steps, hv, dv, device="cuda", dtype=torch.float64)
+    q, k = q.repeat_interleave(hv // hk, 2), k.repeat_interleave(hv // hk, 2)
+    for i in range(steps):
+        ref = ref * decay[:, i, :, None, None]
+        d = (v[:, i] - (k[:, i, :, :, None] * ref).sum(-2)) * beta[:, i, :, None]
+        ref = ref + k[:, i, :, :, None] * d[:, :, None]
+        want[:, i] = (q[:, i, :, :, None] * ref).sum(-2)
+    for lanes in (16, 32) if dk == 128 else (16,):
+        s, out = state.clone(), torch.empty(batch, steps, hv, dv, device="cuda")
+        _native.delta_rule(act, gates, s, out, batch, steps, hk, hv, dk, dv, held, lanes)
+        # the state stays below about 4; its float32 error grows with the steps it remembers
+        close(s, ref, 2e-6 * (1 + ref.abs()) * min(steps, 16))
+        close(out, want, 2e-6 * (1 + want.abs()) * min(steps, 16))
+
+
+@pytest.mark.parametrize("d,half", [(64, 8), (128, 64), (256, 32)])
+def test_rope_and_page_write(d, half):
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    batch, steps, hq, hkv, start = 2, 5, 4, 2, 254
+    q, k, v = bf16(gen, batch, steps, hq, 2, d), bf16(gen, batch, steps, hkv, d), bf16(gen, batch, steps, hkv, d)
+    wq, wk = bf16(gen, d, scale=0.1), bf16(gen, d, scale=0.1)
+    inv = (10000.0 ** (-torch.arange(half, device="cuda") / half)).to(torch.bfloat16)
+    positions = torch.arange(start, start + steps, device="cuda")
+    tables = torch.tensor([[3, 1], [0, -1]], dtype=torch.int32, device="cuda")
+    pages = torch.full((2, 4, 256, hkv, d), 7.0, device="cuda", dtype=torch.bfloat16)
+    rope = torch.empty(steps, half, 2, device="cuda")
+    _native.rope_table(positions, inv, rope)
+    angle = positions.double()[:, None] * inv.double()
+    close(rope[..., 0], angle.cos(), 2e-7 + 0 * angle)
+    close(rope[..., 1], angle.sin(), 2e-7 + 0 * angle)
+    q_out, k_out = torch.empty(batch, steps, hq, d, device="cuda").bfloat16(), torch.empty_like(k)
+    _native.qk_rope(q, k, v, wq, wk, rope, q_out, k_out, pages[0], pages[1], tables, positions, batch,
+                    steps, hq, hkv, d, half, 1e-6)
+
+    def turned(x, w):
+        x = x.double()
+        x = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * (1 + w.double())
+        a, b, rest = x[..., :half], x[..., half:2 * half], x[..., 2 * half:]
+        c, s = angle.cos()[:, None], angle.sin()[:, None]
+        return torch.cat([a * c - b * s, b * c + a * s, rest], -1)
+
+    for got, x, w in ((q_out, q[..., 0, :], wq), (k_out, k, wk)):
+        ref = turned(x, w)
+        close(got, ref, 1e-5 + 0 * ref, bf16_out=True)
+    want = torch.full_like(pages, 7.0)
+    for i, at in enumerate(positions.tolist()):
+        for b in range(batch):
+            page = int(tables[b, at // 256])
+            if page >= 0:
+                want[0, page, at % 256], want[1, page, at % 256] = k_out[b, i], v[b, i]
+    assert torch.equal(pages, want)
+
+
+@pytest.mark.parametrize("hk,hv,dk,dv,length", [(4, 4, 64, 64, 1), (2, 4, 128, 128, 19), (2, 2, 64, 128, 300)])
+def test_layers_agree_with_the_modules(hk, hv, dk, dv, length):
+    """One model on the kernels and, with a hook on a layer, on transformers' modules."""
+    cfg = H.decoder_config(num_hidden_layers=4, hidden_size=256, intermediate_size=512,
+                           vocab_size=512, linear_num_key_heads=hk, linear_key_head_dim=dk,
+                           linear_num_value_heads=hv, linear_value_head_dim=dv)
+    model = H.random_init_model(cfg, "cuda", seed=1)
+    prompt = [[(7 * i + j) % 512 for i in range(length)] for j in range(2)]
+    results = []
+    for hooked in (False, True):
+        handle = model.model.layers[1].mlp.register_forward_hook(lambda *a: None) if hooked else None
+        runner = H.HybridRunner(model=model, backend="hip_matched", batch=2, max_context=400)
+        assert (DL.decoder_weights(model, runner.cache.pool.block.device) is None) == hooked
+        logits = [runner.prefill(prompt)]
+        for s in range(3):
+            logits.append(runner.decode_step(torch.tensor([5 + s, 9 + s], device="cuda"), length + s))
+        states = [t.float().clone() for t in runner.cache.state_tensors()]
+        pages = runner.cache.pool.tables[:, 0].long()
+        results.append((logits, states, runner.cache.pool.block[:, :, pages, :min(length, 256)].float()))
+        if handle:
+            handle.remove()
+    # bf16 roundings at different places, through four layers
+    for a, b in zip(results[0][0] + results[0][1] + [results[0][2]],
+                    results[1][0] + results[1][1] + [results[1][2]]):
+        assert (a.float() - b.float()).norm() <= 0.03 * b.float().norm()
