@@ -357,6 +357,38 @@ int pd_qk_rope(const void* q, const void* k, const void* v, const void* q_weight
                int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t half, double eps,
                pd_stream_t stream);
 
+/* One token per sequence: products of 1 to 16 rows whose norms, gates,
+ * convolution and residual run in the same launch.  dim (the input features)
+ * is a multiple of 64; weights are bf16 [features, dim]. */
+
+/* h = x rms(x)^-1 (1 + norm); outs[i] = h weights[i]^T, bf16 [rows,
+ * features[i]].  With taps, outs[0] is instead float32 silu of the causal
+ * convolution of its channels, whose conv_state [rows, features[0], 4] moves
+ * one step (from zeros without has_prev).  The three arrays are host arrays of
+ * `count` <= 4. */
+int pd_norm_linears(const void* x, const void* norm, double eps, int32_t rows, int32_t dim,
+                    int32_t count, const void* const* weights, const int32_t* features,
+                    void* const* outs, const void* taps, void* conv_state, int32_t has_prev,
+                    pd_stream_t stream);
+
+/* out = silu(h gate^T) (h up^T), h as above. */
+int pd_norm_gate_up(const void* x, const void* norm, double eps, int32_t rows, int32_t dim,
+                    const void* gate, const void* up, void* out, int32_t features,
+                    pd_stream_t stream);
+
+/* x [rows, features] += h weight^T; with gate (rows of heads [dim / head_dim,
+ * 2, head_dim], pointing at the second half of the first), h sigmoid(gate) in
+ * the place of h. */
+int pd_linear_add(const void* h, const void* gate, int32_t head_dim, const void* weight, void* x,
+                  int32_t rows, int32_t dim, int32_t features, pd_stream_t stream);
+
+/* One token of pd_delta_rule and pd_gated_norm from act float32 [batch, C]
+ * (silu of the convolution; heads are normed here): out bf16 [batch, hv, dv]. */
+int pd_delta_step(const float* act, const void* a, const void* b, const void* a_log,
+                  const void* dt_bias, const void* z, const void* norm, double eps, float* state,
+                  void* out, int32_t batch, int32_t hk, int32_t hv, int32_t dk, int32_t dv,
+                  int32_t has_prev, pd_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

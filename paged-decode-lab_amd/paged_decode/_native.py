@@ -62,6 +62,11 @@ SIGNATURES = {
     "pd_rope_table": [_vp, _vp, _i32, _vp, _i32, _i32, _vp],
     "pd_qk_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp,
                    _i32, _i32, _i32, _i32, _i32, _i32, _dbl, _vp],
+    "pd_norm_linears": [_vp, _vp, _dbl, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp],
+    "pd_norm_gate_up": [_vp, _vp, _dbl, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
+    "pd_linear_add": [_vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _vp],
+    "pd_delta_step": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _dbl, _vp, _vp, _i32, _i32, _i32, _i32,
+                      _i32, _i32, _vp],
 }
 
 _lib = None
@@ -324,3 +329,34 @@ def qk_rope(q, k, v, q_weight, k_weight, rope, q_out, k_out, k_pages, v_pages, t
                            v_pages.data_ptr(), k_pages.shape[0], tables.data_ptr(),
                            tables.stride(0), tables.shape[1], positions.data_ptr(), batch, steps,
                            hq, hkv, d, half, eps, stream_handle(q.device)))
+
+
+def norm_linears(x, norm, eps, weights, outs, taps=None, conv_state=None, has_prev=False):
+    """outs[i] = norm(x) weights[i]^T; with taps outs[0] (float32) is convolved."""
+    n = len(weights)
+    check(lib().pd_norm_linears(
+        x.data_ptr(), norm.data_ptr(), eps, x.shape[0], x.shape[1], n,
+        (_vp * n)(*[w.data_ptr() for w in weights]), (_i32 * n)(*[w.shape[0] for w in weights]),
+        (_vp * n)(*[o.data_ptr() for o in outs]), None if taps is None else taps.data_ptr(),
+        None if conv_state is None else conv_state.data_ptr(), int(has_prev),
+        stream_handle(x.device)))
+
+
+def norm_gate_up(x, norm, eps, gate, up, out):
+    check(lib().pd_norm_gate_up(x.data_ptr(), norm.data_ptr(), eps, x.shape[0], x.shape[1],
+                                gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.shape[0],
+                                stream_handle(x.device)))
+
+
+def linear_add(h, weight, x, gate=None, head_dim=0):
+    """x += h weight^T, or (h sigmoid(gate)) weight^T."""
+    check(lib().pd_linear_add(h.data_ptr(), None if gate is None else gate.data_ptr(), head_dim,
+                              weight.data_ptr(), x.data_ptr(), x.shape[0], weight.shape[1],
+                              weight.shape[0], stream_handle(x.device)))
+
+
+def delta_step(act, a, b, a_log, dt_bias, z, norm, eps, state, out, batch, hk, hv, dk, dv, has_prev):
+    check(lib().pd_delta_step(act.data_ptr(), a.data_ptr(), b.data_ptr(), a_log.data_ptr(),
+                              dt_bias.data_ptr(), z.data_ptr(), norm.data_ptr(), eps,
+                              state.data_ptr(), out.data_ptr(), batch, hk, hv, dk, dv,
+                              int(has_prev), stream_handle(act.device)))

@@ -3,7 +3,8 @@
 ``decoder_weights`` reads the model's modules and says whether every one of them is the
 plain form the kernels compute; ``decoder_forward`` is then one forward of the model, with
 the residual stream, the norms, the gated delta rule, rotary embedding, the K/V write and
-the gates in HIP kernels between the matrix products.  A model that was changed (hooks,
+the gates in HIP kernels between the matrix products.  One token per sequence of up to
+``TOKEN_ROWS`` sequences runs the products in them too.  A model that was changed (hooks,
 replaced or compiled modules, biases, other dtypes or sizes) keeps transformers' modules:
 the weights are read from the modules on every forward, nothing is kept of them.
 """
@@ -19,6 +20,7 @@ from . import _native
 from .prefill import batched_prefill
 
 MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
+TOKEN_ROWS = 16         # rows of one MFMA operand
 
 
 def _plain_module(module, kind):
@@ -251,17 +253,68 @@ def _full_attention(h, w, weights, rope, runner, batch, steps, attend):
     return F.linear(y, o_proj)
 
 
-def decoder_forward(runner, weights, states, tokens, positions, attend):
-    """Logits of the last token; as HybridRunner._forward, on the kernels.  ``attend`` is
-    the decode attention of one layer over its pages."""
-    model, text = runner.model, runner.text
-    batch, steps = tokens.shape
-    runner.cache.pool.begin_step(positions)
-    x = text.embed_tokens(tokens)
-    rows, hid = batch * steps, x.shape[-1]
-    x = x.view(rows, hid)
-    rope = torch.empty((steps, weights.half, 2), device=x.device, dtype=torch.float32)
-    _native.rope_table(positions, weights.inv_freq, rope)
+def _token_form(weights, rows):
+    """One token per sequence of few sequences: products that read each weight once, with
+    everything between them folded in.  The normed rows must fit a workgroup's LDS."""
+    hid = weights.head.shape[1]
+    mid = weights.layers[0].down.shape[1] if weights.layers else 64
+    hk, hv, dk, dv = weights.linear
+    full = [w.mixer[5].shape[1] for w in weights.layers if w.module is not None]
+    return (rows <= TOKEN_ROWS and hid % 64 == 0 and mid % 64 == 0 and hv * dv % 64 == 0
+            and all(k % 64 == 0 for k in full) and rows * (hid + 8) * 2 + 16384 <= 160 * 1024)
+
+
+def _token_linear(x, w, weights, states, batch):
+    hk, hv, dk, dv = weights.linear
+    qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
+    conv, state, held = states
+    act = torch.empty((batch, qkv.shape[0]), device=x.device, dtype=torch.float32)
+    rest = torch.empty((2 * batch * (hv * dv + 8 * hv)), device=x.device, dtype=torch.bfloat16)
+    gate = rest[:batch * hv * dv]
+    beta, decay = rest[gate.numel():], rest[gate.numel() + 8 * batch * hv:]
+    out = rest[gate.numel() + 16 * batch * hv:]
+    _native.norm_linears(x, w.in_norm[0], w.in_norm[1], (qkv, z, b, a), (act, gate, beta, decay), taps,
+                         conv, held)
+    _native.delta_step(act, decay, beta, a_log, dt_bias, gate, norm, eps, state, out, batch, hk, hv,
+                       dk, dv, held)
+    _native.linear_add(out, out_proj, x)
+
+
+def _token_full(x, w, weights, rope, runner, batch, attend):
+    spec, pool = runner.spec, runner.cache.pool
+    hq, hkv, d = spec.num_heads, spec.num_kv_heads, spec.head_dim
+    q_proj, k_proj, v_proj, (q_norm, eps), (k_norm, _), o_proj = w.mixer
+    rows = lambda *shape: torch.empty(shape, device=x.device, dtype=torch.bfloat16)  # noqa: E731
+    q, k, v, query = rows(batch, hq, 2 * d), rows(batch, hkv, d), rows(batch, hkv, d), rows(batch, hq, d)
+    _native.norm_linears(x, w.in_norm[0], w.in_norm[1], (q_proj, k_proj, v_proj), (q, k, v))
+    k_pages, v_pages = pool.pages(w.index)
+    fill = runner.cache.phase == "prefill"
+    keys = torch.empty_like(k) if fill else None
+    _native.qk_rope(q, k, v, q_norm, k_norm, rope, query, keys, k_pages, v_pages, pool.tables,
+                    pool.positions, batch, 1, hq, hkv, d, weights.half, eps)
+    if fill:
+        out = batched_prefill(query[:, :, None], keys[:, :, None], v[:, :, None], w.module.scaling)
+    else:
+        out = attend(runner, w.module, query, k_pages, v_pages)
+    _native.linear_add(out, o_proj, x, q[..., d:], d)
+
+
+def _token_layers(x, runner, weights, states, rope, attend):
+    batch = x.shape[0]
+    for w in weights.layers:
+        if w.module is None:
+            _token_linear(x, w, weights, states[w.index], batch)
+            runner.cache.linear[w.index].has_previous_state[0] = True
+        else:
+            _token_full(x, w, weights, rope, runner, batch, attend)
+        h = torch.empty((batch, w.gate.shape[0]), device=x.device, dtype=torch.bfloat16)
+        _native.norm_gate_up(x, w.post_norm[0], w.post_norm[1], w.gate, w.up, h)
+        _native.linear_add(h, w.down, x)
+
+
+def _row_layers(x, runner, weights, states, rope, batch, steps, attend):
+    """Any number of rows: library products with the kernels between them; returns the
+    last layer's output, not yet added to the residual stream x."""
     y = None
     for w in weights.layers:
         h = torch.empty_like(x)
@@ -275,9 +328,35 @@ def decoder_forward(runner, weights, states, tokens, positions, attend):
         gate, up = F.linear(h, w.gate), F.linear(h, w.up)
         _native.silu_mul(gate, up, gate)
         y = F.linear(gate, w.down)
-    if steps > 1:
-        x = x.view(batch, steps, hid)[:, -1].contiguous()
-        y = y.view(batch, steps, hid)[:, -1].contiguous()
+    return y
+
+
+def decoder_forward(runner, weights, states, tokens, positions, attend):
+    """Logits of the last token; as HybridRunner._forward, on the kernels.  ``attend`` is
+    the decode attention of one layer over its pages."""
+    text = runner.text
+    batch, steps = tokens.shape
+    runner.cache.pool.begin_step(positions)
+    x = text.embed_tokens(tokens)
+    hid = x.shape[-1]
+    x = x.view(batch * steps, hid)
+    rope = torch.empty((steps, weights.half, 2), device=x.device, dtype=torch.float32)
+    _native.rope_table(positions, weights.inv_freq, rope)
+    y = None
+    if steps == 1 and _token_form(weights, batch):
+        _token_layers(x, runner, weights, states, rope, attend)
+    else:
+        y = _row_layers(x, runner, weights, states, rope, batch, steps, attend)
+        if steps > 1:
+            x = x.view(batch, steps, hid)[:, -1].contiguous()
+            y = y if y is None else y.view(batch, steps, hid)[:, -1].contiguous()
+    norm, eps = weights.norm
+    if _token_form(weights, batch):
+        if y is not None:
+            x = x + y
+        logits = torch.empty((batch, weights.head.shape[0]), device=x.device, dtype=x.dtype)
+        _native.norm_linears(x, norm, eps, (weights.head,), (logits,))
+        return logits
     h = torch.empty_like(x)
-    _native.add_rms_norm(x, y, weights.norm[0], h, weights.norm[1])
+    _native.add_rms_norm(x, y, norm, h, eps)
     return F.linear(h, weights.head)
