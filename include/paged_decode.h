@@ -326,21 +326,31 @@ int pd_sigmoid_gate(const void* x, const void* gate, int64_t gate_stride, void* 
 
 /* Gated delta rule inputs of x [batch, steps, C], C = 2 hk dk + hv dv channels
  * (queries, keys, values): causal convolution with taps [C, 4], silu, unit
- * query (times dk^-1/2) and key heads -> act float32 [batch, steps, C]; decay
- * = exp(-exp(a_log) softplus(a + dt_bias)) and sigmoid(b) -> gates float32
- * [batch, steps, hv, 2].  conv_state [batch, C, 4] receives the last four
- * inputs; with has_prev (at most 16 steps) it holds the four before them. */
-int pd_conv_gates(const void* x, const void* taps, const void* a, const void* b, const void* a_log,
-                  const void* dt_bias, void* conv_state, float* act, float* gates, int32_t batch,
+ * query (times dk^-1/2) and key heads -> act float32 [batch, steps, C].
+ * conv_state [batch, C, 4] receives the last four inputs; with has_prev (at
+ * most 16 steps) it holds the four before them. */
+int pd_conv(const void* x, const void* taps, void* conv_state, float* act, int32_t batch,
+            int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t has_prev,
+            pd_stream_t stream);
+
+/* gates float32 [rows, hv, 2] = (-exp(a_log) softplus(h wa^T + dt_bias),
+ * sigmoid(h wb^T)): the log decay and beta of h [rows, dim]. */
+int pd_gates(const void* h, const void* wa, const void* wb, const void* a_log, const void* dt_bias,
+             float* gates, int64_t rows, int32_t dim, int32_t hv, pd_stream_t stream);
+
+/* S = decay S; S += k (beta (v - S^T k))^T; out = S^T q per value head and
+ * token, one after the other; state float32 [batch, hv, dk, dv], read with has_prev, written;
+ * out float32 [batch, steps, hv, dv]. */
+int pd_delta_rule(const float* act, const float* gates, float* state, float* out, int32_t batch,
                   int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t has_prev,
                   pd_stream_t stream);
 
-/* S = decay S; S += k (beta (v - S^T k))^T; out = S^T q per value head and
- * token; state float32 [batch, hv, dk, dv], read with has_prev, written;
- * out float32 [batch, steps, hv, dv]; lanes per state column 16 or 32. */
-int pd_delta_rule(const float* act, const float* gates, float* state, float* out, int32_t batch,
-                  int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t has_prev,
-                  int32_t lanes, pd_stream_t stream);
+/* The same in chunks of 64 tokens; workspace of pd_delta_workspace floats. */
+int pd_delta_chunks(const float* act, const float* gates, float* state, float* out,
+                    float* workspace, int32_t batch, int32_t steps, int32_t hk, int32_t hv,
+                    int32_t dk, int32_t dv, int32_t has_prev, pd_stream_t stream);
+int pd_delta_workspace(int32_t batch, int32_t steps, int32_t hv, int32_t dk, int32_t dv,
+                       int64_t* floats);
 
 /* table float32 [steps, half, 2]: cos and sin of positions x inv_freq. */
 int pd_rope_table(const int64_t* positions, const void* inv_freq, int32_t is_bf16, float* table,

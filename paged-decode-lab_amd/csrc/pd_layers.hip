@@ -157,132 +157,229 @@ gate_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
   *reinterpret_cast<u32x4_t*>(out + 8 * p) = pack8(x);
 }
 
-// -------------------------------------------------- convolution and gates
-// Causal depthwise convolution of 4 taps, silu, the unit norm of the query and
-// key heads (queries times dk^-1/2), and the delta rule's decay and beta.  A
-// wavefront runs kConvSteps tokens of one unit, the three earlier inputs in
-// registers: units 0 .. hk - 1 are a key head and its query head, the rest a
-// value head and its gates.  Channels: [hk dk queries | hk dk keys | hv dv].
+// ------------------------------------------------------------- convolution
+// Causal depthwise convolution of 4 taps, silu, and the unit norm of the query
+// and key heads (queries times dk^-1/2).  Units: 0 .. hk - 1 are a key head and
+// its query head, the rest a value head; a wavefront serves one unit.  Lanes
+// hold 8 channels of a head (16-byte loads), D / 8 lanes a row, and each lane
+// group takes kConvTokens consecutive tokens with the three rows before them,
+// all loaded before the first is used.  Channels: [hk dk queries | hk dk keys |
+// hv dv].  512 tokens of 6144 channels: 27 us with a token loop per wavefront
+// (4-byte loads, two 64-lane sums a token), 8.6 us in this form.
 //
 // conv_state [B, C, 4] receives the last four inputs; with `has_prev` it holds
 // the four before this call, and the call's steps fit one wavefront's, so that
 // the wavefront that reads a channel's state is the one that writes it.
-constexpr int kConvSteps = 16;
+constexpr int kConvTokens = 4;
 
 struct ConvArgs {
-  const uint16_t *x, *taps, *a, *b, *a_log, *dt_bias;
+  const uint16_t *x, *taps;
   uint16_t* conv_state;
-  float *act, *gates;  // [B, S, C], [B, S, hv, 2] = (decay, beta)
+  float* act;  // [B, S, C]
   int steps, hk, hv, has_prev;
 };
 
-template <int E>
-struct ConvRun {  // E channels of a lane
-  float tap[4][E], x[4][E];
+// Sum over the N = 8 or 16 lanes of a group, in every lane, by DPP moves: row
+// rotations, or for half rows lane ^ 1, lane ^ 2 and the mirrored half row.
+template <int N>
+__device__ __forceinline__ float group_sum(float x) {
+  const auto dpp = [](float v, auto ctrl) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl.value, 0xF, 0xF, false));
+  };
+  if constexpr (N == 16) {
+    x += dpp(x, std::integral_constant<int, 0x128>{});
+    x += dpp(x, std::integral_constant<int, 0x124>{});
+    x += dpp(x, std::integral_constant<int, 0x122>{});
+    return x + dpp(x, std::integral_constant<int, 0x121>{});
+  } else {
+    static_assert(N == 8, "lanes of a group");
+    x += dpp(x, std::integral_constant<int, 0xB1>{});
+    x += dpp(x, std::integral_constant<int, 0x4E>{});
+    return x + dpp(x, std::integral_constant<int, 0x141>{});
+  }
+}
 
-  __device__ __forceinline__ void begin(const ConvArgs& p, int64_t b, int C, int c, int t0) {
+// The convolved rows t0 .. t0 + kConvTokens - 1 of 8 channels from c.
+struct ConvRows {
+  u32x4_t x[kConvTokens + 3];
+  float tap[8][4];
+
+  __device__ __forceinline__ void load(const ConvArgs& p, int64_t b, int C, int c, int t0) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const u32x2_t w = *reinterpret_cast<const u32x2_t*>(p.taps + 4 * (c + e));
-      tap[0][e] = bf16_lo(w.x), tap[1][e] = bf16_hi(w.x);
-      tap[2][e] = bf16_lo(w.y), tap[3][e] = bf16_hi(w.y);
+    for (int i = 0; i < kConvTokens + 3; ++i) {
+      const int t = t0 - 3 + i;
+      x[i] = u32x4_t{};
+      if (t >= 0 && t < p.steps) x[i] = load16(p.x + (b * p.steps + t) * C + c);
     }
+    u32x4_t w[4];
 #pragma unroll
-    for (int j = 1; j < 4; ++j) {
-      const int t = t0 - 4 + j;
-      if (t >= 0) {
-        load_bf16<E>(p.x + (b * p.steps + t) * C + c, x[j]);
-      } else {
+    for (int i = 0; i < 4; ++i) w[i] = load16(p.taps + 4 * c + 8 * i);
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-          x[j][e] = p.has_prev ? bf16_lo(p.conv_state[(b * C + c + e) * 4 + 4 + t]) : 0.f;
-      }
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t lo = w[e / 2][2 * (e & 1)], hi = w[e / 2][2 * (e & 1) + 1];
+      tap[e][0] = bf16_lo(lo), tap[e][1] = bf16_hi(lo), tap[e][2] = bf16_lo(hi), tap[e][3] = bf16_hi(hi);
+    }
+    if (p.has_prev && t0 < 3) {  // rows -3 .. -1 are elements 1 .. 3 of the state
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (t0 - 3 + i < 0) {
+          uint16_t v[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = p.conv_state[(b * C + c + e) * 4 + 4 + (t0 - 3 + i)];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[i][e] = v[2 * e] | uint32_t(v[2 * e + 1]) << 16;
+        }
     }
   }
-  __device__ __forceinline__ void step(const ConvArgs& p, int64_t row, int C, int c, float (&y)[E]) {
+  __device__ __forceinline__ void row(int i, float (&y)[8]) const {
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[0][e] = x[1][e], x[1][e] = x[2][e], x[2][e] = x[3][e];
-    load_bf16<E>(p.x + row * C + c, x[3]);
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
+    for (int e = 0; e < 8; ++e) {
       float s = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s = fmaf(x[j][e], tap[j][e], s);
+      for (int j = 0; j < 4; ++j)
+        s = fmaf(e & 1 ? bf16_hi(x[i + j][e / 2]) : bf16_lo(x[i + j][e / 2]), tap[e][j], s);
       y[e] = silu(s);
     }
   }
-  __device__ __forceinline__ void finish(const ConvArgs& p, int64_t b, int C, int c) {
+  // The four inputs up to row i as the channels' new state.
+  __device__ __forceinline__ void finish(const ConvArgs& p, int64_t b, int C, int c, int i) const {
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      *reinterpret_cast<u32x2_t*>(p.conv_state + (b * C + c + e) * 4) =
-          u32x2_t{pack_bf16(x[0][e], x[1][e]), pack_bf16(x[2][e], x[3][e])};
+    for (int e = 0; e < 8; e += 2) {
+      u32x4_t s;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const auto at = [&](int j) {
+          return k ? x[i + j][e / 2] >> 16 : x[i + j][e / 2] & 0xffffu;
+        };
+        s[2 * k] = at(0) | at(1) << 16;
+        s[2 * k + 1] = at(2) | at(3) << 16;
+      }
+      *reinterpret_cast<u32x4_t*>(p.conv_state + (b * C + c + e) * 4) = s;
+    }
   }
 };
 
-__device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
-
 template <int DK, int DV>
-__global__ void __launch_bounds__(256) conv_gates_kernel(const ConvArgs p) {
+__global__ void __launch_bounds__(256) conv_kernel(const ConvArgs p) {
+  constexpr int kWaveTokens = 64 / (DK / 8) * kConvTokens;  // of a key head's unit
   const int lane = threadIdx.x & 63;
   const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (unit >= p.hk + p.hv) return;
-  const int t0 = blockIdx.y * kConvSteps, t1 = min(t0 + kConvSteps, p.steps);
   const int64_t b = blockIdx.z;
   const int C = 2 * p.hk * DK + p.hv * DV;
+  const int begin = blockIdx.y * kWaveTokens;
+  const auto store = [&](int t, int c, const float (&y)[8]) {
+    float* out = p.act + (b * p.steps + t) * C + c;
+    *reinterpret_cast<floatx4_t*>(out) = floatx4_t{y[0], y[1], y[2], y[3]};
+    *reinterpret_cast<floatx4_t*>(out + 4) = floatx4_t{y[4], y[5], y[6], y[7]};
+  };
   if (unit < p.hk) {
-    constexpr int E = DK / 64;
-    const int cq = unit * DK + E * lane, ck = cq + p.hk * DK;
-    ConvRun<E> q, k;
-    q.begin(p, b, C, cq, t0);
-    k.begin(p, b, C, ck, t0);
-    for (int t = t0; t < t1; ++t) {
-      const int64_t row = b * p.steps + t;
-      float yq[E], yk[E], sq = 0.f, sk = 0.f;
-      q.step(p, row, C, cq, yq);
-      k.step(p, row, C, ck, yk);
+    constexpr int L = DK / 8;
+    const int cq = unit * DK + 8 * (lane % L), ck = cq + p.hk * DK;
+    const int t0 = begin + kConvTokens * (lane / L);
+    ConvRows q, k;
+    q.load(p, b, C, cq, t0);
+    k.load(p, b, C, ck, t0);
 #pragma unroll
-      for (int e = 0; e < E; ++e) sq = fmaf(yq[e], yq[e], sq), sk = fmaf(yk[e], yk[e], sk);
-      const float rq = rsqrtf(wave_sum(sq) + 1e-6f) * rsqrtf(float(DK));
-      const float rk = rsqrtf(wave_sum(sk) + 1e-6f);
+    for (int i = 0; i < kConvTokens; ++i) {
+      float yq[8], yk[8], sq = 0.f, sk = 0.f;
+      q.row(i, yq);
+      k.row(i, yk);
 #pragma unroll
-      for (int e = 0; e < E; ++e) yq[e] *= rq, yk[e] *= rk;
-      store_f32<E>(p.act + row * C + cq, yq);
-      store_f32<E>(p.act + row * C + ck, yk);
-    }
-    if (t1 == p.steps) {
-      q.finish(p, b, C, cq);
-      k.finish(p, b, C, ck);
+      for (int e = 0; e < 8; ++e) sq = fmaf(yq[e], yq[e], sq), sk = fmaf(yk[e], yk[e], sk);
+      const float rq = rsqrtf(group_sum<L>(sq) + 1e-6f) * rsqrtf(float(DK));
+      const float rk = rsqrtf(group_sum<L>(sk) + 1e-6f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) yq[e] *= rq, yk[e] *= rk;
+      if (t0 + i < p.steps) {
+        store(t0 + i, cq, yq);
+        store(t0 + i, ck, yk);
+      }
+      if (t0 + i == p.steps - 1) {
+        q.finish(p, b, C, cq, i);
+        k.finish(p, b, C, ck, i);
+      }
     }
   } else {
-    constexpr int E = DV / 64;
-    const int h = unit - p.hk, c = 2 * p.hk * DK + h * DV + E * lane;
-    ConvRun<E> v;
-    v.begin(p, b, C, c, t0);
-    for (int t = t0; t < t1; ++t) {
-      const int64_t row = b * p.steps + t;
-      float y[E];
-      v.step(p, row, C, c, y);
-      store_f32<E>(p.act + row * C + c, y);
-    }
-    if (t1 == p.steps) v.finish(p, b, C, c);
-    if (t0 + lane < t1) {
-      const int64_t at = (b * p.steps + t0 + lane) * p.hv + h;
-      const float a = bf16_lo(p.a[at]) + bf16_lo(p.dt_bias[h]);
-      const float g = -expf(bf16_lo(p.a_log[h])) * softplus(a);
-      *reinterpret_cast<floatx2_t*>(p.gates + 2 * at) =
-          floatx2_t{expf(g), sigmoid(bf16_lo(p.b[at]))};
+    // A value head's tokens of this block, in as many passes as its lane
+    // groups need.
+    constexpr int L = DV / 8, kPass = 64 / L * kConvTokens;
+    const int c = 2 * p.hk * DK + (unit - p.hk) * DV + 8 * (lane % L);
+    for (int t = begin; t < begin + kWaveTokens; t += kPass) {
+      const int t0 = t + kConvTokens * (lane / L);
+      ConvRows v;
+      v.load(p, b, C, c, t0);
+#pragma unroll
+      for (int i = 0; i < kConvTokens; ++i) {
+        float y[8];
+        v.row(i, y);
+        if (t0 + i < min(p.steps, begin + kWaveTokens)) store(t0 + i, c, y);
+        if (t0 + i == p.steps - 1 && t0 + i < begin + kWaveTokens) v.finish(p, b, C, c, i);
+      }
     }
   }
+}
+
+// ------------------------------------------------------------------- gates
+// (log decay, beta) = (-exp(a_log) softplus(h wa + dt_bias), sigmoid(h wb)) of
+// every token and value head: two products of few output features, 16 tokens a
+// workgroup, whose wavefronts split K in units of 64 elements (weights the row
+// operand, tokens the column operand).  Two library products took 21 us at 512
+// tokens of 2048, 7.3 us here.
+constexpr int kGateWaves = 8;
+
+__device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+
+__global__ void __launch_bounds__(64 * kGateWaves)
+gates_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wa,
+             const uint16_t* __restrict__ wb, const uint16_t* __restrict__ a_log,
+             const uint16_t* __restrict__ dt_bias, float* __restrict__ gates, int64_t rows, int K,
+             int hv) {
+  __shared__ __attribute__((aligned(16))) float part[2][kGateWaves][16][16];
+  const int tid = threadIdx.x, lane = tid & 63, op = lane & 15, quad = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t r0 = int64_t(blockIdx.x) * 16;
+  const int f0 = blockIdx.y * 16;
+  const int64_t feature = int64_t(min(f0 + op, hv - 1)) * K + 8 * quad;
+  const uint16_t* x = h + min(r0 + op, rows - 1) * K + 8 * quad;
+  const auto mfma = [](u32x4_t a, u32x4_t b, floatx4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  };
+  floatx4_t acc[2] = {};
+#pragma unroll 4
+  for (int k = 64 * w; k < K; k += 64 * kGateWaves) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const u32x4_t xv = load16(x + k + 32 * s);
+      acc[0] = mfma(load16(wa + feature + k + 32 * s), xv, acc[0]);
+      acc[1] = mfma(load16(wb + feature + k + 32 * s), xv, acc[1]);
+    }
+  }
+  mfma_result_barrier(acc);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    *reinterpret_cast<floatx4_t*>(&part[i][w][op][4 * quad]) = acc[i];
+  __syncthreads();
+  const int f = tid & 15, row = tid >> 4;
+  if (tid >= 256 || f0 + f >= hv || r0 + row >= rows) return;
+  float a = 0.f, b = 0.f;
+#pragma unroll
+  for (int v = 0; v < kGateWaves; ++v) a += part[0][v][row][f], b += part[1][v][row][f];
+  const float g = -expf(bf16_lo(a_log[f0 + f])) * softplus(a + bf16_lo(dt_bias[f0 + f]));
+  *reinterpret_cast<floatx2_t*>(gates + ((r0 + row) * hv + f0 + f) * 2) = floatx2_t{g, sigmoid(b)};
 }
 
 // -------------------------------------------------------- gated delta rule
 // Per value head and column j of its state S [dk, dv], over the tokens:
 //   S_j *= decay;  d = beta (v_j - k . S_j);  S_j += d k;  o_j = q . S_j.
-// The columns are independent, so each is one group of L lanes that hold
-// DK / L of its elements in registers for the whole sequence; what is serial
-// is the chain of a token's dot, its reduction over the L lanes (lane moves)
-// and the update.  L = 32 halves the work of a token's chain, L = 16 the total
-// work.  A workgroup of two wavefronts stages kDeltaSteps tokens of k, q, v
+// The columns are independent, so each is one group of 16 lanes that hold
+// DK / 16 of its elements in registers for the whole sequence; what is serial
+// is the chain of a token's dot, its reduction over the 16 lanes (lane moves)
+// and the update, 174 ns a token (32 lanes a column: no faster with one
+// sequence, a third slower with eight).  For few tokens; more run in chunks
+// (pd_delta_chunks).  A workgroup of two wavefronts stages kDeltaSteps tokens of k, q, v
 // and the gates in LDS, the next ones loaded to registers meanwhile.
 constexpr int kDeltaSteps = 16;
 
@@ -292,26 +389,9 @@ struct DeltaArgs {
   int steps, hk, hv, has_prev;
 };
 
-template <int L>
-__device__ __forceinline__ float lanes_sum(float x) {
-  const auto ror = [](float v, auto n) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n.value, 0xF,
-                                                      0xF, false));
-  };
-  x += ror(x, std::integral_constant<int, 8>{});
-  x += ror(x, std::integral_constant<int, 4>{});
-  x += ror(x, std::integral_constant<int, 2>{});
-  x += ror(x, std::integral_constant<int, 1>{});
-  if constexpr (L == 32) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  }
-  return x;
-}
-
-template <int DK, int DV, int L>
+template <int DK, int DV>
 __global__ void __launch_bounds__(128) delta_kernel(const DeltaArgs p) {
-  constexpr int T = kDeltaSteps, N = DK / L, P = N / 4;  // elements, 16-byte pieces a lane
+  constexpr int L = 16, T = kDeltaSteps, N = DK / L, P = N / 4;  // elements, 16-byte pieces a lane
   constexpr int kCols = 128 / L;                         // columns per workgroup
   constexpr int kRowLoads = 2 * T * DK / 4 / 128;        // 16-byte pieces of q and k per thread
   static_assert(N % 4 == 0 && kCols * T <= 128, "one v element per thread");
@@ -335,7 +415,7 @@ __global__ void __launch_bounds__(128) delta_kernel(const DeltaArgs p) {
 
   floatx4_t fq[kRowLoads];
   float fv = 0.f;
-  floatx2_t fg = {1.f, 0.f};
+  floatx2_t fg = {0.f, 0.f};
   const auto fetch = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < kRowLoads; ++i) {
@@ -354,7 +434,7 @@ __global__ void __launch_bounds__(128) delta_kernel(const DeltaArgs p) {
     for (int i = 0; i < kRowLoads; ++i)
       *reinterpret_cast<floatx4_t*>(&qk[buf][0][0][0] + 4 * (128 * i + tid)) = fq[i];
     if (tid < T * kCols) (&vs[buf][0][0])[tid] = fv;
-    if (tid < T) gs[buf][tid] = fg;
+    if (tid < T) gs[buf][tid] = floatx2_t{expf(fg.x), fg.y};
   };
 
   fetch(0);
@@ -380,7 +460,7 @@ __global__ void __launch_bounds__(128) delta_kernel(const DeltaArgs p) {
         d0 = fmaf(k[i / 4][i % 4], s[i], d0);
         d1 = fmaf(k[i / 4][i % 4 + 1], s[i + 1], d1);
       }
-      const float d = g.y * fmaf(-g.x, lanes_sum<L>(d0 + d1), v);
+      const float d = g.y * fmaf(-g.x, group_sum<L>(d0 + d1), v);
       float o0 = 0.f, o1 = 0.f;
 #pragma unroll
       for (int i = 0; i < N; ++i) s[i] = fmaf(k[i / 4][i % 4], d, g.x * s[i]);
@@ -389,7 +469,7 @@ __global__ void __launch_bounds__(128) delta_kernel(const DeltaArgs p) {
         o0 = fmaf(q[i / 4][i % 4], s[i], o0);
         o1 = fmaf(q[i / 4][i % 4 + 1], s[i + 1], o1);
       }
-      const float o = lanes_sum<L>(o0 + o1);
+      const float o = group_sum<L>(o0 + o1);
       if (sub == t) keep = o;
     };
     if (n == T) {
@@ -587,56 +667,65 @@ extern "C" int pd_sigmoid_gate(const void* x, const void* gate, int64_t gate_str
   return launch_status("pd_sigmoid_gate");
 }
 
-extern "C" int pd_conv_gates(const void* x, const void* taps, const void* a, const void* b,
-                             const void* a_log, const void* dt_bias, void* conv_state, float* act,
-                             float* gates, int32_t batch, int32_t steps, int32_t hk, int32_t hv,
-                             int32_t dk, int32_t dv, int32_t has_prev, pd_stream_t stream) {
+extern "C" int pd_conv(const void* x, const void* taps, void* conv_state, float* act, int32_t batch,
+                       int32_t steps, int32_t hk, int32_t hv, int32_t dk, int32_t dv,
+                       int32_t has_prev, pd_stream_t stream) {
   pd::clear_error();
   if (batch < 1 || batch > 65535 || steps < 1 || hk < 1 || hv < 1 || hv % hk)
     return pd::fail(PD_EINVAL, "batch, steps and heads must be positive, value heads a multiple");
   if (!valid_linear_dims(dk, dv)) return pd::fail(PD_EINVAL, "linear heads of 64 or 128 elements");
-  if (has_prev && steps > kConvSteps)
-    return pd::fail(PD_EINVAL, "at most %d steps continue a state", kConvSteps);
-  const int64_t chunks = (int64_t(steps) + kConvSteps - 1) / kConvSteps;
+  const int tokens = 64 / (dk / 8) * kConvTokens;  // of a wavefront
+  if (has_prev && steps > 16)
+    return pd::fail(PD_EINVAL, "at most 16 steps continue a state");
+  const int64_t chunks = (int64_t(steps) + tokens - 1) / tokens;
   if (chunks > 65535) return pd::fail(PD_EINVAL, "too many steps");
-  if (!x || !taps || !a || !b || !a_log || !dt_bias || !conv_state || !act || !gates ||
-      !all_aligned16(x, taps, conv_state, act, gates))
+  if (!x || !taps || !conv_state || !act || !all_aligned16(x, taps, conv_state, act))
     return pd::fail(PD_EINVAL, "tensors must be present and 16-byte aligned");
-  const ConvArgs p{u16(x), u16(taps), u16(a), u16(b), u16(a_log), u16(dt_bias), u16(conv_state),
-                   act, gates, steps, hk, hv, has_prev};
+  const ConvArgs p{u16(x), u16(taps), u16(conv_state), act, steps, hk, hv, has_prev};
   const dim3 grid(unsigned((hk + hv + 3) / 4), unsigned(chunks), unsigned(batch));
   const auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), p);
   };
   if (dk == 64)
-    dv == 64 ? go(conv_gates_kernel<64, 64>) : go(conv_gates_kernel<64, 128>);
+    dv == 64 ? go(conv_kernel<64, 64>) : go(conv_kernel<64, 128>);
   else
-    dv == 64 ? go(conv_gates_kernel<128, 64>) : go(conv_gates_kernel<128, 128>);
-  return launch_status("pd_conv_gates");
+    dv == 64 ? go(conv_kernel<128, 64>) : go(conv_kernel<128, 128>);
+  return launch_status("pd_conv");
+}
+
+extern "C" int pd_gates(const void* h, const void* wa, const void* wb, const void* a_log,
+                        const void* dt_bias, float* gates, int64_t rows, int32_t dim, int32_t hv,
+                        pd_stream_t stream) {
+  pd::clear_error();
+  if (rows < 0 || rows > 0x7fffffff || hv < 1 || hv > 16 * 65535 || dim < 64 || dim % 64)
+    return pd::fail(PD_EINVAL, "input features must be a multiple of 64");
+  if (rows == 0) return PD_OK;
+  if (!h || !wa || !wb || !a_log || !dt_bias || !gates || !all_aligned16(h, wa, wb, gates))
+    return pd::fail(PD_EINVAL, "tensors must be present and 16-byte aligned");
+  const dim3 grid(unsigned((rows + 15) / 16), unsigned((hv + 15) / 16));
+  hipLaunchKernelGGL(gates_kernel, grid, dim3(64 * kGateWaves), 0, as_stream(stream), u16(h), u16(wa),
+                     u16(wb), u16(a_log), u16(dt_bias), gates, rows, dim, hv);
+  return launch_status("pd_gates");
 }
 
 extern "C" int pd_delta_rule(const float* act, const float* gates, float* state, float* out,
                              int32_t batch, int32_t steps, int32_t hk, int32_t hv, int32_t dk,
-                             int32_t dv, int32_t has_prev, int32_t lanes, pd_stream_t stream) {
+                             int32_t dv, int32_t has_prev, pd_stream_t stream) {
   pd::clear_error();
   if (batch < 1 || batch > 65535 || steps < 1 || hk < 1 || hv < 1 || hv > 65535 || hv % hk)
     return pd::fail(PD_EINVAL, "batch, steps and heads must be positive, value heads a multiple");
   if (!valid_linear_dims(dk, dv)) return pd::fail(PD_EINVAL, "linear heads of 64 or 128 elements");
   if (!act || !gates || !state || !out || !all_aligned16(act, gates, state, out))
     return pd::fail(PD_EINVAL, "tensors must be present and 16-byte aligned");
-  if (lanes != 16 && (lanes != 32 || dk != 128))
-    return pd::fail(PD_EINVAL, "16 lanes a column, or 32 at 128 elements");
   const DeltaArgs p{act, gates, state, out, steps, hk, hv, has_prev};
-  const dim3 grid(unsigned(dv * lanes / 128), unsigned(hv), unsigned(batch));
+  const dim3 grid(unsigned(dv / 8), unsigned(hv), unsigned(batch));
   const auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(128), 0, as_stream(stream), p);
   };
   if (dk == 64)
-    dv == 64 ? go(delta_kernel<64, 64, 16>) : go(delta_kernel<64, 128, 16>);
-  else if (lanes == 16)
-    dv == 64 ? go(delta_kernel<128, 64, 16>) : go(delta_kernel<128, 128, 16>);
+    dv == 64 ? go(delta_kernel<64, 64>) : go(delta_kernel<64, 128>);
   else
-    dv == 64 ? go(delta_kernel<128, 64, 32>) : go(delta_kernel<128, 128, 32>);
+    dv == 64 ? go(delta_kernel<128, 64>) : go(delta_kernel<128, 128>);
   return launch_status("pd_delta_rule");
 }
 

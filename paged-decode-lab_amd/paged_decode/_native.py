@@ -56,9 +56,11 @@ SIGNATURES = {
     "pd_gated_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
     "pd_silu_mul": [_vp, _vp, _vp, _i64, _vp],
     "pd_sigmoid_gate": [_vp, _vp, _i64, _vp, _i64, _i32, _vp],
-    "pd_conv_gates": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32,
-                      _i32, _i32, _vp],
-    "pd_delta_rule": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp],
+    "pd_conv": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp],
+    "pd_gates": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _vp],
+    "pd_delta_rule": [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp],
+    "pd_delta_chunks": [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp],
+    "pd_delta_workspace": [_i32, _i32, _i32, _i32, _i32, ctypes.POINTER(_i64)],
     "pd_rope_table": [_vp, _vp, _i32, _vp, _i32, _i32, _vp],
     "pd_qk_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp,
                    _i32, _i32, _i32, _i32, _i32, _i32, _dbl, _vp],
@@ -300,17 +302,33 @@ def sigmoid_gate(x, gate, out, rows, cols):
                                 cols, stream_handle(x.device)))
 
 
-def conv_gates(x, taps, a, b, a_log, dt_bias, conv_state, act, gates, batch, steps, hk, hv, dk, dv,
-               has_prev):
-    check(lib().pd_conv_gates(x.data_ptr(), taps.data_ptr(), a.data_ptr(), b.data_ptr(),
-                              a_log.data_ptr(), dt_bias.data_ptr(), conv_state.data_ptr(),
-                              act.data_ptr(), gates.data_ptr(), batch, steps, hk, hv, dk, dv,
-                              int(has_prev), stream_handle(x.device)))
+def conv(x, taps, conv_state, act, batch, steps, hk, hv, dk, dv, has_prev):
+    check(lib().pd_conv(x.data_ptr(), taps.data_ptr(), conv_state.data_ptr(), act.data_ptr(), batch,
+                        steps, hk, hv, dk, dv, int(has_prev), stream_handle(x.device)))
 
 
-def delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, has_prev, lanes):
+def gates(h, wa, wb, a_log, dt_bias, out):
+    """out float32 [N, hv, 2] = (log decay, beta) of h [N, dim]."""
+    check(lib().pd_gates(h.data_ptr(), wa.data_ptr(), wb.data_ptr(), a_log.data_ptr(),
+                         dt_bias.data_ptr(), out.data_ptr(), h.shape[0], h.shape[1], wa.shape[0],
+                         stream_handle(h.device)))
+
+
+def delta_workspace(batch, steps, hv, dk, dv):
+    floats = _i64(0)
+    check(lib().pd_delta_workspace(batch, steps, hv, dk, dv, ctypes.byref(floats)))
+    return floats.value
+
+
+def delta_chunks(act, gates, state, out, workspace, batch, steps, hk, hv, dk, dv, has_prev):
+    check(lib().pd_delta_chunks(act.data_ptr(), gates.data_ptr(), state.data_ptr(), out.data_ptr(),
+                                workspace.data_ptr(), batch, steps, hk, hv, dk, dv, int(has_prev),
+                                stream_handle(act.device)))
+
+
+def delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, has_prev):
     check(lib().pd_delta_rule(act.data_ptr(), gates.data_ptr(), state.data_ptr(), out.data_ptr(),
-                              batch, steps, hk, hv, dk, dv, int(has_prev), lanes,
+                              batch, steps, hk, hv, dk, dv, int(has_prev),
                               stream_handle(act.device)))
 
 

@@ -21,6 +21,7 @@ from .prefill import batched_prefill
 
 MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
 TOKEN_ROWS = 16         # rows of one MFMA operand
+CHUNK_STEPS = 96        # tokens from which the delta rule is faster in chunks (one sequence)
 
 
 def _plain_module(module, kind):
@@ -137,7 +138,7 @@ def decoder_weights(model, device):
     hk, hv = cfg.linear_num_key_heads, cfg.linear_num_value_heads
     dk, dv, hid, mid = (cfg.linear_key_head_dim, cfg.linear_value_head_dim, cfg.hidden_size,
                         cfg.intermediate_size)
-    if (cfg._attn_implementation != "paged_decode_lab_hip" or hid % 8 or hid > MAX_HIDDEN or mid % 8
+    if (cfg._attn_implementation != "paged_decode_lab_hip" or hid % 64 or hid > MAX_HIDDEN or mid % 8
             or dk not in (64, 128) or dv not in (64, 128) or hk < 1 or hv % hk
             or cfg.head_dim not in (64, 128, 256)):
         return None
@@ -206,27 +207,23 @@ def decoder_states(runner, weights, steps):
     return found
 
 
-def _delta_lanes(columns, dk, device):
-    """Lanes per state column: 32 halve the chain of a token where the columns leave the
-    SIMDs idle, 16 take less work in all."""
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
-    return 32 if dk == 128 and columns <= 8 * cus else 16
-
-
 def _linear_attention(h, w, weights, states, batch, steps):
     hk, hv, dk, dv = weights.linear
     qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
     conv, state, held = states
     mixed, gate = F.linear(h, qkv), F.linear(h, z)
-    beta, decay = F.linear(h, b), F.linear(h, a)
     rows = batch * steps
     act = torch.empty((rows, mixed.shape[1]), device=h.device, dtype=torch.float32)
     gates = torch.empty((rows, hv, 2), device=h.device, dtype=torch.float32)
-    _native.conv_gates(mixed, taps, decay, beta, a_log, dt_bias, conv, act, gates, batch, steps,
-                       hk, hv, dk, dv, held)
+    _native.conv(mixed, taps, conv, act, batch, steps, hk, hv, dk, dv, held)
+    _native.gates(h, a, b, a_log, dt_bias, gates)
     out = torch.empty((rows, hv * dv), device=h.device, dtype=torch.float32)
-    _native.delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, held,
-                       _delta_lanes(batch * hv * dv, dk, h.device))
+    if steps >= CHUNK_STEPS:
+        work = torch.empty(_native.delta_workspace(batch, steps, hv, dk, dv), device=h.device,
+                           dtype=torch.float32)
+        _native.delta_chunks(act, gates, state, out, work, batch, steps, hk, hv, dk, dv, held)
+    else:
+        _native.delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, held)
     y = torch.empty((rows, hv * dv), device=h.device, dtype=torch.bfloat16)
     _native.gated_norm(out, gate, norm, y, rows * hv, dv, eps)
     return F.linear(y, out_proj)

@@ -64,13 +64,13 @@ def linear_case(batch, steps, hk, hv, dk, dv, seed):
     gen = torch.Generator(device="cuda").manual_seed(seed)
     c = 2 * hk * dk + hv * dv
     return dict(x=bf16(gen, batch, steps, c), taps=bf16(gen, c, 1, 4, scale=0.3),
-                a=bf16(gen, batch, steps, hv, scale=3), b=bf16(gen, batch, steps, hv),
-                a_log=bf16(gen, hv), dt=bf16(gen, hv, scale=2),
+                decay=-3 * torch.rand((batch, steps, hv), generator=gen, device="cuda") ** 3,
+                beta=torch.rand((batch, steps, hv), generator=gen, device="cuda"),
                 conv=bf16(gen, batch, c, 4),
                 state=torch.randn((batch, hv, dk, dv), generator=gen, device="cuda") * 0.1)
 
 
-def linear_exact(t, hk, hv, dk, dv, held):
+def conv_exact(t, hk, hv, dk, dv, held):
     x, taps = t["x"].double(), t["taps"].double()[:, 0]
     batch, steps, c = x.shape
     prev = t["conv"].double().transpose(1, 2) if held else torch.zeros(batch, 4, c, device="cuda").double()
@@ -79,42 +79,85 @@ def linear_exact(t, hk, hv, dk, dv, held):
     unit = lambda y: y * torch.rsqrt(y.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
     q, k, v = act.split([hk * dk, hk * dk, hv * dv], -1)
     q, k = unit(q.reshape(batch, steps, hk, dk)) * dk ** -0.5, unit(k.reshape(batch, steps, hk, dk))
-    decay = torch.exp(-t["a_log"].double().exp() * F.softplus(t["a"].double() + t["dt"].double()))
-    return (q, k, v.reshape(batch, steps, hv, dv), decay, torch.sigmoid(t["b"].double()),
-            full[:, -4:].transpose(1, 2))
+    return q, k, v.reshape(batch, steps, hv, dv), full[:, -4:].transpose(1, 2)
 
 
-@pytest.mark.parametrize("hk,hv,dk,dv", [(4, 4, 64, 64), (2, 4, 128, 128), (1, 2, 64, 128), (3, 3, 128, 64)])
-@pytest.mark.parametrize("batch,steps,held", [(1, 1, False), (2, 1, True), (2, 3, False), (1, 3, True),
-                                              (1, 16, True), (2, 17, False), (1, 50, False)])
+def delta_exact(q, k, v, decay, beta, state):
+    """The recurrence in 64 bits: (outputs, last state)."""
+    group = v.shape[2] // q.shape[2]
+    q, k = q.repeat_interleave(group, 2), k.repeat_interleave(group, 2)
+    out = torch.empty_like(v)
+    for i in range(q.shape[1]):
+        state = state * decay[:, i, :, None, None].exp()
+        d = (v[:, i] - (k[:, i, :, :, None] * state).sum(-2)) * beta[:, i, :, None]
+        state = state + k[:, i, :, :, None] * d[:, :, None]
+        out[:, i] = (q[:, i, :, :, None] * state).sum(-2)
+    return out, state
+
+
+HEADS = pytest.mark.parametrize("hk,hv,dk,dv", [(4, 4, 64, 64), (2, 4, 128, 128), (1, 2, 64, 128),
+                                                (3, 3, 128, 64)])
+
+
+@HEADS
+@pytest.mark.parametrize("batch,steps,held", [(1, 1, False), (2, 1, True), (2, 2, False), (2, 3, True),
+                                              (1, 16, True), (2, 17, False), (1, 63, False),
+                                              (1, 64, False), (2, 70, False), (1, 300, False)])
 def test_conv_and_delta_rule(hk, hv, dk, dv, batch, steps, held):
     t = linear_case(batch, steps, hk, hv, dk, dv, steps + dk)
-    q, k, v, decay, beta, conv = linear_exact(t, hk, hv, dk, dv, held)
-    rows, c = batch * steps, t["x"].shape[-1]
-    act = torch.empty(batch, steps, c, device="cuda")
-    gates = torch.empty(batch, steps, hv, 2, device="cuda")
-    state = t["state"].clone()
-    _native.conv_gates(t["x"], t["taps"], t["a"], t["b"], t["a_log"], t["dt"], t["conv"], act, gates,
-                       batch, steps, hk, hv, dk, dv, held)
+    q, k, v, conv = conv_exact(t, hk, hv, dk, dv, held)
+    act = torch.empty(batch, steps, t["x"].shape[-1], device="cuda")
+    gates = torch.stack([t["decay"], t["beta"]], -1).contiguous()
+    _native.conv(t["x"], t["taps"], t["conv"], act, batch, steps, hk, hv, dk, dv, held)
     assert torch.equal(t["conv"].double(), conv)
     ref = torch.cat([q.flatten(2), k.flatten(2), v.flatten(2)], -1)
     close(act, ref, 1e-6 * (ref.abs() + 1))
-    close(gates[..., 0], decay, 4e-6 * (decay + 0.01))
-    close(gates[..., 1], beta, 1e-6)
-    ref = state.double() if held else torch.zeros_like(state).double()
-    want = torch.empty(batch, steps, hv, dv, device="cuda", dtype=torch.float64)
-    q, k = q.repeat_interleave(hv // hk, 2), k.repeat_interleave(hv // hk, 2)
-    for i in range(steps):
-        ref = ref * decay[:, i, :, None, None]
-        d = (v[:, i] - (k[:, i, :, :, None] * ref).sum(-2)) * beta[:, i, :, None]
-        ref = ref + k[:, i, :, :, None] * d[:, :, None]
-        want[:, i] = (q[:, i, :, :, None] * ref).sum(-2)
-    for lanes in (16, 32) if dk == 128 else (16,):
-        s, out = state.clone(), torch.empty(batch, steps, hv, dv, device="cuda")
-        _native.delta_rule(act, gates, s, out, batch, steps, hk, hv, dk, dv, held, lanes)
-        # the state stays below about 4; its float32 error grows with the steps it remembers
-        close(s, ref, 2e-6 * (1 + ref.abs()) * min(steps, 16))
-        close(out, want, 2e-6 * (1 + want.abs()) * min(steps, 16))
+    q, k, v = (a.double().reshape(batch, steps, -1, d) for a, d in
+               zip(act.split([hk * dk, hk * dk, hv * dv], -1), (dk, dk, dv)))
+    start = t["state"].double() if held else torch.zeros_like(t["state"]).double()
+    want, ref = delta_exact(q, k, v, t["decay"].double(), t["beta"].double(), start)
+    work = torch.full((_native.delta_workspace(batch, steps, hv, dk, dv),), float("nan"), device="cuda")
+    forms = [lambda s, o: _native.delta_chunks(act, gates, s, o, work, batch, steps, hk, hv, dk, dv, held)]
+    forms.append(lambda s, o: _native.delta_rule(act, gates, s, o, batch, steps, hk, hv, dk, dv, held))
+    for form in forms:
+        s, out = t["state"].clone(), torch.empty(batch, steps, hv, dv, device="cuda")
+        form(s, out)
+        # values of order 1, sums of up to 128 terms, remembered for some tens of tokens
+        close(s, ref, 4e-6 * (1 + ref.abs()))
+        close(out, want, 4e-6 * (1 + want.abs()))
+
+
+def test_delta_rule_forgets_without_overflow():
+    """Log decays from 0 to -1000 in one chunk: ratios of decays neither over- nor underflow
+    into the tokens that remember, and infinite decay clears the state."""
+    t = linear_case(1, 130, 2, 2, 128, 128, 5)
+    t["decay"][0, :, 0] = torch.where(torch.arange(130, device="cuda") % 9 == 4, -1000.0, -1e-3)
+    t["decay"][0, 70, 1] = -1e30
+    q, k, v, _ = conv_exact(t, 2, 2, 128, 128, False)
+    act = torch.cat([q.flatten(2), k.flatten(2), v.flatten(2)], -1).float()
+    gates = torch.stack([t["decay"], t["beta"]], -1).contiguous()
+    q, k, v = (a.double().reshape(1, 130, 2, 128) for a in act.split(256, -1))
+    want, ref = delta_exact(q, k, v, t["decay"].double(), t["beta"].double(),
+                            torch.zeros_like(t["state"]).double())
+    work = torch.empty(_native.delta_workspace(1, 130, 2, 128, 128), device="cuda")
+    s, out = t["state"].clone(), torch.empty(1, 130, 2, 128, device="cuda")
+    _native.delta_chunks(act, gates, s, out, work, 1, 130, 2, 2, 128, 128, False)
+    close(s, ref, 4e-6 * (1 + ref.abs()))
+    close(out, want, 4e-6 * (1 + want.abs()))
+
+
+@pytest.mark.parametrize("rows,dim,hv", [(1, 64, 4), (17, 256, 16), (40, 2048, 16), (33, 576, 20)])
+def test_gates(rows, dim, hv):
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    h, wa, wb = bf16(gen, rows, dim), bf16(gen, hv, dim, scale=0.05), bf16(gen, hv, dim, scale=0.05)
+    a_log, dt = bf16(gen, hv), bf16(gen, hv, scale=3)
+    out = torch.empty(rows, hv, 2, device="cuda")
+    _native.gates(h, wa, wb, a_log, dt, out)
+    a, b = h.double() @ wa.double().T, h.double() @ wb.double().T
+    # float32 products of up to 2048 terms of size about 0.05
+    ref = -a_log.double().exp() * F.softplus(a + dt.double())
+    close(out[..., 0], ref, 2e-5 * (0.1 + ref.abs()) * a_log.double().exp().clamp(min=1))
+    close(out[..., 1], torch.sigmoid(b), 1e-5 + 0 * b)
 
 
 @pytest.mark.parametrize("d,half", [(64, 8), (128, 64), (256, 32)])
