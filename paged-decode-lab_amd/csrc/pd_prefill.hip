@@ -10,8 +10,8 @@
 // sum as well, at four matrix units per score where 16-bit probabilities
 // would take two.
 //
-// Split of the work.  A workgroup of four wavefronts serves kRows = 128 packed
-// rows of one kv head of one sequence; packed row r is query head r % G of the
+// Split of the work.  A workgroup of four wavefronts serves 128 packed rows (64
+// at head_dim 256) of one kv head of one sequence; packed row r is query head r % G of the
 // kv head's group and token r / G, so any group size fills the rows and all of
 // a workgroup's rows read the same K and V.  A wavefront owns 32 rows and
 // multiplies transposed: S^T = K Q^T and O^T = V^T P^T with 32 x 32 x 16 MFMAs.
@@ -20,16 +20,30 @@
 // i) is the operand layout of P^T up to an order of the keys that the V reads
 // follow: no probability crosses a lane or the LDS.
 //
+// At head_dim 256 the O and Q of 32 rows alone are 192 registers a lane, which
+// leaves one wavefront a SIMD and nothing to run under its waits.  There two
+// wavefronts share 32 rows: each takes half of D in the scores, whose halves
+// are added through LDS, and half of the columns of O.
+//
 // K and V tiles of 16 KB each are double-buffered in LDS: the next tile's rows
 // are loaded to registers before a tile's MFMAs and written after them, one
 // barrier a tile.  The loads are buffer loads whose range ends at the last
 // live row, so rows past the sequence, pages outside the pool and entries past
 // the table's width read as zeros and never touch other memory.
 //
+// What bounds it: instructions.  A 32 x 32 tile of scores at head_dim 128 is 32
+// MFMAs (1024 clocks) and, an element, an FMA, an exponential, an addition, half
+// a maximum and 5.5 operations of the split, about 160 vector instructions (640
+// clocks and the exponentials' 190); counters show half of the SIMDs' time in
+// either, little of it at once.  So the split is the cheap one and a row tile
+// that met 0 x infinity is taken again with the other; masks are a branch in
+// the tiles that need them.
+//
 // Measured on MI355X, K/V write included: four prompts of 17 to 2048 tokens, Hq
-// 32 / Hkv 8 / D 128, 3964 -> 210 us (float32 products of the materialized
-// scores before); 1000 tokens after 3072 cached, Hq 16 / Hkv 4 / D 256, 1144
-// -> 171 us.
+// 32 / Hkv 8 / D 128, 3964 -> 204 us (float32 products of the materialized
+// scores before; 210 with the longer split and masks in line); 1000 tokens after
+// 3072 cached, Hq 16 / Hkv 4 / D 256, 1144 -> 168 us; 512 tokens, Hq 8 / Hkv 2 /
+// D 256, 31 us in one span (45 with 32 whole rows a wavefront).
 //
 // Few rows leave CUs idle (128 rows of each kv head a workgroup): grid.y > 1
 // cuts each row tile's keys into equal spans whose float32 (m, l, O) partials
@@ -48,7 +62,6 @@ using namespace pdk;
 
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kRows = 128;  // packed rows per workgroup, 32 a wavefront
 
 struct PrefillArgs {
   const uint16_t *q, *k, *v;
@@ -68,8 +81,12 @@ struct Prefill {
   static constexpr int kPieces = D / 8;                  // 16-byte pieces per row
   static constexpr int kLoads = kTile * kPieces / 256;   // pieces per thread, K or V
   static constexpr int kTileBytes = kTile * D * 2;
-  static constexpr int kSteps = D / 16;                  // QK MFMAs per block
-  static constexpr int kOut = D / 32;                    // 32-column blocks of O
+  // D = 256: two wavefronts share 32 rows, each with half of D (see above).
+  static constexpr int kParts = D == 256 ? 2 : 1;
+  static constexpr int kRows = 128 / kParts;             // packed rows per workgroup
+  static constexpr int kCols = D / kParts;               // of a wavefront
+  static constexpr int kSteps = kCols / 16;              // QK MFMAs per block
+  static constexpr int kOut = kCols / 32;                // 32-column blocks of O
 };
 
 // Piece permutation of a V row: a transposed read takes 64 bytes of four
@@ -81,17 +98,24 @@ __device__ __forceinline__ int v_swizzle(int row) {
 }
 
 // p = hi + mid + lo exactly, each a bf16 (the top 16 bits of a float32): every
-// term takes the next eight significant bits, truncated.  Subtracting one from
-// the bits before truncating keeps the remainder of a nonzero p nonzero, so no
-// term of it is zero and an infinite V contributes an infinity, not a NaN.
+// term takes the next eight significant bits, truncated.  kSafe: subtracting
+// one from the bits before truncating keeps the remainder of a nonzero p
+// nonzero, so no term of it is zero and an infinite V contributes an infinity
+// and not the NaN of 0 x infinity.
 struct Split3 {
   uint32_t hi, mid, lo;
 };
+template <bool kSafe>
+__device__ __forceinline__ uint32_t truncated(float x) {
+  const uint32_t u = __float_as_uint(x);
+  return (kSafe ? __builtin_elementwise_sub_sat(u, 1u) : u) & 0xffff0000u;
+}
+template <bool kSafe>
 __device__ __forceinline__ Split3 split3(float p) {
   Split3 s;
-  s.hi = __builtin_elementwise_sub_sat(__float_as_uint(p), 1u) & 0xffff0000u;
+  s.hi = truncated<kSafe>(p);
   const float r = p - __uint_as_float(s.hi);
-  s.mid = __builtin_elementwise_sub_sat(__float_as_uint(r), 1u) & 0xffff0000u;
+  s.mid = truncated<kSafe>(r);
   s.lo = __float_as_uint(r - __uint_as_float(s.mid));
   return s;
 }
@@ -108,6 +132,7 @@ __device__ __forceinline__ floatx16_t mfma32(u32x4_t a, u32x4_t b, floatx16_t c)
 // The sequence and row tile of grid tile `t` (counted from the last), for
 // packed sequences: the tiles of 64 sequences at a time, one a lane, summed by
 // a wavefront prefix.  Returns false past the last tile.
+template <int kRows>
 __device__ __forceinline__ bool find_tile(const PrefillArgs& a, int t, int lane, int& seq,
                                           int& tile) {
   for (int base = 0; base < a.num_seqs; base += 64) {
@@ -139,10 +164,14 @@ __device__ __forceinline__ bool find_tile(const PrefillArgs& a, int t, int lane,
 // kPaged: K and V are pages read through the table, page_size a multiple of
 // the tile; else rows of the call's own tensors.
 template <int D, bool kPaged>
-__global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const PrefillArgs a) {
+__global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
   using P = Prefill<D>;
+  constexpr int kRows = P::kRows;
   __shared__ __attribute__((aligned(16))) char lds[2][2][P::kTileBytes];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ __attribute__((aligned(16))) floatx4_t partial[P::kParts == 2 ? 4 : 1][4][64];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wave % (kRows / 32), part = wave / (kRows / 32);  // rows 32 w, columns of `part`
   const int half = lane >> 5, col = lane & 31;
 
   // Longest first: tiles are counted from the last, whose rows see most keys.
@@ -154,7 +183,7 @@ __global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const Pr
   int64_t q0, k0;
   int nq, nk;
   if (a.cu_q) {
-    if (!find_tile(a, t_rev, lane, seq, tile)) return;
+    if (!find_tile<kRows>(a, t_rev, lane, seq, tile)) return;
     seq = __builtin_amdgcn_readfirstlane(seq);
     tile = __builtin_amdgcn_readfirstlane(tile);
     q0 = max(0, a.cu_q[seq]);
@@ -197,55 +226,56 @@ __global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const Pr
     const uint16_t* qrow = a.q + seq * a.qsb + (q0 + token) * a.qsn + head * a.qsh;
 #pragma unroll
     for (int s = 0; s < P::kSteps; ++s) {
-      qf[s] = load16(qrow + 16 * s + 8 * half);
+      qf[s] = load16(qrow + P::kCols * part + 16 * s + 8 * half);
 #pragma unroll
       for (int e = 0; e < 4; ++e) qf[s][e] ^= flip;
     }
   }
 
-  // Piece i of this thread: row and piece of the tile, LDS position.
-  int src_k[P::kLoads], src_v[P::kLoads], dst_k[P::kLoads], dst_v[P::kLoads];
-#pragma unroll
-  for (int i = 0; i < P::kLoads; ++i) {
-    const int idx = 256 * i + tid, r = idx / P::kPieces, p = idx % P::kPieces;
-    src_k[i] = int((r * a.ksn + 8 * p) * 2);
-    src_v[i] = int((r * a.vsn + 8 * p) * 2);
-    dst_k[i] = r * D * 2 + 16 * (p ^ kswz<D>(r));
-    dst_v[i] = r * D * 2 + 16 * (p ^ v_swizzle<D>(r));
-  }
+  // Piece i of this thread is piece 0 kStep rows further down; the swizzles
+  // repeat within 16 rows, and 8 rows further down K's differs in one bit.
+  constexpr int kStep = 256 / P::kPieces;
+  static_assert(kStep % 16 == 0 || (kStep == 8 && D >= 128), "swizzles by up to four bits of the row");
+  const int row0 = tid / P::kPieces, piece0 = tid % P::kPieces;
+  const int src_k = int((row0 * a.ksn + 8 * piece0) * 2), src_v = int((row0 * a.vsn + 8 * piece0) * 2);
+  const int dst_k = row0 * D * 2 + 16 * (piece0 ^ kswz<D>(row0));
+  const int dst_v = row0 * D * 2 + 16 * (piece0 ^ v_swizzle<D>(row0));
+  const uint16_t* k_first = a.k + kvh * a.ksh + (kPaged ? 0 : seq * a.ksb + k0 * a.ksn);
+  const uint16_t* v_first = a.v + kvh * a.vsh + (kPaged ? 0 : seq * a.vsb + k0 * a.vsn);
   u32x4_t kr[P::kLoads], vr[P::kLoads];
   const auto fetch = [&](int t) {
     const int first = t * P::kTile;
-    int live = min(P::kTile, nk - first);
-    int64_t page = 0, slot = 0;
+    int live = min(P::kTile, nk - first), slot = first;
+    const uint16_t *kp = k_first, *vp = v_first;
     if constexpr (kPaged) {
-      page = a.table[seq * a.tsb + first / a.page_size];
+      int64_t page = a.table[seq * a.tsb + first / a.page_size];
       slot = first % a.page_size;
       if (page < 0 || page >= a.num_pages) live = 0, page = 0;
-    } else {
-      page = seq;
-      slot = k0 + first;
+      kp += page * a.ksb, vp += page * a.vsb;
     }
-    const uint16_t* kp = a.k + page * a.ksb + slot * a.ksn + kvh * a.ksh;
-    const uint16_t* vp = a.v + page * a.vsb + slot * a.vsn + kvh * a.vsh;
+    kp += slot * a.ksn, vp += slot * a.vsn;
     const auto rk = buffer_rsrc(kp, int(live * a.ksn * 2));
     const auto rv = buffer_rsrc(vp, int(live * a.vsn * 2));
+    // Opaque to the compiler, which would keep every sum in a register.
+    int step_k = int(kStep * a.ksn * 2), step_v = int(kStep * a.vsn * 2);
+    asm volatile("" : "+s"(step_k), "+s"(step_v));
 #pragma unroll
-    for (int i = 0; i < P::kLoads; ++i) kr[i] = buffer_load16(rk, src_k[i]);
+    for (int i = 0; i < P::kLoads; ++i) kr[i] = buffer_load16(rk, src_k + i * step_k);
 #pragma unroll
-    for (int i = 0; i < P::kLoads; ++i) vr[i] = buffer_load16(rv, src_v[i]);
+    for (int i = 0; i < P::kLoads; ++i) vr[i] = buffer_load16(rv, src_v + i * step_v);
   };
   const auto place = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < P::kLoads; ++i) *reinterpret_cast<u32x4_t*>(lds[b][0] + dst_k[i]) = kr[i];
+    for (int i = 0; i < P::kLoads; ++i)
+      *reinterpret_cast<u32x4_t*>(lds[b][0] + (dst_k ^ (kStep == 8 && i % 2 ? 128 : 0)) +
+                                  i * kStep * D * 2) = kr[i];
 #pragma unroll
-    for (int i = 0; i < P::kLoads; ++i) *reinterpret_cast<u32x4_t*>(lds[b][1] + dst_v[i]) = vr[i];
+    for (int i = 0; i < P::kLoads; ++i)
+      *reinterpret_cast<u32x4_t*>(lds[b][1] + dst_v + i * kStep * D * 2) = vr[i];
   };
 
   floatx16_t o[P::kOut];
-#pragma unroll
-  for (int j = 0; j < P::kOut; ++j) o[j] = floatx16_t{};
-  float m = -INFINITY, l = 0.f;  // m in units of log2; l of this lane's keys
+  float m, l;  // m in units of log2; l of this lane's keys
 
   // Transposed V reads: lane's row of a 16-key group and its byte in the row
   // for 32-column blocks j = 0..3 (mod 4).
@@ -253,108 +283,154 @@ __global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const Pr
   int vat[P::kOut < 4 ? P::kOut : 4];
 #pragma unroll
   for (int j = 0; j < (P::kOut < 4 ? P::kOut : 4); ++j) {
-    const int piece = 4 * j + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    const int piece = P::kCols / 8 * part + 4 * j + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
     vat[j] = vrow * D * 2 + 16 * (piece ^ v_swizzle<D>(vrow)) + 8 * (lane & 1);
   }
 
-  if (t_begin < t_end) {
-    fetch(t_begin);
-    place(0);
-  }
-  for (int t = t_begin; t < t_end; ++t) {
-    const int b = (t - t_begin) & 1;
-    __syncthreads();
-    if (t + 1 < t_end) fetch(t + 1);
-    const int first = t * P::kTile;
-    if (first <= wave_last) {
-      const char* ks = lds[b][0];
-      const char* vs = lds[b][1];
-      floatx16_t s[P::kBlocks];
+  const auto sweep = [&](auto safe) {
+    constexpr bool kSafe = decltype(safe)::value;
 #pragma unroll
-      for (int n = 0; n < P::kBlocks; ++n) {
-        s[n] = floatx16_t{};
-        const int r = 32 * n + col;
+    for (int j = 0; j < P::kOut; ++j) o[j] = floatx16_t{};
+    m = -INFINITY, l = 0.f;
+    if (t_begin < t_end) {
+      fetch(t_begin);
+      place(0);
+    }
+    for (int t = t_begin; t < t_end; ++t) {
+      const int b = (t - t_begin) & 1;
+      __syncthreads();
+      if (t + 1 < t_end) fetch(t + 1);
+      const int first = t * P::kTile;
+      if (P::kParts == 2 || first <= wave_last) {
+        const char* ks = lds[b][0];
+        const char* vs = lds[b][1];
+        // Two sums in turn (32-key blocks, or halves of the contraction): a
+        // product right behind the one it adds to waits for its result.
+        floatx16_t s[2] = {};
+        constexpr int kChain = P::kBlocks == 2 ? 1 : 2;
 #pragma unroll
-        for (int d = 0; d < P::kSteps; ++d) {
-          const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
-              ks + r * D * 2 + 16 * ((2 * d + half) ^ kswz<D>(r)));
-          s[n] = mfma32(kf, qf[d], s[n]);
+        for (int d = 0; d < P::kSteps; d += kChain)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            const int r = (P::kBlocks == 2 ? 32 * n : 0) + col, step = d + (kChain == 2 ? n : 0);
+            const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
+                ks + r * D * 2 + P::kCols * 2 * part + 16 * ((2 * step + half) ^ kswz<D>(r)));
+            s[n] = mfma32(kf, qf[step], s[n]);
+          }
+        if constexpr (P::kBlocks == 1) s[0] += s[1];
+        if constexpr (P::kParts == 2) {
+          // The two halves of the contraction meet in LDS; both wavefronts add
+          // them in the same order and go on with the same scores.
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            partial[wave][g][lane] =
+                floatx4_t{s[0][4 * g], s[0][4 * g + 1], s[0][4 * g + 2], s[0][4 * g + 3]};
+          lds_barrier();
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const floatx4_t other = partial[wave ^ 2][g][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[0][4 * g + e] += other[e];
+          }
         }
-      }
-      // Keys past the row's limit, only in tiles that reach past the first
-      // row's: their scores leave the maximum and their probabilities are 0.
-      const bool edge = first + P::kTile - 1 > wave_first;
-      if (edge) {
+        // Keys past the row's limit, only in tiles that reach past the first
+        // row's: their scores leave the maximum and their probabilities are 0.
+        const bool edge = first + P::kTile - 1 > wave_first;
+        if (edge) {
+          asm volatile("");  // a branch, not selects in every tile
+#pragma unroll
+          for (int n = 0; n < P::kBlocks; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              if (first + 32 * n + 8 * (i / 4) + 4 * half + i % 4 > limit) s[n][i] = -INFINITY;
+        }
+        float top = s[0][0];
 #pragma unroll
         for (int n = 0; n < P::kBlocks; ++n)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (first + 32 * n + 8 * (i / 4) + 4 * half + i % 4 > limit) s[n][i] = -INFINITY;
-      }
-      float top = s[0][0];
+          for (int i = 0; i < 16; ++i) top = fmaxf(top, s[n][i]);
+        top = fmaxf(top, xor_lanes<32>(top, lane));
+        // A scale of 0 leaves a zero score where a masked row's top is -inf.
+        const float mt = top == -INFINITY ? -INFINITY : top * c;
+        // The running maximum moves only when a row's grows by more than 2^8:
+        // the probabilities stay below 2^8 and the sums are the same.
+        if (__any(mt > m + 8.f)) {
+          const float up = fmaxf(m, mt);
+          const float f = exp2_fast(m - (up == -INFINITY ? 0.f : up));
+          m = up;
+          l *= f;
 #pragma unroll
-      for (int n = 0; n < P::kBlocks; ++n)
+          for (int j = 0; j < P::kOut; ++j)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) top = fmaxf(top, s[n][i]);
-      top = fmaxf(top, xor_lanes<32>(top, lane));
-      // A scale of 0 leaves a zero score where a masked row's top is -inf.
-      const float mt = top == -INFINITY ? -INFINITY : top * c;
-      // The running maximum moves only when a row's grows by more than 2^8:
-      // the probabilities stay below 2^8 and the sums are the same.
-      if (__any(mt > m + 8.f)) {
-        const float up = fmaxf(m, mt);
-        const float f = exp2_fast(m - (up == -INFINITY ? 0.f : up));
-        m = up;
-        l *= f;
-#pragma unroll
-        for (int j = 0; j < P::kOut; ++j)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[j][i] *= f;
-      }
-      const float base = m == -INFINITY ? 0.f : m;
-#pragma unroll
-      for (int n = 0; n < P::kBlocks; ++n) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[n][i] = exp2_fast(fmaf(s[n][i], c, -base));
-        if (edge) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (first + 32 * n + 8 * (i / 4) + 4 * half + i % 4 > limit) s[n][i] = 0.f;
+            for (int i = 0; i < 16; ++i) o[j][i] *= f;
         }
+        const float base = m == -INFINITY ? 0.f : m;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) l += s[n][i];
+        for (int n = 0; n < P::kBlocks; ++n) {
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {  // 16 keys a step
-          u32x4_t hi, mid, lo;
+          for (int i = 0; i < 16; ++i) s[n][i] = exp2_fast(fmaf(s[n][i], c, -base));
+          if (edge) {
+          asm volatile("");  // a branch, not selects in every tile
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const Split3 x = split3(s[n][8 * g + 2 * e]), y = split3(s[n][8 * g + 2 * e + 1]);
-            hi[e] = upper_halves(x.hi, y.hi);
-            mid[e] = upper_halves(x.mid, y.mid);
-            lo[e] = upper_halves(x.lo, y.lo);
+            for (int i = 0; i < 16; ++i)
+              if (first + 32 * n + 8 * (i / 4) + 4 * half + i % 4 > limit) s[n][i] = 0.f;
           }
-          const char* vg = vs + (32 * n + 16 * g) * D * 2;
 #pragma unroll
-          for (int j = 0; j < P::kOut; ++j) {
-            const char* p = vg + vat[j & 3] + 256 * (j >> 2);
-            const short4_t v0 = lds_read_tr(p), v1 = lds_read_tr(p + 8 * D * 2);
-            const uint64_t a0 = __builtin_bit_cast(uint64_t, v0), a1 = __builtin_bit_cast(uint64_t, v1);
-            const u32x4_t vf = {uint32_t(a0), uint32_t(a0 >> 32), uint32_t(a1), uint32_t(a1 >> 32)};
-            o[j] = mfma32(vf, lo, o[j]);
-            o[j] = mfma32(vf, mid, o[j]);
-            o[j] = mfma32(vf, hi, o[j]);
+          for (int i = 0; i < 16; ++i) l += s[n][i];
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {  // 16 keys a step
+            u32x4_t hi, mid, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const Split3 x = split3<kSafe>(s[n][8 * g + 2 * e]),
+                           y = split3<kSafe>(s[n][8 * g + 2 * e + 1]);
+              hi[e] = upper_halves(x.hi, y.hi);
+              mid[e] = upper_halves(x.mid, y.mid);
+              lo[e] = upper_halves(x.lo, y.lo);
+            }
+            const char* vg = vs + (32 * n + 16 * g) * D * 2;
+            u32x4_t vf[P::kOut];
+#pragma unroll
+            for (int j = 0; j < P::kOut; ++j) {
+              const char* p = vg + vat[j & 3] + 256 * (j >> 2);
+              const short4_t v0 = lds_read_tr(p), v1 = lds_read_tr(p + 8 * D * 2);
+              const uint64_t a0 = __builtin_bit_cast(uint64_t, v0), a1 = __builtin_bit_cast(uint64_t, v1);
+              vf[j] = u32x4_t{uint32_t(a0), uint32_t(a0 >> 32), uint32_t(a1), uint32_t(a1 >> 32)};
+            }
+#pragma unroll
+            for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], lo, o[j]);
+#pragma unroll
+            for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], mid, o[j]);
+#pragma unroll
+            for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], hi, o[j]);
           }
         }
       }
+      if (t + 1 < t_end) place(b ^ 1);
     }
-    if (t + 1 < t_end) place(b ^ 1);
-  }
 
-  // The loop's last MFMAs and the reads below are in different blocks: 24 wait
-  // states cover them.
-  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+    // The loop's last MFMAs and the reads below are in different blocks: 24 wait
+    // states cover them.
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #pragma unroll
-  for (int j = 0; j < P::kOut; ++j) asm volatile("" : "+v"(o[j]));
+    for (int j = 0; j < P::kOut; ++j) asm volatile("" : "+v"(o[j]));
+  };
+  sweep(std::false_type{});
+  // A NaN may be a zero term times an infinity: such row tiles are taken again
+  // with terms that are not zero.
+  float odd = 0.f;
+#pragma unroll
+  for (int j = 0; j < P::kOut; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) odd = fmaf(o[j][i], 0.f, odd);  // NaN of an infinity too
+  int* flags = reinterpret_cast<int*>(&lds[0][0][0]);
+  __syncthreads();
+  const int any_odd = __any(odd != 0.f);
+  if (lane == 0) flags[wave] = any_odd;
+  __syncthreads();
+  const bool again = flags[0] | flags[1] | flags[2] | flags[3];
+  __syncthreads();
+  if (again) sweep(std::true_type{});
   l += xor_lanes<32>(l, lane);
 
   if (a.splits > 1) {
@@ -367,9 +443,9 @@ __global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const Pr
       for (int j = 0; j < P::kOut; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<floatx4_t*>(po + 32 * j + 8 * g + 4 * half) =
+          *reinterpret_cast<floatx4_t*>(po + P::kCols * part + 32 * j + 8 * g + 4 * half) =
               floatx4_t{o[j][4 * g], o[j][4 * g + 1], o[j][4 * g + 2], o[j][4 * g + 3]};
-      if (half == 0) {
+      if (half == 0 && part == 0) {
         a.part_ml[2 * pr] = m;
         a.part_ml[2 * pr + 1] = l;
       }
@@ -380,26 +456,31 @@ __global__ void __launch_bounds__(256, D == 256 ? 1 : 2) prefill_kernel(const Pr
   // Output rows through LDS (each wavefront its own 32, after every wavefront
   // has read its last tile), stored 16 bytes a lane.
   __syncthreads();
-  char* stage = &lds[0][0][0] + w * 32 * D * 2;
+  char* stage = &lds[0][0][0] + wave * 32 * P::kCols * 2;
   const float inv = 1.f / l;
 #pragma unroll
   for (int j = 0; j < P::kOut; ++j)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int piece = 4 * j + g;
-      uint32_t* d = reinterpret_cast<uint32_t*>(stage + col * D * 2 +
+      uint32_t* d = reinterpret_cast<uint32_t*>(stage + col * P::kCols * 2 +
                                                 16 * (piece ^ (col & 7)) + 8 * half);
-      d[0] = bf16_bits(o[j][4 * g] * inv) | bf16_bits(o[j][4 * g + 1] * inv) << 16;
-      d[1] = bf16_bits(o[j][4 * g + 2] * inv) | bf16_bits(o[j][4 * g + 3] * inv) << 16;
+      d[0] = pack_bf16(o[j][4 * g] * inv, o[j][4 * g + 1] * inv);
+      d[1] = pack_bf16(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv);
     }
+  // A wavefront's own LDS writes are visible to it in order.
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int kRowPieces = P::kCols / 8;
 #pragma unroll
-  for (int i = 0; i < 32 * P::kPieces / 64; ++i) {
-    const int idx = 64 * i + lane, r = idx / P::kPieces, p = idx % P::kPieces;
+  for (int i = 0; i < 32 * kRowPieces / 64; ++i) {
+    const int idx = 64 * i + lane, r = idx / kRowPieces, p = idx % kRowPieces;
     const int pr = tile * kRows + 32 * w + r;
-    const u32x4_t x = *reinterpret_cast<const u32x4_t*>(stage + r * D * 2 + 16 * (p ^ (r & 7)));
+    const u32x4_t x =
+        *reinterpret_cast<const u32x4_t*>(stage + r * P::kCols * 2 + 16 * (p ^ (r & 7)));
     if (pr < rows)
       *reinterpret_cast<u32x4_t*>(a.out + seq * a.osb + (q0 + pr / a.G) * a.osn +
-                                  (kvh * a.G + pr % a.G) * a.osh + 8 * p) = x;
+                                  (kvh * a.G + pr % a.G) * a.osh + P::kCols * part + 8 * p) = x;
   }
 }
 
@@ -483,7 +564,7 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
   for (int i = 1; i < 3; ++i)
     if (all[i][1] < head_dim || all[i][1] > (int64_t(1) << 23))
       return pd::fail(PD_EINVAL, "k and v token strides must lie in [head_dim, 2^23]");
-  const int tile = head_dim == 256 ? 32 : 64;
+  const int tile = head_dim == 256 ? 32 : 64, kRows = head_dim == 256 ? 64 : 128;
   if (table && (table_width < 1 || num_pages < 1 || page_size < tile || page_size % tile))
     return pd::fail(PD_EINVAL, "the page size must be a multiple of %d tokens", tile);
   const int G = num_heads / num_kv_heads;

@@ -13,7 +13,6 @@ import torch
 from . import _native
 
 HEAD_DIMS = (64, 128, 256)
-ROWS = 128              # packed (token, query head of the group) rows of a workgroup
 
 
 def _plain(*tensors):
@@ -46,17 +45,22 @@ def _heads_ok(hq, hkv, dim, scale):
             and math.isfinite(scale))
 
 
+def _rows(dim):
+    """Packed (token, query head of the group) rows of a workgroup."""
+    return 64 if dim == 256 else 128
+
+
 def _splits(workgroups, max_keys, dim, device):
-    """Key spans per row tile: as many as fill the device's slots (one workgroup a CU at
-    head_dim 256, two below) with the workgroups at hand, of 128 keys or more each at
-    head_dim 256 and 256 below, where a span costs less than its partials.  Measured, one
-    span against the rule's: 269 and 159 us (1000 rows after 3072, Hq 16 / Hkv 4, D 256,
-    128 workgroups, 2 spans), 43 and 30 us (512 rows, Hq 8 / Hkv 2, D 256, 4 spans), 75 and
-    25 us (128 after 2048, Hq 8 / Hkv 2, D 128, 8 spans); two spans where the workgroups
-    fill the slots alone: 101 instead of 88 us (2048 rows, Hq 32 / Hkv 8, D 128)."""
+    """Key spans per row tile, of 256 keys or more each: as many as fill the device's slots
+    (two workgroups a CU), and at head_dim 256, where a workgroup's rows are few and its
+    spans uneven, twice that.  Measured, one span against the rule's: 104 and 78 us (2049
+    rows, Hq 8 / Hkv 2, D 256, 260 workgroups, 4 spans; 2 spans 89), 155 and 37 us (100 rows
+    after 3072, Hq 16 / Hkv 4, D 256, 16 spans), 73 and 24 us (128 after 2048, Hq 8 / Hkv 2,
+    D 128, 8 spans); two spans where the workgroups fill the slots alone: 101 instead of 84
+    us (2048 rows, Hq 32 / Hkv 8, D 128)."""
     cus = torch.cuda.get_device_properties(device).multi_processor_count
-    slots, least = (cus, 128) if dim == 256 else (2 * cus, 256)
-    return max(1, min((slots + workgroups // 2) // workgroups, max_keys // least, 16))
+    slots = 4 * cus if dim == 256 else 2 * cus
+    return max(1, min((slots + workgroups // 2) // workgroups, max_keys // 256, 16))
 
 
 def _workspace(splits, total_q, heads, dim, device):
@@ -82,7 +86,7 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0):
     if n == 0 or seqs < 1:
         return out
     page_size, num_pages = (k.shape[1], k.shape[0]) if tables is not None else (0, 0)
-    splits = _splits((n * (hq // hkv) // ROWS + seqs) * hkv, max_keys, d, q.device)
+    splits = _splits((n * (hq // hkv) // _rows(d) + seqs) * hkv, max_keys, d, q.device)
     part_o, part_ml = _workspace(splits, n, hq, d, q.device)
     rows = lambda t: (t.stride(0) if t.dim() == 4 else 0, t.stride(-3), t.stride(-2))  # noqa: E731
     _native.prefill(q, rows(q), k, rows(k), v, rows(v), out, rows(out), cu_q, cu_k, seqs, 0, n,
@@ -150,7 +154,7 @@ def batched_prefill(query, key, value, scale):
     b, hq, s, d = query.shape
     hkv = key.shape[1]
     out = torch.empty((b, s, hq, d), device=query.device, dtype=query.dtype)
-    splits = _splits(b * -(-s * (hq // hkv) // ROWS) * hkv, s, d, query.device)
+    splits = _splits(b * -(-s * (hq // hkv) // _rows(d)) * hkv, s, d, query.device)
     part_o, part_ml = _workspace(splits, b * s, hq, d, query.device)
     rows = lambda t: (t.stride(0), t.stride(2), t.stride(1))  # noqa: E731
     _native.prefill(query, rows(query), key, rows(key), value, rows(value), out,
