@@ -195,10 +195,14 @@ def _linear_states(cache, index, batch, weights, device):
     return conv, state, held
 
 
-def decoder_states(runner, weights, steps):
+def decoder_states(runner, weights, tokens):
     """The linear-attention states of every layer, or None where the kernels cannot run:
-    several steps on top of earlier tokens, or states of another form."""
+    another batch than the runner's, several steps on top of earlier tokens, or states of
+    another form."""
     cache, found = runner.cache, {}
+    if tokens.dim() != 2 or tokens.shape[0] != runner.batch or tokens.shape[1] < 1:
+        return None
+    steps = tokens.shape[1]
     for index in cache.linear:
         states = _linear_states(cache, index, runner.batch, weights, runner.device)
         if states is None or (states[2] and steps > 1):

@@ -315,7 +315,7 @@ class HybridRunner:
         """Logits of the last token; tokens [B, S] at ``positions`` [S] (device tensors)."""
         weights = decoder_weights(self.model, self.cache.pool.block.device)
         if weights is not None:
-            states = decoder_states(self, weights, tokens.shape[1])
+            states = decoder_states(self, weights, tokens)
             if states is not None:
                 return decoder_forward(self, weights, states, tokens, positions, _decode_attention)
         # Several runners may share one model: the attention layers serve whichever

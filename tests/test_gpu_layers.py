@@ -223,3 +223,14 @@ def test_layers_agree_with_the_modules(hk, hv, dk, dv, length):
     for a, b in zip(results[0][0] + results[0][1] + [results[0][2]],
                     results[1][0] + results[1][1] + [results[1][2]]):
         assert (a.float() - b.float()).norm() <= 0.03 * b.float().norm()
+
+
+def test_other_batches_are_refused_as_before():
+    cfg = H.decoder_config(num_hidden_layers=4, hidden_size=256, intermediate_size=512,
+                           vocab_size=512, linear_num_key_heads=4, linear_key_head_dim=64,
+                           linear_num_value_heads=4, linear_value_head_dim=64)
+    model = H.random_init_model(cfg, "cuda", seed=1)
+    for rows in (1, 3):
+        runner = H.HybridRunner(model=model, backend="hip_matched", batch=2, max_context=300)
+        with pytest.raises((RuntimeError, ValueError)):
+            runner.prefill([[1, 2, 3]] * rows)
