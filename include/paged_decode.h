@@ -367,6 +367,13 @@ int pd_qk_rope(const void* q, const void* k, const void* v, const void* q_weight
                int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t half, double eps,
                pd_stream_t stream);
 
+/* Products of x [rows, dim] with `count` <= 4 weight matrices [features[i],
+ * dim], dim a multiple of 64, features of 4; the arrays are host arrays.  form
+ * 0: outs[i] = x weights[i]^T; form 1 (two matrices of one size): outs[0] =
+ * silu(x weights[0]^T) (x weights[1]^T). */
+int pd_linears(const void* x, int32_t rows, int32_t dim, int32_t count, const void* const* weights,
+               const int32_t* features, void* const* outs, int32_t form, pd_stream_t stream);
+
 /* One token per sequence: products of 1 to 16 rows whose norms, gates,
  * convolution and residual run in the same launch.  dim (the input features)
  * is a multiple of 64; weights are bf16 [features, dim]. */

@@ -64,6 +64,7 @@ SIGNATURES = {
     "pd_rope_table": [_vp, _vp, _i32, _vp, _i32, _i32, _vp],
     "pd_qk_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp,
                    _i32, _i32, _i32, _i32, _i32, _i32, _dbl, _vp],
+    "pd_linears": [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
     "pd_norm_linears": [_vp, _vp, _dbl, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp],
     "pd_norm_gate_up": [_vp, _vp, _dbl, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
     "pd_linear_add": [_vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _vp],
@@ -347,6 +348,19 @@ def qk_rope(q, k, v, q_weight, k_weight, rope, q_out, k_out, k_pages, v_pages, t
                            v_pages.data_ptr(), k_pages.shape[0], tables.data_ptr(),
                            tables.stride(0), tables.shape[1], positions.data_ptr(), batch, steps,
                            hq, hkv, d, half, eps, stream_handle(q.device)))
+
+
+LINEAR_STORE, LINEAR_SILU_MUL = 0, 1
+
+
+def linears(x, weights, outs, form=LINEAR_STORE):
+    """outs[i] = x weights[i]^T, or outs[0] = silu(x gate^T) (x up^T)."""
+    n = len(weights)
+    check(lib().pd_linears(x.data_ptr(), x.shape[0], x.shape[1], n,
+                           (_vp * n)(*[w.data_ptr() for w in weights]),
+                           (_i32 * n)(*[w.shape[0] for w in weights]),
+                           (_vp * n)(*[outs[i % len(outs)].data_ptr() for i in range(n)]), form,
+                           stream_handle(x.device)))
 
 
 def norm_linears(x, norm, eps, weights, outs, taps=None, conv_state=None, has_prev=False):

@@ -211,11 +211,41 @@ def decoder_states(runner, weights, tokens):
     return found
 
 
+def _products(h, *matrices):
+    """h times each matrix: one launch while its 128 x 128 tiles are one round of the CUs
+    (pd_linears), else the library's products."""
+    rows, dim = h.shape
+    features = [m.shape[0] for m in matrices]
+    if not _one_round(rows, dim, features, 128, h.device):
+        return [F.linear(h, m) for m in matrices]
+    outs = [torch.empty((rows, f), device=h.device, dtype=h.dtype) for f in features]
+    _native.linears(h, matrices, outs)
+    return outs
+
+
+def _gate_up(h, gate, up):
+    """silu(h gate^T) (h up^T), on the same rule; 64 features of either are a tile."""
+    rows, dim = h.shape
+    if not _one_round(rows, dim, [gate.shape[0]], 64, h.device):
+        a, b = F.linear(h, gate), F.linear(h, up)
+        _native.silu_mul(a, b, a)
+        return a
+    out = torch.empty((rows, gate.shape[0]), device=h.device, dtype=h.dtype)
+    _native.linears(h, (gate, up), (out,), _native.LINEAR_SILU_MUL)
+    return out
+
+
+def _one_round(rows, dim, features, per_tile, device):
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    tiles = sum(-(-f // per_tile) for f in features) * -(-rows // 128)
+    return tiles <= cus and dim % 64 == 0 and all(f % 4 == 0 for f in features)
+
+
 def _linear_attention(h, w, weights, states, batch, steps):
     hk, hv, dk, dv = weights.linear
     qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
     conv, state, held = states
-    mixed, gate = F.linear(h, qkv), F.linear(h, z)
+    mixed, gate = _products(h, qkv, z)
     rows = batch * steps
     act = torch.empty((rows, mixed.shape[1]), device=h.device, dtype=torch.float32)
     gates = torch.empty((rows, hv, 2), device=h.device, dtype=torch.float32)
@@ -237,7 +267,7 @@ def _full_attention(h, w, weights, rope, runner, batch, steps, attend):
     spec, pool = runner.spec, runner.cache.pool
     hq, hkv, d = spec.num_heads, spec.num_kv_heads, spec.head_dim
     q_proj, k_proj, v_proj, (q_norm, eps), (k_norm, _), o_proj = w.mixer
-    q, k, v = F.linear(h, q_proj), F.linear(h, k_proj), F.linear(h, v_proj)
+    q, k, v = _products(h, q_proj, k_proj, v_proj)
     fill = runner.cache.phase == "prefill"
     query = torch.empty((batch, steps, hq, d), device=h.device, dtype=torch.bfloat16)
     keys = torch.empty((batch, steps, hkv, d), device=h.device, dtype=torch.bfloat16) if fill else None
@@ -326,9 +356,7 @@ def _row_layers(x, runner, weights, states, rope, batch, steps, attend):
         else:
             y = _full_attention(h, w, weights, rope, runner, batch, steps, attend)
         _native.add_rms_norm(x, y, w.post_norm[0], h, w.post_norm[1])
-        gate, up = F.linear(h, w.gate), F.linear(h, w.up)
-        _native.silu_mul(gate, up, gate)
-        y = F.linear(gate, w.down)
+        y = F.linear(_gate_up(h, w.gate, w.up), w.down)
     return y
 
 

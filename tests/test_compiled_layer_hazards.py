@@ -8,7 +8,7 @@ import subprocess
 import pytest
 from test_compiled_hazards import CSRC, HIPCC, ROOT, short_mfma_reads, unwaited_lds_results
 
-SOURCES = {"pd_prefill": 500, "pd_delta": 500, "pd_token": 100, "pd_layers": 2}
+SOURCES = {"pd_prefill": 500, "pd_delta": 500, "pd_token": 100, "pd_linear": 100, "pd_layers": 2}
 
 
 @pytest.mark.parametrize("source", sorted(SOURCES))
