@@ -3,8 +3,8 @@
 ``decoder_weights`` reads the model's modules and says whether every one of them is the
 plain form the kernels compute; ``decoder_forward`` is then one forward of the model, with
 the residual stream, the norms, the gated delta rule, rotary embedding, the K/V write and
-the gates in HIP kernels between the matrix products.  One token per sequence of up to
-``TOKEN_ROWS`` sequences runs the products in them too.  A model that was changed (hooks,
+the gates in HIP kernels between the matrix products.  Up to ``TOKEN_ROWS`` rows run the
+products in them too.  A model that was changed (hooks,
 replaced or compiled modules, biases, other dtypes or sizes) keeps transformers' modules:
 the weights are read from the modules on every forward, nothing is kept of them.
 """
@@ -17,7 +17,7 @@ from transformers.activations import SiLUActivation
 from transformers.models.qwen3_5 import modeling_qwen3_5 as qwen
 
 from . import _native
-from .prefill import batched_prefill
+from .prefill import batched_prefill, device_cus
 
 MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
 TOKEN_ROWS = 16         # rows of one MFMA operand
@@ -236,16 +236,15 @@ def _gate_up(h, gate, up):
 
 
 def _one_round(rows, dim, features, per_tile, device):
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
     tiles = sum(-(-f // per_tile) for f in features) * -(-rows // 128)
-    return tiles <= cus and dim % 64 == 0 and all(f % 4 == 0 for f in features)
+    return tiles <= device_cus(device) and dim % 64 == 0 and all(f % 4 == 0 for f in features)
 
 
-def _linear_attention(h, w, weights, states, batch, steps):
+def _delta_attention(h, mixed, gate, w, weights, states, batch, steps):
+    """The layer's output before its projection, of the normed rows and their products."""
     hk, hv, dk, dv = weights.linear
-    qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
+    _, _, b, a, taps, a_log, dt_bias, (norm, eps), _ = w.mixer
     conv, state, held = states
-    mixed, gate = _products(h, qkv, z)
     rows = batch * steps
     act = torch.empty((rows, mixed.shape[1]), device=h.device, dtype=torch.float32)
     gates = torch.empty((rows, hv, 2), device=h.device, dtype=torch.float32)
@@ -260,7 +259,7 @@ def _linear_attention(h, w, weights, states, batch, steps):
         _native.delta_rule(act, gates, state, out, batch, steps, hk, hv, dk, dv, held)
     y = torch.empty((rows, hv * dv), device=h.device, dtype=torch.bfloat16)
     _native.gated_norm(out, gate, norm, y, rows * hv, dv, eps)
-    return F.linear(y, out_proj)
+    return y
 
 
 def _full_attention(h, w, weights, rope, runner, batch, steps, attend):
@@ -285,8 +284,8 @@ def _full_attention(h, w, weights, rope, runner, batch, steps, attend):
 
 
 def _token_form(weights, rows):
-    """One token per sequence of few sequences: products that read each weight once, with
-    everything between them folded in.  The normed rows must fit a workgroup's LDS."""
+    """Few rows: products that read each weight once, with the norms, gates and residuals
+    folded in.  The normed rows must fit a workgroup's LDS."""
     hid = weights.head.shape[1]
     mid = weights.layers[0].down.shape[1] if weights.layers else 64
     hk, hv, dk, dv = weights.linear
@@ -296,6 +295,8 @@ def _token_form(weights, rows):
 
 
 def _token_linear(x, w, weights, states, batch):
+    """One token of each sequence: the convolution in the projection, the delta rule's
+    single step with its gated norm."""
     hk, hv, dk, dv = weights.linear
     qkv, z, b, a, taps, a_log, dt_bias, (norm, eps), out_proj = w.mixer
     conv, state, held = states
@@ -311,34 +312,48 @@ def _token_linear(x, w, weights, states, batch):
     _native.linear_add(out, out_proj, x)
 
 
-def _token_full(x, w, weights, rope, runner, batch, attend):
+def _few_linear(x, w, weights, states, batch, steps):
+    """Several tokens of each sequence, in few rows."""
+    qkv, z, _, _, _, _, _, _, out_proj = w.mixer
+    rows = lambda m: torch.empty((x.shape[0], m.shape[0]), device=x.device, dtype=x.dtype)  # noqa: E731
+    mixed, gate, h = rows(qkv), rows(z), torch.empty_like(x)
+    _native.norm_linears(x, w.in_norm[0], w.in_norm[1], (qkv, z), (mixed, gate))
+    _native.add_rms_norm(x, None, w.in_norm[0], h, w.in_norm[1])
+    _native.linear_add(_delta_attention(h, mixed, gate, w, weights, states, batch, steps), out_proj, x)
+
+
+def _token_full(x, w, weights, rope, runner, batch, steps, attend):
     spec, pool = runner.spec, runner.cache.pool
     hq, hkv, d = spec.num_heads, spec.num_kv_heads, spec.head_dim
     q_proj, k_proj, v_proj, (q_norm, eps), (k_norm, _), o_proj = w.mixer
-    rows = lambda *shape: torch.empty(shape, device=x.device, dtype=torch.bfloat16)  # noqa: E731
-    q, k, v, query = rows(batch, hq, 2 * d), rows(batch, hkv, d), rows(batch, hkv, d), rows(batch, hq, d)
+    rows = lambda *shape: torch.empty((batch, steps, *shape), device=x.device, dtype=x.dtype)  # noqa: E731
+    q, k, v, query = rows(hq, 2 * d), rows(hkv, d), rows(hkv, d), rows(hq, d)
     _native.norm_linears(x, w.in_norm[0], w.in_norm[1], (q_proj, k_proj, v_proj), (q, k, v))
     k_pages, v_pages = pool.pages(w.index)
     fill = runner.cache.phase == "prefill"
     keys = torch.empty_like(k) if fill else None
     _native.qk_rope(q, k, v, q_norm, k_norm, rope, query, keys, k_pages, v_pages, pool.tables,
-                    pool.positions, batch, 1, hq, hkv, d, weights.half, eps)
+                    pool.positions, batch, steps, hq, hkv, d, weights.half, eps)
     if fill:
-        out = batched_prefill(query[:, :, None], keys[:, :, None], v[:, :, None], w.module.scaling)
+        out = batched_prefill(query.transpose(1, 2), keys.transpose(1, 2), v.transpose(1, 2),
+                              w.module.scaling)
     else:
-        out = attend(runner, w.module, query, k_pages, v_pages)
+        out = attend(runner, w.module, query.view(batch, hq, d), k_pages, v_pages)
     _native.linear_add(out, o_proj, x, q[..., d:], d)
 
 
-def _token_layers(x, runner, weights, states, rope, attend):
-    batch = x.shape[0]
+def _token_layers(x, runner, weights, states, rope, batch, steps, attend):
+    """Up to TOKEN_ROWS rows, added to the residual stream x."""
     for w in weights.layers:
-        if w.module is None:
-            _token_linear(x, w, weights, states[w.index], batch)
-            runner.cache.linear[w.index].has_previous_state[0] = True
+        if w.module is not None:
+            _token_full(x, w, weights, rope, runner, batch, steps, attend)
         else:
-            _token_full(x, w, weights, rope, runner, batch, attend)
-        h = torch.empty((batch, w.gate.shape[0]), device=x.device, dtype=torch.bfloat16)
+            if steps == 1:
+                _token_linear(x, w, weights, states[w.index], batch)
+            else:
+                _few_linear(x, w, weights, states[w.index], batch, steps)
+            runner.cache.linear[w.index].has_previous_state[0] = True
+        h = torch.empty((x.shape[0], w.gate.shape[0]), device=x.device, dtype=x.dtype)
         _native.norm_gate_up(x, w.post_norm[0], w.post_norm[1], w.gate, w.up, h)
         _native.linear_add(h, w.down, x)
 
@@ -351,7 +366,9 @@ def _row_layers(x, runner, weights, states, rope, batch, steps, attend):
         h = torch.empty_like(x)
         _native.add_rms_norm(x, y, w.in_norm[0], h, w.in_norm[1])
         if w.module is None:
-            y = _linear_attention(h, w, weights, states[w.index], batch, steps)
+            mixed, gate = _products(h, w.mixer[0], w.mixer[1])
+            y = F.linear(_delta_attention(h, mixed, gate, w, weights, states[w.index], batch, steps),
+                         w.mixer[8])
             runner.cache.linear[w.index].has_previous_state[0] = True
         else:
             y = _full_attention(h, w, weights, rope, runner, batch, steps, attend)
@@ -372,13 +389,13 @@ def decoder_forward(runner, weights, states, tokens, positions, attend):
     rope = torch.empty((steps, weights.half, 2), device=x.device, dtype=torch.float32)
     _native.rope_table(positions, weights.inv_freq, rope)
     y = None
-    if steps == 1 and _token_form(weights, batch):
-        _token_layers(x, runner, weights, states, rope, attend)
+    if _token_form(weights, batch * steps):
+        _token_layers(x, runner, weights, states, rope, batch, steps, attend)
     else:
         y = _row_layers(x, runner, weights, states, rope, batch, steps, attend)
-        if steps > 1:
-            x = x.view(batch, steps, hid)[:, -1].contiguous()
-            y = y if y is None else y.view(batch, steps, hid)[:, -1].contiguous()
+    if steps > 1:
+        x = x.view(batch, steps, hid)[:, -1].contiguous()
+        y = y if y is None else y.view(batch, steps, hid)[:, -1].contiguous()
     norm, eps = weights.norm
     if _token_form(weights, batch):
         if y is not None:

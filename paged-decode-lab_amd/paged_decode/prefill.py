@@ -6,6 +6,7 @@ tiles.  Everything else (other types and head dims, CPU tensors, tensors that au
 a functorch transform follows, odd layouts, host metadata) keeps the PyTorch form, which
 materializes the scores of one sequence at a time.
 """
+import functools
 import math
 
 import torch
@@ -50,6 +51,11 @@ def _rows(dim):
     return 64 if dim == 256 else 128
 
 
+@functools.lru_cache(maxsize=None)
+def device_cus(device):
+    return torch.cuda.get_device_properties(device).multi_processor_count
+
+
 def _splits(workgroups, max_keys, dim, device):
     """Key spans per row tile, of 256 keys or more each: as many as fill the device's slots
     (two workgroups a CU), and at head_dim 256, where a workgroup's rows are few and its
@@ -58,7 +64,7 @@ def _splits(workgroups, max_keys, dim, device):
     after 3072, Hq 16 / Hkv 4, D 256, 16 spans), 73 and 24 us (128 after 2048, Hq 8 / Hkv 2,
     D 128, 8 spans); two spans where the workgroups fill the slots alone: 101 instead of 84
     us (2048 rows, Hq 32 / Hkv 8, D 128)."""
-    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    cus = device_cus(device)
     slots = 4 * cus if dim == 256 else 2 * cus
     return max(1, min((slots + workgroups // 2) // workgroups, max_keys // 256, 16))
 

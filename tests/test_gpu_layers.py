@@ -198,7 +198,8 @@ def test_rope_and_page_write(d, half):
     assert torch.equal(pages, want)
 
 
-@pytest.mark.parametrize("hk,hv,dk,dv,length", [(4, 4, 64, 64, 1), (2, 4, 128, 128, 19), (2, 2, 64, 128, 300)])
+@pytest.mark.parametrize("hk,hv,dk,dv,length", [(4, 4, 64, 64, 1), (2, 4, 128, 128, 8), (2, 4, 128, 128, 19),
+                                                (2, 2, 64, 128, 300)])
 def test_layers_agree_with_the_modules(hk, hv, dk, dv, length):
     """One model on the kernels and, with a hook on a layer, on transformers' modules."""
     cfg = H.decoder_config(num_hidden_layers=4, hidden_size=256, intermediate_size=512,
