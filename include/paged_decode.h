@@ -370,9 +370,11 @@ int pd_qk_rope(const void* q, const void* k, const void* v, const void* q_weight
 /* Products of x [rows, dim] with `count` <= 4 weight matrices [features[i],
  * dim], dim a multiple of 64, features of 4; the arrays are host arrays.  form
  * 0: outs[i] = x weights[i]^T; form 1 (two matrices of one size): outs[0] =
- * silu(x weights[0]^T) (x weights[1]^T). */
+ * silu(x weights[0]^T) (x weights[1]^T).  tile: 128 or 256 weight rows a
+ * workgroup. */
 int pd_linears(const void* x, int32_t rows, int32_t dim, int32_t count, const void* const* weights,
-               const int32_t* features, void* const* outs, int32_t form, pd_stream_t stream);
+               const int32_t* features, void* const* outs, int32_t form, int32_t tile,
+               pd_stream_t stream);
 
 /* One token per sequence: products of 1 to 16 rows whose norms, gates,
  * convolution and residual run in the same launch.  dim (the input features)

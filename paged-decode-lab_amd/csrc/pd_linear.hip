@@ -2,26 +2,31 @@
 // operands, float32 sums, with the gate of a gated MLP in the epilogue and
 // several weight matrices of one input in a launch.
 //
-// Bound: the weights' way in.  At 512 rows each weight is used 512 times, so
-// the product is short and a workgroup streams its rows of W from HBM, about 2
-// us away: the next kRing stages (32 KB each, 128 KB of a CU's register file)
-// are always in flight to registers.  From there a stage goes to LDS, one of
-// two buffers, and as 32x32x16 MFMA operands to registers a stage ahead:
-//   write the next stage to LDS and load the stage kRing ahead (the writes
-//   land under) the first half of this stage's products; barrier; read the
-//   next stage's operands under the second half.
-// One workgroup of four wavefronts a CU, each a quarter of the 128 x 128 tile.
-// Tiles that share rows of W are on one XCD and share its L2.  A stage takes
-// 0.85 us however few rows there are, so a product is worth it while its tiles
-// are one round of the CUs.
+// A workgroup of four wavefronts a CU has a tile of BM features by 128 rows;
+// a stage is 64 elements of K.  Copies from memory go straight to LDS (no
+// registers, no LDS write instructions), kRing stages of them: 128 KB in
+// flight for the 2 us to HBM.  Per stage and wavefront, one wait for its own
+// copies of the next stage and one barrier; then it reads the next stage's
+// operands, sends for the stage kRing ahead (its place is free: the operands
+// of this stage are in registers) and multiplies this one.  Tiles that share
+// rows of W are on one XCD and share its L2.
 //
-// Measured on MI355X, inputs of 2048, this form and library products with the
-// gate's launch: 8192 features in two matrices 28 and 38 us of kernels at 512
-// rows; gate and up of 6144 29 and 50 us at 256, 52 and 55 at 512 (two
-// rounds); three matrices of 5120 in all 27 and 40 us at 512 (53 us of host
-// time).  Products of 2048 features, 64 such tiles at 512 rows, were no faster
-// than the library's with 64 x 64 tiles (13.5 and 13.4 us; 31 and 29 us with
-// inputs of 6144) and are left to it.
+// Bound: LDS.  A stage of 128 x 128 is 64 KB of operand reads and 32 KB of
+// copies, 0.37 us at the LDS rate, takes 0.44 us (0.21 of MFMAs) and took 0.85
+// with the ring in registers and stores to LDS.  256 x 128 reads a quarter
+// less for each product: 0.82 us.
+//
+// A product is worth it while its tiles are one round of the CUs: the start
+// and end of a tile, 5 us, meet nobody else's work.  Of two tiles that are, 128
+// is the shorter, and 256 is one round for twice the features.  Measured on
+// MI355X, inputs of 2048, this form, with the ring in registers and library
+// products with the gate's launch (host-bound below 768 rows: 18 us a product):
+// 8192 features in two matrices at 512 rows 24, 28 and 36 us, at 1024 (256)
+// 41, - and 44; gate and up of 6144 at 256 rows 24, 29 and 50, at 512 38 (256;
+// 43 in two rounds of 128), 52 and 54, at 1024, two rounds of either, 66, - and
+// 71, at 2049 145, - and 108; three matrices of 5120 in all at 512 rows 21, 27
+// and 54.  Products of 2048 features, 64 tiles at 512 rows, take 20 us and with
+// inputs of 6144 48; the library's take 13 and 22 to 29, and are used.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -37,9 +42,7 @@ using namespace pdk;
 typedef float floatx16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kMaxSegments = 4;
-constexpr int kRing = 4;
-
-constexpr int BM = 128, BN = 128;
+constexpr int BN = 128;
 
 enum { kStore, kSiluMul };
 
@@ -56,15 +59,24 @@ __device__ __forceinline__ floatx16_t mfma32(u32x4_t a, u32x4_t b, floatx16_t c)
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// Waits until at most `n` of this wavefront's copies are under way.
+template <int n>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");
+}
+
 // BM operand rows of W (kSiluMul: 32 features of the gate and the same 32 of
 // up in turn) by BN rows of X; a stage is 64 elements of K.
-template <int kEpi>
+template <int kEpi, int BM>
 __global__ void __launch_bounds__(256, 1) linear_kernel(const LinearArgs a) {
   constexpr int FM = BM / 64, FN = BN / 64, kSteps = 4;
-  constexpr int kW = BM * 8 / 256, kX = BN * 8 / 256;       // pieces per thread
   constexpr int kPerTile = kEpi == kSiluMul ? BM / 2 : BM;  // features
-  static_assert(kEpi != kSiluMul || FM == 2, "a wavefront's two blocks are gate and up");
-  __shared__ __attribute__((aligned(16))) char lds[2][(BM + BN) * 128];
+  constexpr int kStage = (BM + BN) * 128, kRing = BM == 128 ? 4 : 3;
+  // One array a stage: the compiler then tells a stage's reads from the copies
+  // on their way into the others.
+  __shared__ __attribute__((aligned(16))) char lds0[kStage], lds1[kStage], lds2[kStage],
+      lds3[kRing == 4 ? kStage : 16];
+  char* const ring[4] = {lds0, lds1, lds2, lds3};
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
 
@@ -83,42 +95,31 @@ __global__ void __launch_bounds__(256, 1) linear_kernel(const LinearArgs a) {
   }
   const int m0 = tile * kPerTile, M = a.m[seg];
 
-  // Piece i of this thread: its source row (clamped to the last one, whose
-  // copies are not stored) and its place in a stage.
-  const uint16_t *wp[kW], *xp[kX];
-  int wd[kW], xd[kX];
-  const auto place_of = [&](int i, int& row, int& at, int& k) {
-    const int idx = 256 * i + tid, piece = idx & 7;
-    row = idx / 8;
-    k = 8 * piece;
-    at = row * 128 + 16 * (piece ^ kswz<64>(row));
+  // Copy i of a wavefront fills rows 32 i + 8 wave .. + 7 of the stage, 16
+  // bytes a lane in lane order, so the lanes' sources carry the swizzle.  Rows
+  // past the matrix read as zeros and their products are not stored.
+  const auto rsrc_of = [&](const uint16_t* base, int first, int count, int rows) {
+    const int held = __builtin_amdgcn_readfirstlane(max(min(count, rows - first), 0));
+    return buffer_rsrc(base + int64_t(first) * a.K, held * a.K * 2);
   };
-#pragma unroll
-  for (int i = 0; i < kW; ++i) {
-    int row, k;
-    place_of(i, row, wd[i], k);
-    if constexpr (kEpi == kSiluMul) {
-      const int f = min(m0 + 32 * (row >> 6) + (row & 31), M - 1);
-      wp[i] = ((row >> 5) & 1 ? a.w[1] : a.w[0]) + int64_t(f) * a.K + k;
-    } else {
-      wp[i] = a.w[seg] + int64_t(min(m0 + row, M - 1)) * a.K + k;
-    }
+  __amdgpu_buffer_rsrc_t wr[kEpi == kSiluMul ? 2 : 1];
+  if constexpr (kEpi == kSiluMul) {
+    wr[0] = rsrc_of(a.w[0], m0, kPerTile, M);
+    wr[1] = rsrc_of(a.w[1], m0, kPerTile, M);
+  } else {
+    wr[0] = rsrc_of(a.w[seg], m0, BM, M);
   }
+  const __amdgpu_buffer_rsrc_t xr = rsrc_of(a.x, n0, BN, a.rows);
+  int at[BM / 32];
 #pragma unroll
-  for (int i = 0; i < kX; ++i) {
-    int row, k;
-    place_of(i, row, xd[i], k);
-    xp[i] = a.x + int64_t(min(n0 + row, a.rows - 1)) * a.K + k;
-    xd[i] += BM * 128;
+  for (int i = 0; i < BM / 32; ++i) {
+    const int row = 32 * i + 8 * wave + lane / 8;
+    at[i] = row * a.K * 2 + 16 * ((lane & 7) ^ kswz<64>(row));
   }
 
-  struct Stage {
-    u32x4_t w[kW], x[kX];
-  };
   struct Operands {
     u32x4_t w[kSteps][FM], x[kSteps][FN];
   };
-  Stage ring[kRing];
   Operands ops[2];
   floatx16_t acc[FM][FN];
 #pragma unroll
@@ -127,77 +128,73 @@ __global__ void __launch_bounds__(256, 1) linear_kernel(const LinearArgs a) {
     for (int n = 0; n < FN; ++n) acc[m][n] = floatx16_t{};
 
   const int stages = a.K / 64;
-  const auto fetch = [&](int stage, Stage& s) {
-    // Past the last stage it is loaded again, so that the loads in flight are
+  const auto fetch = [&](int stage, char* to) {
+    // Past the last stage it is copied again, so that the copies in flight are
     // the same number everywhere.
-    const int64_t k = int64_t(min(stage, stages - 1)) * 64;
+    const int k = min(stage, stages - 1) * 128;
+    char* mine = to + wave * 1024;
 #pragma unroll
-    for (int i = 0; i < kW; ++i) s.w[i] = load16(wp[i] + k);
+    for (int i = 0; i < BM / 32; ++i) {
+      if constexpr (kEpi == kSiluMul)
+        lds_copy16(wr[i & 1], mine + 4096 * i, at[i] - (i + 1) / 2 * 64 * a.K + k);
+      else
+        lds_copy16(wr[0], mine + 4096 * i, at[i] + k);
+    }
 #pragma unroll
-    for (int i = 0; i < kX; ++i) s.x[i] = load16(xp[i] + k);
+    for (int i = 0; i < BN / 32; ++i) lds_copy16(xr, mine + BM * 128 + 4096 * i, at[i] + k);
   };
-  const auto put = [&](int buf, const Stage& s) {
-#pragma unroll
-    for (int i = 0; i < kW; ++i) *reinterpret_cast<u32x4_t*>(lds[buf] + wd[i]) = s.w[i];
-#pragma unroll
-    for (int i = 0; i < kX; ++i) *reinterpret_cast<u32x4_t*>(lds[buf] + xd[i]) = s.x[i];
-  };
-  const auto read = [&](int buf, Operands& o) {
+  const auto read = [&](const char* lds, Operands& o) {
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       const int at = col * 128 + 16 * ((2 * s + half) ^ kswz<64>(col));
 #pragma unroll
       for (int m = 0; m < FM; ++m)
         o.w[s][m] = *reinterpret_cast<const u32x4_t*>(
-            lds[buf] + (wm * (BM / 2) + 32 * m) * 128 + at);
+            lds + (wm * (BM / 2) + 32 * m) * 128 + at);
 #pragma unroll
       for (int n = 0; n < FN; ++n)
         o.x[s][n] = *reinterpret_cast<const u32x4_t*>(
-            lds[buf] + (BM + wn * (BN / 2) + 32 * n) * 128 + at);
+            lds + (BM + wn * (BN / 2) + 32 * n) * 128 + at);
     }
   };
-  const auto multiply = [&](const Operands& o, int from, int to) {
+  const auto multiply = [&](const Operands& o) {
 #pragma unroll
-    for (int s = from; s < to; ++s)
+    for (int s = 0; s < kSteps; ++s)
 #pragma unroll
       for (int m = 0; m < FM; ++m)
 #pragma unroll
         for (int n = 0; n < FN; ++n) acc[m][n] = mfma32(o.w[s][m], o.x[s][n], acc[m][n]);
   };
 
-  // Scheduling barriers keep the loads in this order, which the waits count on.
+  constexpr int kCopies = (BM + BN) / 32, kUnroll = kRing == 4 ? 4 : 6;
 #pragma unroll
-  for (int i = 0; i < kRing; ++i) {
-    fetch(i, ring[i]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  put(0, ring[0]);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch(kRing, ring[0]);
-  __builtin_amdgcn_sched_barrier(0);
+  for (int i = 0; i < kRing; ++i) fetch(i, ring[i]);
+  wait_copies<kCopies * (kRing - 1)>();
   lds_barrier();
-  read(0, ops[0]);
-  // Every exit leaves the loop for good: a way back to its head would put the
-  // shortest path's waits there.
-  for (int k = 0;;) {
+  read(ring[0], ops[0]);
+  // Stage k: its operands are in registers, so its place in LDS is free, and
+  // stage k + 1 is there once every wavefront's copies of it are.
+  const auto step = [&](int k, int u) {
+    wait_copies<kCopies * (kRing - 2)>();
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read(ring[(u + 1) % kRing], ops[(u + 1) & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(k + kRing, ring[u % kRing]);
+    multiply(ops[u & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int k = 0;
+  for (; k + kUnroll <= stages; k += kUnroll) {
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) {
-      const int next = (u + 1) % kRing;
-      put((u + 1) & 1, ring[next]);
-      __builtin_amdgcn_sched_barrier(0);
-      fetch(k + 1 + kRing, ring[next]);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(ops[u & 1], 0, kSteps / 2);
-      __builtin_amdgcn_sched_barrier(0);
-      lds_barrier();
-      read((u + 1) & 1, ops[(u + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(ops[u & 1], kSteps / 2, kSteps);
-      __builtin_amdgcn_sched_barrier(0);
-      if (++k == stages) goto done;
-    }
+    for (int u = 0; u < kUnroll; ++u) step(k + u, u);
   }
-done:
+#pragma unroll
+  for (int u = 0; u < kUnroll - 1; ++u) {
+    if (k + u >= stages) break;
+    step(k + u, u);
+  }
+  wait_copies<0>();  // none may land in LDS that has a new owner
   // The last MFMAs and the reads below are in different blocks.
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #pragma unroll
@@ -211,10 +208,11 @@ done:
     const int row = n0 + wn * (BN / 2) + 32 * n + col;
     if (row >= a.rows) continue;
 #pragma unroll
-    for (int m = 0; m < (kEpi == kSiluMul ? 1 : FM); ++m)
+    for (int m = 0; m < FM; m += kEpi == kSiluMul ? 2 : 1)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int f = m0 + wm * (kPerTile / 2) + 32 * m + 8 * g + 4 * half;
+        const int f = m0 + wm * (kPerTile / 2) + 32 * (kEpi == kSiluMul ? m / 2 : m) + 8 * g +
+                      4 * half;
         if (f >= M) continue;
         u32x2_t* out = reinterpret_cast<u32x2_t*>(a.out[seg] + int64_t(row) * M + f);
         float y[4];
@@ -222,7 +220,7 @@ done:
         for (int e = 0; e < 4; ++e) {
           y[e] = acc[m][n][4 * g + e];
           if constexpr (kEpi == kSiluMul)
-            y[e] = y[e] / (1.f + exp_fast(-y[e])) * acc[1][n][4 * g + e];
+            y[e] = y[e] / (1.f + exp_fast(-y[e])) * acc[m + 1][n][4 * g + e];
         }
         *out = u32x2_t{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
       }
@@ -231,7 +229,7 @@ done:
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <int kEpi>
+template <int kEpi, int BM>
 int launch(LinearArgs& a, pd_stream_t stream) {
   constexpr int per = kEpi == kSiluMul ? BM / 2 : BM;
   int64_t tiles = 0;
@@ -240,7 +238,7 @@ int launch(LinearArgs& a, pd_stream_t stream) {
   const int64_t grid = (tiles + 7) / 8 * 8 * a.row_tiles;
   if (grid > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
   a.feature_tiles = int(tiles);
-  hipLaunchKernelGGL(linear_kernel<kEpi>, dim3(unsigned(grid)), dim3(256), 0,
+  hipLaunchKernelGGL((linear_kernel<kEpi, BM>), dim3(unsigned(grid)), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), a);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
@@ -252,14 +250,16 @@ int launch(LinearArgs& a, pd_stream_t stream) {
 
 extern "C" int pd_linears(const void* x, int32_t rows, int32_t dim, int32_t count,
                           const void* const* weights, const int32_t* features, void* const* outs,
-                          int32_t form, pd_stream_t stream) {
+                          int32_t form, int32_t tile, pd_stream_t stream) {
   pd::clear_error();
   if (rows < 0) return pd::fail(PD_EINVAL, "rows must be non-negative");
   if (rows == 0) return PD_OK;
-  if (dim < 64 || dim % 64) return pd::fail(PD_EINVAL, "input features must be a multiple of 64");
+  if (dim < 64 || dim % 64 || dim > 1 << 22)  // a tile's rows are one buffer under 2 GiB
+    return pd::fail(PD_EINVAL, "input features must be a multiple of 64, at most 2^22");
   if (count < 1 || count > kMaxSegments || form < kStore || form > kSiluMul ||
       (form == kSiluMul && count != 2))
     return pd::fail(PD_EINVAL, "1 to %d matrices, 2 for gate and up", kMaxSegments);
+  if (tile != 128 && tile != 256) return pd::fail(PD_EINVAL, "tiles of 128 or 256 features");
   if (!x || !weights || !features || !outs || !aligned16(x))
     return pd::fail(PD_EINVAL, "tensors must be present and 16-byte aligned");
   LinearArgs a{};
@@ -274,5 +274,7 @@ extern "C" int pd_linears(const void* x, int32_t rows, int32_t dim, int32_t coun
   }
   a.x = static_cast<const uint16_t*>(x);
   a.segments = form == kSiluMul ? 1 : count, a.rows = rows, a.K = dim;
-  return form == kSiluMul ? launch<kSiluMul>(a, stream) : launch<kStore>(a, stream);
+  if (tile == 128)
+    return form == kSiluMul ? launch<kSiluMul, 128>(a, stream) : launch<kStore, 128>(a, stream);
+  return form == kSiluMul ? launch<kSiluMul, 256>(a, stream) : launch<kStore, 256>(a, stream);
 }

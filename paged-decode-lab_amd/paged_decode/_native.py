@@ -64,7 +64,7 @@ SIGNATURES = {
     "pd_rope_table": [_vp, _vp, _i32, _vp, _i32, _i32, _vp],
     "pd_qk_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _i32, _vp,
                    _i32, _i32, _i32, _i32, _i32, _i32, _dbl, _vp],
-    "pd_linears": [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
+    "pd_linears": [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _i32, _vp],
     "pd_norm_linears": [_vp, _vp, _dbl, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp],
     "pd_norm_gate_up": [_vp, _vp, _dbl, _i32, _i32, _vp, _vp, _vp, _i32, _vp],
     "pd_linear_add": [_vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _vp],
@@ -353,13 +353,14 @@ def qk_rope(q, k, v, q_weight, k_weight, rope, q_out, k_out, k_pages, v_pages, t
 LINEAR_STORE, LINEAR_SILU_MUL = 0, 1
 
 
-def linears(x, weights, outs, form=LINEAR_STORE):
-    """outs[i] = x weights[i]^T, or outs[0] = silu(x gate^T) (x up^T)."""
+def linears(x, weights, outs, form=LINEAR_STORE, tile=128):
+    """outs[i] = x weights[i]^T, or outs[0] = silu(x gate^T) (x up^T); ``tile`` weight rows a
+    workgroup."""
     n = len(weights)
     check(lib().pd_linears(x.data_ptr(), x.shape[0], x.shape[1], n,
                            (_vp * n)(*[w.data_ptr() for w in weights]),
                            (_i32 * n)(*[w.shape[0] for w in weights]),
-                           (_vp * n)(*[outs[i % len(outs)].data_ptr() for i in range(n)]), form,
+                           (_vp * n)(*[outs[i % len(outs)].data_ptr() for i in range(n)]), form, tile,
                            stream_handle(x.device)))
 
 

@@ -212,32 +212,41 @@ def decoder_states(runner, weights, tokens):
 
 
 def _products(h, *matrices):
-    """h times each matrix: one launch while its 128 x 128 tiles are one round of the CUs
+    """h times each matrix: one launch while its tiles are one round of the CUs
     (pd_linears), else the library's products."""
     rows, dim = h.shape
     features = [m.shape[0] for m in matrices]
-    if not _one_round(rows, dim, features, 128, h.device):
+    tile = _one_round_tile(rows, dim, features, h.device)
+    if not tile:
         return [F.linear(h, m) for m in matrices]
     outs = [torch.empty((rows, f), device=h.device, dtype=h.dtype) for f in features]
-    _native.linears(h, matrices, outs)
+    _native.linears(h, matrices, outs, tile=tile)
     return outs
 
 
 def _gate_up(h, gate, up):
-    """silu(h gate^T) (h up^T), on the same rule; 64 features of either are a tile."""
+    """silu(h gate^T) (h up^T), on the same rule; half a tile's features are the gate's."""
     rows, dim = h.shape
-    if not _one_round(rows, dim, [gate.shape[0]], 64, h.device):
+    tile = gate.shape[0] % 4 == 0 and _one_round_tile(rows, dim, [2 * gate.shape[0]], h.device)
+    if not tile:
         a, b = F.linear(h, gate), F.linear(h, up)
         _native.silu_mul(a, b, a)
         return a
     out = torch.empty((rows, gate.shape[0]), device=h.device, dtype=h.dtype)
-    _native.linears(h, (gate, up), (out,), _native.LINEAR_SILU_MUL)
+    _native.linears(h, (gate, up), (out,), _native.LINEAR_SILU_MUL, tile)
     return out
 
 
-def _one_round(rows, dim, features, per_tile, device):
-    tiles = sum(-(-f // per_tile) for f in features) * -(-rows // 128)
-    return tiles <= device_cus(device) and dim % 64 == 0 and all(f % 4 == 0 for f in features)
+def _one_round_tile(rows, dim, features, device):
+    """The features of a tile whose 128-row tiles are one round of the CUs, 0 if none's are.
+    The smaller tile is the faster one where both would do (24 and 36 us, 8192 features of
+    2048 at 512 rows)."""
+    if dim % 64 or any(f % 4 for f in features):
+        return 0
+    for tile in (128, 256):
+        if sum(-(-f // tile) for f in features) * -(-rows // 128) <= device_cus(device):
+            return tile
+    return 0
 
 
 def _delta_attention(h, mixed, gate, w, weights, states, batch, steps):

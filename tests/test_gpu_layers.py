@@ -228,25 +228,28 @@ def test_layers_agree_with_the_modules(hk, hv, dk, dv, length):
 
 @pytest.mark.parametrize("rows", [1, 127, 128, 129, 300])
 @pytest.mark.parametrize("dim,features", [(64, (4, 100)), (128, (128,)), (192, (260, 4, 128)),
-                                          (256, (384,)), (320, (36, 64)), (2048, (132,))])
-def test_linears(rows, dim, features):
+                                          (256, (384,)), (320, (36, 64)), (2048, (132,)),
+                                          (384, (252, 516)), (448, (256,))])
+@pytest.mark.parametrize("tile", [128, 256])
+def test_linears(rows, dim, features, tile):
     gen = torch.Generator(device="cuda").manual_seed(rows + dim)
     x = bf16(gen, rows, dim)
     weights = [bf16(gen, f, dim, scale=dim ** -0.5) for f in features]
     outs = [torch.empty(rows, f, device="cuda", dtype=torch.bfloat16) for f in features]
-    _native.linears(x, weights, outs)
+    _native.linears(x, weights, outs, tile=tile)
     for w, out in zip(weights, outs):
         # float32 sums of dim products of order dim^-1/2
         close(out, x.double() @ w.double().T, 1e-5, bf16_out=True)
 
 
-@pytest.mark.parametrize("rows,dim,features", [(1, 64, 4), (130, 192, 68), (257, 2048, 200)])
-def test_linears_of_gate_and_up(rows, dim, features):
+@pytest.mark.parametrize("rows,dim,features", [(1, 64, 4), (130, 192, 68), (257, 2048, 200), (129, 448, 132)])
+@pytest.mark.parametrize("tile", [128, 256])
+def test_linears_of_gate_and_up(rows, dim, features, tile):
     gen = torch.Generator(device="cuda").manual_seed(rows + dim)
     x = bf16(gen, rows, dim)
     gate, up = (bf16(gen, features, dim, scale=2 * dim ** -0.5) for _ in range(2))
     out = torch.empty(rows, features, device="cuda", dtype=torch.bfloat16)
-    _native.linears(x, (gate, up), (out,), _native.LINEAR_SILU_MUL)
+    _native.linears(x, (gate, up), (out,), _native.LINEAR_SILU_MUL, tile)
     a, b = x.double() @ gate.double().T, x.double() @ up.double().T
     close(out, F.silu(a) * b, 1e-4, bf16_out=True)
 
