@@ -4,8 +4,8 @@
 //
 // A workgroup of four wavefronts a CU has a tile of BM features by 128 rows;
 // a stage is 64 elements of K.  Copies from memory go straight to LDS (no
-// registers, no LDS write instructions), kRing stages of them: 128 KB in
-// flight for the 2 us to HBM.  Per stage and wavefront, one wait for its own
+// registers, no LDS write instructions), kRing stages of them: 128 or
+// 144 KB a CU for the 2 us to HBM.  Per stage and wavefront, one wait for its own
 // copies of the next stage and one barrier; then it reads the next stage's
 // operands, sends for the stage kRing ahead (its place is free: the operands
 // of this stage are in registers) and multiplies this one.  Tiles that share

@@ -368,7 +368,7 @@ def _token_layers(x, runner, weights, states, rope, batch, steps, attend):
 
 
 def _row_layers(x, runner, weights, states, rope, batch, steps, attend):
-    """Any number of rows: library products with the kernels between them; returns the
+    """Any number of rows: products with the kernels between them; returns the
     last layer's output, not yet added to the residual stream x."""
     y = None
     for w in weights.layers:
