@@ -154,7 +154,8 @@ def _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out):
 
 def batched_prefill(query, key, value, scale):
     """Attention of equally long sequences without a prefix; query [B, Hq, S, D], key and
-    value [B, Hkv, S, D], returns [B, S, Hq, D]."""
+    value [B, Hkv, S, D], returns [B, S, Hq, D], contiguous in either form: the decoder's
+    kernels read it by its address."""
     if not _batched_ok(query, key, value, scale):
         return _batched_torch(query, key, value, scale)
     b, hq, s, d = query.shape
@@ -192,4 +193,4 @@ def _batched_torch(query, key, value, scale):
     scores = torch.matmul(q, k) * scale
     future = torch.ones(s, s, dtype=torch.bool, device=query.device).triu(1)
     probs = scores.masked_fill(future, float("-inf")).softmax(-1)
-    return torch.matmul(probs, v).transpose(1, 2).to(query.dtype)
+    return torch.matmul(probs, v).transpose(1, 2).to(query.dtype).contiguous()

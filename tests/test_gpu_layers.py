@@ -3,6 +3,7 @@
 float32 results are held to a few float32 ulps of the largest terms of their sums, bf16
 results to half a bf16 ulp (2^-8 of the value) more.
 """
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
@@ -13,6 +14,7 @@ if not torch.cuda.is_available():
 from paged_decode import _native
 from paged_decode import decoder_layers as DL
 from paged_decode import hybrid as H
+from paged_decode import prefill as PF
 
 pytestmark = pytest.mark.gpu
 
@@ -263,3 +265,27 @@ def test_other_batches_are_refused_as_before():
         runner = H.HybridRunner(model=model, backend="hip_matched", batch=2, max_context=300)
         with pytest.raises((RuntimeError, ValueError)):
             runner.prefill([[1, 2, 3]] * rows)
+
+
+def small_model(layers=4, **overrides):
+    sizes = dict(hidden_size=256, intermediate_size=512, vocab_size=512, linear_num_key_heads=4,
+                 linear_key_head_dim=64, linear_num_value_heads=4, linear_value_head_dim=64)
+    return H.random_init_model(H.decoder_config(num_hidden_layers=layers, **{**sizes, **overrides}),
+                               "cuda", seed=1)
+
+
+@pytest.mark.parametrize("length", [5, 40])
+def test_layers_read_the_general_prefill_form(length):
+    """A scale that the prefill kernel does not take sends the attention to its PyTorch form,
+    in the few-row and in the row layers; outputs differ by the attention's roundings."""
+    model = small_model()
+    prompt = [[(7 * i + 3 * j) % 512 for i in range(length)] for j in range(2)]
+    runner = H.HybridRunner(model=model, backend="hip_matched", batch=2, max_context=300)
+    want = runner.prefill(prompt).float()
+    module = runner.attention_modules[0]
+    q = torch.zeros(1, 8, 4, 256, device="cuda", dtype=torch.bfloat16)
+    assert not PF._batched_ok(q, q[:, :2], q[:, :2], np.float32(module.scaling))
+    module.scaling = np.float32(module.scaling)
+    assert DL.decoder_weights(model, runner.cache.pool.block.device) is not None
+    got = runner.prefill(prompt).float()
+    assert (got - want).norm() <= 0.01 * want.norm()
