@@ -4,17 +4,24 @@
 plain form the kernels compute; ``decoder_forward`` is then one forward of the model, with
 the residual stream, the norms, the gated delta rule, rotary embedding, the K/V write and
 the gates in HIP kernels between the matrix products.  Up to ``TOKEN_ROWS`` rows run the
-products in them too.  A model that was changed (hooks,
-replaced or compiled modules, biases, other dtypes or sizes) keeps transformers' modules:
-the weights are read from the modules on every forward, nothing is kept of them.
+products in them too.  A model that was changed (hooks, replaced or compiled modules,
+biases, other dtypes or sizes, patched classes or functions of its file) keeps transformers'
+modules: the weights are read from the modules on every forward, nothing is kept of them.
 """
+import operator
+import os
+import types
 from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
+import transformers
 from torch import nn
 from transformers.activations import SiLUActivation
 from transformers.models.qwen3_5 import modeling_qwen3_5 as qwen
+from transformers.models.qwen3_5.modeling_qwen3_5 import (
+    Qwen3_5Attention, Qwen3_5DecoderLayer, Qwen3_5GatedDeltaNet, Qwen3_5MLP, Qwen3_5RMSNorm,
+    Qwen3_5RMSNormGated, Qwen3_5TextRotaryEmbedding)
 
 from . import _native
 from .prefill import batched_prefill, device_cus
@@ -23,11 +30,55 @@ MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workg
 TOKEN_ROWS = 16         # rows of one MFMA operand
 CHUNK_STEPS = 96        # tokens from which the delta rule is faster in chunks (one sequence)
 
+KINDS = (nn.Embedding, nn.Linear, nn.Conv1d, SiLUActivation, Qwen3_5Attention, Qwen3_5DecoderLayer,
+         Qwen3_5GatedDeltaNet, Qwen3_5MLP, Qwen3_5RMSNorm, Qwen3_5RMSNormGated,
+         Qwen3_5TextRotaryEmbedding)
+
+
+def _definitions():
+    """(getter, owner, names, values) of what runs in a plain layer: the functions and classes
+    of the model's file, and the methods that a call of each kind goes through, found on the
+    class as a call finds them."""
+    space = vars(qwen)
+    names = [n for n, f in space.items()
+             if isinstance(f, types.FunctionType) and f.__module__ == qwen.__name__]
+    names += [k.__name__ for k in KINDS if k.__module__ == qwen.__name__]
+    found = [(operator.itemgetter(*names), space, names)]
+    for kind in KINDS:
+        own = {n for c in kind.__mro__ if c not in (nn.Module, object) for n, f in vars(c).items()
+               if isinstance(f, types.FunctionType)}
+        names = sorted(own - {"__init__", "__setstate__", "extra_repr", "reset_parameters"}
+                       | {"forward", "__call__", "_call_impl", "_wrapped_call_impl", "__getattr__"})
+        found.append((operator.attrgetter(*names), kind, names))
+    return [(get, owner, names, get(owner)) for get, owner, names in found]
+
+
+def _installed(value):
+    """A function of the installed packages, or no function."""
+    code = getattr(value, "__code__", None)
+    return code is None or code.co_filename.startswith(
+        tuple(os.path.dirname(p.__file__) + os.sep for p in (torch, transformers)))
+
+
+# Compared on every forward: a patch made after this import shows as another value, one made
+# before it as a function or class of another file.
+_DEFINITIONS = _definitions()
+_INSTALLED = (all(_installed(value) for *_, values in _DEFINITIONS for value in values)
+              and all(k.__module__.split(".")[0] in ("torch", "transformers") for k in KINDS))
+
+
+def _as_installed():
+    for get, owner, _, values in _DEFINITIONS:
+        if get(owner) != values:
+            return False
+    return _INSTALLED
+
 
 def _plain_module(module, kind):
     """`module` runs the forward its class defines and nothing else."""
+    own = module.__dict__
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
-            and "forward" not in module.__dict__ and module._compiled_call_impl is None
+            and "forward" not in own and "_norm" not in own and module._compiled_call_impl is None
             and not module.training)
 
 
@@ -62,12 +113,14 @@ class _Reader:
             self.ok = False
         return self.weight(module, (rows, cols))
 
-    def norm(self, parent, name, dim, kind=qwen.Qwen3_5RMSNorm):
+    def norm(self, parent, name, dim, kind=Qwen3_5RMSNorm):
         module = self.module(parent, name, kind)
         if not self.ok:
             return None, 0.0
-        return self.weight(module, (dim,)), float(
-            module.variance_epsilon if kind is qwen.Qwen3_5RMSNormGated else module.eps)
+        if kind is Qwen3_5RMSNorm:
+            return self.weight(module, (dim,)), float(module.eps)
+        self.ok = module.__dict__.get("activation", "silu") == "silu"
+        return self.weight(module, (dim,)), float(module.variance_epsilon)
 
 
 @dataclass
@@ -95,7 +148,7 @@ class DecoderWeights:
 def _linear_mixer(read, layer, cfg):
     hk, hv = cfg.linear_num_key_heads, cfg.linear_num_value_heads
     dk, dv, hid = cfg.linear_key_head_dim, cfg.linear_value_head_dim, cfg.hidden_size
-    m = read.module(layer, "linear_attn", qwen.Qwen3_5GatedDeltaNet)
+    m = read.module(layer, "linear_attn", Qwen3_5GatedDeltaNet)
     if (not read.ok or (m.num_k_heads, m.num_v_heads, m.head_k_dim, m.head_v_dim) != (hk, hv, dk, dv)
             or m.conv_kernel_size != 4 or m.activation != "silu"):
         read.ok = False
@@ -109,14 +162,14 @@ def _linear_mixer(read, layer, cfg):
     return (read.linear(m, "in_proj_qkv", channels, hid), read.linear(m, "in_proj_z", hv * dv, hid),
             read.linear(m, "in_proj_b", hv, hid), read.linear(m, "in_proj_a", hv, hid),
             read.weight(conv, (channels, 1, 4)), read.weight(m, (hv,), "A_log"),
-            read.weight(m, (hv,), "dt_bias"), read.norm(m, "norm", dv, qwen.Qwen3_5RMSNormGated),
+            read.weight(m, (hv,), "dt_bias"), read.norm(m, "norm", dv, Qwen3_5RMSNormGated),
             read.linear(m, "out_proj", hid, hv * dv))
 
 
 def _full_mixer(read, layer, cfg):
     hq, hkv, d, hid = (cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim,
                        cfg.hidden_size)
-    m = read.module(layer, "self_attn", qwen.Qwen3_5Attention)
+    m = read.module(layer, "self_attn", Qwen3_5Attention)
     if not read.ok or m.head_dim != d:
         read.ok = False
         return None
@@ -133,7 +186,7 @@ def decoder_weights(model, device):
     text, cfg = model.model, model.model.config
     hooks = nn.modules.module
     read = _Reader(device)
-    if hooks._global_forward_hooks or hooks._global_forward_pre_hooks:
+    if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or not _as_installed():
         return None
     hk, hv = cfg.linear_num_key_heads, cfg.linear_num_value_heads
     dk, dv, hid, mid = (cfg.linear_key_head_dim, cfg.linear_value_head_dim, cfg.hidden_size,
@@ -143,7 +196,7 @@ def decoder_weights(model, device):
             or cfg.head_dim not in (64, 128, 256)):
         return None
     embed = read.module(text, "embed_tokens", nn.Embedding)
-    rope = read.module(text, "rotary_emb", qwen.Qwen3_5TextRotaryEmbedding)
+    rope = read.module(text, "rotary_emb", Qwen3_5TextRotaryEmbedding)
     if not read.ok or read.weight(embed, (cfg.vocab_size, hid)) is None:
         return None
     inv = rope._buffers.get("inv_freq")
@@ -154,10 +207,10 @@ def decoder_weights(model, device):
     layers = []
     for i, layer in enumerate(text.layers):
         full = cfg.layer_types[i] == "full_attention"
-        if not _plain_module(layer, qwen.Qwen3_5DecoderLayer):
+        if not _plain_module(layer, Qwen3_5DecoderLayer):
             return None
         mixer = _full_mixer(read, layer, cfg) if full else _linear_mixer(read, layer, cfg)
-        mlp = read.module(layer, "mlp", qwen.Qwen3_5MLP)
+        mlp = read.module(layer, "mlp", Qwen3_5MLP)
         if not read.ok:
             return None
         read.module(mlp, "act_fn", SiLUActivation)
