@@ -8,6 +8,7 @@ materializes the scores of one sequence at a time.
 """
 import functools
 import math
+import numbers
 
 import torch
 
@@ -64,6 +65,8 @@ def _splits(workgroups, max_keys, dim, device):
     after 3072, Hq 16 / Hkv 4, D 256, 16 spans), 73 and 24 us (128 after 2048, Hq 8 / Hkv 2,
     D 128, 8 spans); two spans where the workgroups fill the slots alone: 101 instead of 84
     us (2048 rows, Hq 32 / Hkv 8, D 128)."""
+    if not isinstance(max_keys, numbers.Integral):
+        return 1
     cus = device_cus(device)
     slots = 4 * cus if dim == 256 else 2 * cus
     return max(1, min((slots + workgroups // 2) // workgroups, max_keys // 256, 16))
@@ -82,7 +85,7 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0):
     ``cu_q``/``cu_k``: cumulative new and visible tokens per sequence.  Without ``tables``
     k and v are the packed rows [M, Hkv, D]; with them the paged caches
     [blocks, block_size, Hkv, D], which hold every visible token already.  ``max_keys`` is
-    a hint of the longest sequence's visible tokens (0: unknown).
+    a hint of the longest sequence's visible tokens (0 or no whole number: unknown).
     """
     out = torch.empty_like(q)
     if not _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables):
