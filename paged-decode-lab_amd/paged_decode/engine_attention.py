@@ -151,4 +151,5 @@ class Attention(nn.Module):
         if context.block_tables is not None:  # prefix cache: the whole context is paged
             k, v = self.k_cache, self.v_cache
         return packed_prefill(q, k, v, context.cu_seqlens_q, context.cu_seqlens_k, self.scale,
-                              tables=context.block_tables, max_keys=context.max_seqlen_k)
+                              tables=context.block_tables, max_keys=context.max_seqlen_k,
+                              group=self.num_heads // self.num_kv_heads)

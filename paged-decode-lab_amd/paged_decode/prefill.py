@@ -79,17 +79,21 @@ def _workspace(splits, total_q, heads, dim, device):
             torch.empty((splits, total_q, heads, 2), device=device, dtype=torch.float32))
 
 
-def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0):
+def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group=None):
     """Attention of packed sequences; q [N, Hq, D], returns a tensor like it.
 
     ``cu_q``/``cu_k``: cumulative new and visible tokens per sequence.  Without ``tables``
     k and v are the packed rows [M, Hkv, D]; with them the paged caches
     [blocks, block_size, Hkv, D], which hold every visible token already.  ``max_keys`` is
     a hint of the longest sequence's visible tokens (0 or no whole number: unknown).
+    ``group``: query heads per kv head of the layer (None: what the tensors have); tensors
+    with other head counts fail in the PyTorch form.
     """
     out = torch.empty_like(q)
-    if not _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables):
-        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out)
+    if group is None:
+        group = q.shape[1] // k.shape[-2]
+    if not _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables) or q.shape[1] != group * k.shape[-2]:
+        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     n, hq, d = q.shape
     hkv, seqs = k.shape[-2], cu_q.shape[0] - 1
     if n == 0 or seqs < 1:
@@ -134,9 +138,8 @@ def _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables):
     return True
 
 
-def _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out):
+def _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group):
     cu_q, cu_k = cu_q.tolist(), cu_k.tolist()
-    group = q.shape[1] // k.shape[-2]
     for i in range(len(cu_q) - 1):
         nq, nk = cu_q[i + 1] - cu_q[i], cu_k[i + 1] - cu_k[i]
         if tables is None:
