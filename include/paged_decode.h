@@ -306,6 +306,16 @@ int pd_prefill(const void* q, const int64_t* q_strides, const void* k, const int
                int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
                float* part_o, float* part_ml, pd_stream_t stream);
 
+/* Checks the metadata of a packed or paged pd_prefill on the device.  Sets
+ * flags[0] (int32 [2], zeroed by the caller, device or pinned host memory)
+ * where sequences are not rows of the tensors in order, or a sequence of new
+ * tokens has no keys or a page in [-num_pages, -1]; flags[1] where one has
+ * more keys than its table's entries hold or any other page outside the pool. */
+int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs, int64_t total_q,
+                    int64_t total_k, const int32_t* table, int64_t table_stride_b,
+                    int32_t table_width, int32_t page_size, int64_t num_pages, int32_t* flags,
+                    pd_stream_t stream);
+
 /* The decoder layer between its matrix products.  bf16 tensors are contiguous
  * and 16-byte aligned unless strides are given; arithmetic is float32. */
 

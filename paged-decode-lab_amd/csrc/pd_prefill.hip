@@ -190,7 +190,8 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
     nq = int(min(int64_t(a.cu_q[seq + 1]), a.total_q) - q0);
     k0 = max(0, a.cu_k[seq]);
     const int64_t klim = kPaged ? int64_t(a.table_width) * a.page_size : a.total_k - k0;
-    nk = int(max(int64_t(0), min(int64_t(a.cu_k[seq + 1]) - a.cu_k[seq], klim)));
+    nk = int(min(max(int64_t(0), min(int64_t(a.cu_k[seq + 1]) - a.cu_k[seq], klim)),
+                 int64_t(0x7fffffff)));
   } else {
     const int tiles = (int64_t(a.seq_len) * a.G + kRows - 1) / kRows;
     seq = t_rev / tiles;
@@ -512,6 +513,43 @@ prefill_merge_kernel(const PrefillArgs a, int64_t all) {
   for (int e = 0; e < E; ++e) out[e] = uint16_t(bf16_bits(o[e] * inv));
 }
 
+// What the caller must know of packed metadata, which only the device holds:
+// flags[0] where sequences are not rows of the tensors in order, or a sequence
+// of new tokens has no keys or a page counted from the pool's end; flags[1]
+// where a sequence reaches past its table or to a page that does not exist.
+// Other flags are left alone.  One thread a table entry, and a sequence.
+struct PackedCheck {
+  const int32_t *cu_q, *cu_k, *table;
+  int64_t total_q, total_k, num_pages, tsb;
+  int num_seqs, table_width, page_size;
+  int32_t* flags;
+};
+
+__global__ void __launch_bounds__(256) check_packed_kernel(const PackedCheck a) {
+  const int width = a.table ? a.table_width : 1;
+  const int64_t total = int64_t(a.num_seqs) * width, step = int64_t(gridDim.x) * 256;
+  bool odd = false, outside = false;
+  for (int64_t at = int64_t(blockIdx.x) * 256 + threadIdx.x; at < total; at += step) {
+    const int i = int(at / width), entry = int(at % width);
+    const int64_t k0 = a.cu_k[i], k1 = a.cu_k[i + 1], nk = k1 - k0;
+    if (entry == 0) {
+      const int64_t q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
+      odd |= q0 < 0 || q1 < q0 || q1 > a.total_q || nk < 0 || (nk == 0 && q1 > q0);
+      if (a.table)
+        outside |= nk > int64_t(width) * a.page_size;
+      else
+        odd |= k0 < 0 || k1 > a.total_k;
+    }
+    if (a.table && int64_t(entry) * a.page_size < nk) {
+      const int64_t page = a.table[i * a.tsb + entry];
+      odd |= page < 0;
+      outside |= page >= a.num_pages || page < -a.num_pages;
+    }
+  }
+  if (odd) a.flags[0] = 1;
+  if (outside) a.flags[1] = 1;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <int D>
@@ -619,5 +657,25 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return pd::fail(PD_ELAUNCH, "pd_prefill launch failed: %s", hipGetErrorString(err));
+  return PD_OK;
+}
+
+extern "C" int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs,
+                               int64_t total_q, int64_t total_k, const int32_t* table,
+                               int64_t table_stride_b, int32_t table_width, int32_t page_size,
+                               int64_t num_pages, int32_t* flags, pd_stream_t stream) {
+  pd::clear_error();
+  if (num_seqs < 1) return pd::fail(PD_EINVAL, "sequences must be positive");
+  if (!cu_q || !cu_k || !flags) return pd::fail(PD_EINVAL, "null tensor pointer");
+  if (table && (table_width < 1 || page_size < 1))
+    return pd::fail(PD_EINVAL, "empty table or pages");
+  const PackedCheck a{cu_q, cu_k, table, total_q, total_k, num_pages, table_stride_b,
+                      num_seqs, table_width, page_size, flags};
+  const int64_t blocks = (int64_t(num_seqs) * (table ? table_width : 1) + 255) / 256;
+  hipLaunchKernelGGL(check_packed_kernel, dim3(unsigned(blocks < 256 ? blocks : 256)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess)
+    return pd::fail(PD_ELAUNCH, "pd_check_packed launch failed: %s", hipGetErrorString(err));
   return PD_OK;
 }

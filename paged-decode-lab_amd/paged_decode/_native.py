@@ -52,6 +52,7 @@ SIGNATURES = {
                           _i32, _vp, _i32, _i32, _i32, _i32, _vp],
     "pd_prefill": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp,
                    _i64, _i32, _i32, _i64, _i32, _i32, _i32, _dbl, _i32, _vp, _vp, _vp],
+    "pd_check_packed": [_vp, _vp, _i32, _i64, _i64, _vp, _i64, _i32, _i32, _i64, _vp, _vp],
     "pd_add_rms_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
     "pd_gated_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
     "pd_silu_mul": [_vp, _vp, _vp, _i64, _vp],
@@ -277,6 +278,15 @@ def prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu
         page_size, num_pages, heads, kv_heads, head_dim, scale, splits,
         None if part_o is None else part_o.data_ptr(),
         None if part_ml is None else part_ml.data_ptr(), stream_handle(q.device)))
+
+
+def check_packed(cu_q, cu_k, num_seqs, total_q, total_k, tables, page_size, num_pages, flags):
+    """pd_check_packed; flags int32 [2] pinned, zero."""
+    check(lib().pd_check_packed(
+        cu_q.data_ptr(), cu_k.data_ptr(), num_seqs, total_q, total_k,
+        None if tables is None else tables.data_ptr(), 0 if tables is None else tables.stride(0),
+        0 if tables is None else tables.shape[1], page_size, num_pages, flags.data_ptr(),
+        stream_handle(cu_q.device)))
 
 
 def add_rms_norm(x, y, weight, out, eps):

@@ -88,6 +88,11 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group
     a hint of the longest sequence's visible tokens (0 or no whole number: unknown).
     ``group``: query heads per kv head of the layer (None: what the tensors have); tensors
     with other head counts fail in the PyTorch form.
+
+    The metadata are checked on the device ahead of the attention, which reads nothing outside
+    its tensors whatever they hold, and the host waits for that check alone: what does not fit
+    the tensors is left to the PyTorch form, which fails on it, and pages outside the cache
+    raise.  A captured call has no such check: there such rows read as zeros.
     """
     out = torch.empty_like(q)
     if group is None:
@@ -96,15 +101,31 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group
         return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     n, hq, d = q.shape
     hkv, seqs = k.shape[-2], cu_q.shape[0] - 1
-    if n == 0 or seqs < 1:
+    capturing = torch.cuda.is_current_stream_capturing()
+    if seqs < 1 or (n == 0 and capturing):
         return out
+    if n == 0:
+        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     page_size, num_pages = (k.shape[1], k.shape[0]) if tables is not None else (0, 0)
+    total_k = 0 if tables is not None else k.shape[0]
+    if not capturing:
+        flags = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        _native.check_packed(cu_q, cu_k, seqs, n, total_k, tables, page_size, num_pages, flags)
+        checked = torch.cuda.Event()
+        checked.record(torch.cuda.current_stream(q.device))
     splits = _splits((n * (hq // hkv) // _rows(d) + seqs) * hkv, max_keys, d, q.device)
     part_o, part_ml = _workspace(splits, n, hq, d, q.device)
     rows = lambda t: (t.stride(0) if t.dim() == 4 else 0, t.stride(-3), t.stride(-2))  # noqa: E731
     _native.prefill(q, rows(q), k, rows(k), v, rows(v), out, rows(out), cu_q, cu_k, seqs, 0, n,
-                    0 if tables is not None else k.shape[0], tables, page_size, num_pages, hq, hkv,
-                    d, float(scale), splits, part_o, part_ml)
+                    total_k, tables, page_size, num_pages, hq, hkv, d, float(scale), splits, part_o,
+                    part_ml)
+    if not capturing:
+        checked.synchronize()
+        odd, outside = flags.tolist()
+        if outside:
+            raise IndexError("a sequence reaches past its block table or to a page outside the cache")
+        if odd:
+            return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     return out
 
 

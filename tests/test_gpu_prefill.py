@@ -150,3 +150,100 @@ def test_general_form_serves_what_the_kernel_does_not():
     cu = torch.tensor([0, 9], dtype=torch.int32)
     PF.packed_prefill(x, x, x, cu, cu, 0.1).sum().backward()
     assert x.grad.abs().sum() > 0
+
+
+def metadata(d=64, page=None, lens=(20, 1, 37), prefix=64):
+    """A packed call (paged with `page`) as (q, k, v, cu_q, cu_k, scale), keywords, host lists."""
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    total = [n + (prefix if page else 0) for n in lens]
+    q = rows(gen, sum(lens), 4, d)
+    cu = [list(np.cumsum([0, *ns])) for ns in (lens, total)]
+    if page is None:
+        return q, rows(gen, sum(total), 2, d), rows(gen, sum(total), 2, d), *cu, None
+    used = [-(-n // page) for n in total]
+    order = list(np.random.default_rng(d).permutation(sum(used) + 2))
+    table = [[int(order.pop()) for _ in range(n)] + [-1] * (max(used) - n) for n in used]
+    k, v = (rows(gen, sum(used) + 2, page, 2, d) for _ in range(2))
+    return q, k, v, *cu, table
+
+
+def call(q, k, v, cu_q, cu_k, table, form=PF.packed_prefill):
+    device = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    args = (q, k, v, device(cu_q), device(cu_k), 0.1)
+    tables = None if table is None else device(table)
+    if form is PF.packed_prefill:
+        out = torch.empty_like(q)
+        assert q.shape[0] == 0 or PF._packed_ok(*args[:3], out, *args[3:], tables)
+        return form(*args, tables=tables, max_keys=3000)
+    return form(*args, tables, torch.zeros_like(q), 2)
+
+
+@pytest.mark.parametrize("d,page", [(64, None), (256, 32)])
+@pytest.mark.parametrize("fault", ["q_end", "q_order", "q_start", "k_order", "no_rows"])
+def test_sequences_that_are_not_the_tensors_fail(d, page, fault):
+    q, k, v, cu_q, cu_k, table = metadata(d, page)
+    if fault == "q_end":
+        cu_q[-1] += 1
+    elif fault == "q_order":
+        cu_q[1], cu_q[2] = cu_q[2] + 3, cu_q[1]
+    elif fault == "q_start":
+        cu_q[0] = -3
+    elif fault == "k_order":
+        cu_k[2:] = [n - (cu_k[2] - cu_k[1] + 2) for n in cu_k[2:]]
+    else:
+        q = q[:0]
+    for form in (PF.packed_prefill, PF._packed_torch):
+        with pytest.raises(RuntimeError):
+            call(q, k, v, cu_q, cu_k, table, form)
+
+
+@pytest.mark.parametrize("fault", ["k_end", "k_start"])
+def test_keys_that_are_not_the_tensors_fail(fault):
+    q, k, v, cu_q, cu_k, _ = metadata()
+    cu_k[0 if fault == "k_start" else -1] += -2 if fault == "k_start" else 2
+    for form in (PF.packed_prefill, PF._packed_torch):
+        with pytest.raises(RuntimeError):
+            call(q, k, v, cu_q, cu_k, None, form)
+
+
+@pytest.mark.parametrize("fault", ["width", "page", "below"])
+@pytest.mark.parametrize("sequences", [3, 300])
+def test_pages_outside_the_cache_fail(fault, sequences):
+    q, k, v, cu_q, cu_k, table = metadata(256, 32, lens=(5,) * sequences)
+    if fault == "width":
+        cu_k[-1] += 32
+    else:
+        table[-1][1] = k.shape[0] if fault == "page" else -k.shape[0] - 1
+    with pytest.raises(IndexError, match="outside the cache"):
+        call(q, k, v, cu_q, cu_k, table)
+    table[-1][1] = 0     # and the process goes on
+    cu_k[-1] = cu_k[-2] + 69
+    call(q, k, v, cu_q, cu_k, table)
+
+
+@pytest.mark.parametrize("d,page", [(64, 64), (256, 32), (128, None)])
+def test_unusual_metadata_as_in_the_general_form(d, page):
+    """Pages counted from the pool's end, and a sequence of new tokens without keys."""
+    q, k, v, cu_q, cu_k, table = metadata(d, page)
+    if page:
+        table[0][0], table[2][1] = -1, -3
+    cu_k[2:] = [n - (cu_k[2] - cu_k[1]) for n in cu_k[2:]]
+    if not page:
+        k, v = k[:cu_k[-1]], v[:cu_k[-1]]
+    got, want = (call(q, k, v, cu_q, cu_k, table, form) for form in (PF.packed_prefill, PF._packed_torch))
+    assert torch.equal(got, want) and not got[cu_q[1]:cu_q[2]].any()
+
+
+def test_captured_packed_prefill():
+    q, k, v, cu_q, cu_k, table = metadata(256, 32)
+    device = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    args = (q, k, v, device(cu_q), device(cu_k), 0.1)
+    tables = device(table)
+    PF.packed_prefill(*args, tables=tables, max_keys=3000)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = PF.packed_prefill(*args, tables=tables, max_keys=3000)
+    for seed in range(3):
+        q.copy_(rows(torch.Generator(device="cuda").manual_seed(seed), *q.shape))
+        graph.replay()
+        assert torch.equal(out, PF.packed_prefill(*args, tables=tables, max_keys=3000))
