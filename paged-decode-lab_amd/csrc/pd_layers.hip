@@ -138,11 +138,12 @@ gated_norm_kernel(const float* __restrict__ o, const uint16_t* __restrict__ z,
 
 // out = silu(a) b (gate and up projections), or with kSigmoid out = a
 // sigmoid(b) where b's rows of `cols` are `b_stride` apart (attention and the
-// gate half of the query projection's heads); 8 elements a thread.
+// gate half of the query projection's heads); 8 elements a thread.  out may be
+// a: a thread has read its elements when it writes them.
 template <bool kSigmoid>
 __global__ void __launch_bounds__(256)
-gate_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
-            uint16_t* __restrict__ out, int64_t pieces, int cols, int64_t b_stride) {
+gate_kernel(const uint16_t* a, const uint16_t* __restrict__ b, uint16_t* out, int64_t pieces,
+            int cols, int64_t b_stride) {
   const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (p >= pieces) return;
   float x[8], g[8];
