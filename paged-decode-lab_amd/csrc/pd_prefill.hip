@@ -35,15 +35,18 @@
 // MFMAs (1024 clocks) and, an element, an FMA, an exponential, an addition, half
 // a maximum and 5.5 operations of the split, about 160 vector instructions (640
 // clocks and the exponentials' 190); counters show half of the SIMDs' time in
-// either, little of it at once.  So the split is the cheap one and a row tile
-// that met 0 x infinity is taken again with the other; masks are a branch in
-// the tiles that need them.
+// either, little of it at once.  So masks are a branch in the tiles that need
+// them, and infinities and NaN of V are left to a second pass: a row tile whose
+// sums are not finite is taken again with them outside the matrix products,
+// where a zero probability (a masked key's among them) would make a NaN of
+// them, and added for the rows that see their key.
 //
 // Measured on MI355X, K/V write included: four prompts of 17 to 2048 tokens, Hq
 // 32 / Hkv 8 / D 128, 3964 -> 204 us (float32 products of the materialized
-// scores before; 210 with the longer split and masks in line); 1000 tokens after
-// 3072 cached, Hq 16 / Hkv 4 / D 256, 1144 -> 168 us; 512 tokens, Hq 8 / Hkv 2 /
-// D 256, 31 us in one span (45 with 32 whole rows a wavefront).
+// scores before; 210 with a split of 7 operations and masks in line); 1000
+// tokens after 3072 cached, Hq 16 / Hkv 4 / D 256, 1144 -> 168 us; 3 us more in
+// both with the check of the metadata; 512 tokens, Hq 8 / Hkv 2 / D 256, 31 us
+// in one span (45 with 32 whole rows a wavefront).
 //
 // Few rows leave CUs idle (128 rows of each kv head a workgroup): grid.y > 1
 // cuts each row tile's keys into equal spans whose float32 (m, l, O) partials
@@ -98,26 +101,22 @@ __device__ __forceinline__ int v_swizzle(int row) {
 }
 
 // p = hi + mid + lo exactly, each a bf16 (the top 16 bits of a float32): every
-// term takes the next eight significant bits, truncated.  kSafe: subtracting
-// one from the bits before truncating keeps the remainder of a nonzero p
-// nonzero, so no term of it is zero and an infinite V contributes an infinity
-// and not the NaN of 0 x infinity.
+// term takes the next eight significant bits, truncated.
 struct Split3 {
   uint32_t hi, mid, lo;
 };
-template <bool kSafe>
-__device__ __forceinline__ uint32_t truncated(float x) {
-  const uint32_t u = __float_as_uint(x);
-  return (kSafe ? __builtin_elementwise_sub_sat(u, 1u) : u) & 0xffff0000u;
-}
-template <bool kSafe>
 __device__ __forceinline__ Split3 split3(float p) {
   Split3 s;
-  s.hi = truncated<kSafe>(p);
+  s.hi = __float_as_uint(p) & 0xffff0000u;
   const float r = p - __uint_as_float(s.hi);
-  s.mid = truncated<kSafe>(r);
+  s.mid = __float_as_uint(r) & 0xffff0000u;
   s.lo = __float_as_uint(r - __uint_as_float(s.mid));
   return s;
+}
+// 0xffff in each half of x that is an infinity or NaN.
+__device__ __forceinline__ uint32_t odd_halves(uint32_t x) {
+  const uint32_t ones = ((x & 0x7f807f80u) + 0x00800080u) >> 15 & 0x00010001u;
+  return (ones << 16) - ones;
 }
 // The upper halves of (a, b) as one dword, a in the low half.
 __device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) {
@@ -383,8 +382,7 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
             u32x4_t hi, mid, lo;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              const Split3 x = split3<kSafe>(s[n][8 * g + 2 * e]),
-                           y = split3<kSafe>(s[n][8 * g + 2 * e + 1]);
+              const Split3 x = split3(s[n][8 * g + 2 * e]), y = split3(s[n][8 * g + 2 * e + 1]);
               hi[e] = upper_halves(x.hi, y.hi);
               mid[e] = upper_halves(x.mid, y.mid);
               lo[e] = upper_halves(x.lo, y.lo);
@@ -398,12 +396,59 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
               const uint64_t a0 = __builtin_bit_cast(uint64_t, v0), a1 = __builtin_bit_cast(uint64_t, v1);
               vf[j] = u32x4_t{uint32_t(a0), uint32_t(a0 >> 32), uint32_t(a1), uint32_t(a1 >> 32)};
             }
+            // Infinities and NaN of V: not in the products, where a zero term makes a
+            // NaN of them in every row, but added for the rows that see their key.
+            uint32_t found[4] = {};
+            if constexpr (kSafe) {
+#pragma unroll
+              for (int j = 0; j < P::kOut; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const uint32_t odd = odd_halves(vf[j][e]);
+                  vf[j][e] &= ~odd;
+                  found[e] |= odd;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], lo, o[j]);
 #pragma unroll
             for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], mid, o[j]);
 #pragma unroll
             for (int j = 0; j < P::kOut; ++j) o[j] = mfma32(vf[j], hi, o[j]);
+            if constexpr (kSafe) {
+              if (__any(found[0] | found[1] | found[2] | found[3])) {
+                // The products' results are read in another block: 24 wait states.
+                asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < P::kOut; ++j) asm volatile("" : "+v"(o[j]));
+#pragma unroll 1
+                for (int key = 0; key < 16; ++key) {
+                  // Element of this key, in the lanes of one half.
+                  const int e = 4 * (key / 8) + key % 4, r = 32 * n + 16 * g + key;
+                  float p = 0.f;
+#pragma unroll
+                  for (int i = 0; i < 8; ++i)
+                    if (i == e) p = s[n][8 * g + i];
+                  const float other = xor_lanes<32>(p, lane);
+                  if ((key / 4) % 2 != half) p = other;
+                  if (first + r <= limit) {
+#pragma unroll
+                    for (int j = 0; j < P::kOut; ++j)
+#pragma unroll
+                      for (int i = 0; i < 16; i += 4) {
+                        u32x2_t x = *reinterpret_cast<const u32x2_t*>(
+                            vs + r * D * 2 + 8 * half +
+                            16 * ((P::kCols / 8 * part + 4 * j + i / 4) ^ v_swizzle<D>(r)));
+                        x.x &= odd_halves(x.x), x.y &= odd_halves(x.y);
+                        o[j][i] = fmaf(p, bf16_lo(x.x), o[j][i]);
+                        o[j][i + 1] = fmaf(p, bf16_hi(x.x), o[j][i + 1]);
+                        o[j][i + 2] = fmaf(p, bf16_lo(x.y), o[j][i + 2]);
+                        o[j][i + 3] = fmaf(p, bf16_hi(x.y), o[j][i + 3]);
+                      }
+                  }
+                }
+              }
+            }
           }
         }
       }
@@ -417,8 +462,8 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
     for (int j = 0; j < P::kOut; ++j) asm volatile("" : "+v"(o[j]));
   };
   sweep(std::false_type{});
-  // A NaN may be a zero term times an infinity: such row tiles are taken again
-  // with terms that are not zero.
+  // A NaN may be a zero probability times an infinity or NaN: such row tiles are
+  // taken again with those outside the products.
   float odd = 0.f;
 #pragma unroll
   for (int j = 0; j < P::kOut; ++j)

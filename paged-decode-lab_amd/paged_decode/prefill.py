@@ -4,7 +4,9 @@ The kernel serves what an engine on this GPU passes: bf16 tensors with head_dim 
 or 256, 16-byte rows, int32 device metadata, a page size that is a whole number of key
 tiles.  Everything else (other types and head dims, CPU tensors, tensors that autograd or
 a functorch transform follows, odd layouts, host metadata) keeps the PyTorch form, which
-materializes the scores of one sequence at a time.
+materializes the scores of one sequence at a time.  An infinity or NaN in a later token's V
+leaves earlier rows alone in the kernel; the PyTorch form multiplies it by their zero
+probabilities, a NaN.
 """
 import functools
 import math

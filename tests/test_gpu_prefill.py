@@ -247,3 +247,48 @@ def test_captured_packed_prefill():
         q.copy_(rows(torch.Generator(device="cuda").manual_seed(seed), *q.shape))
         graph.replay()
         assert torch.equal(out, PF.packed_prefill(*args, tables=tables, max_keys=3000))
+
+
+@pytest.mark.parametrize("d,page,splits", [(64, None, 1), (64, 64, 3), (128, None, 1), (128, 64, 2),
+                                           (256, None, 1), (256, 32, 1), (256, 256, 3)])
+@pytest.mark.parametrize("special", ["v_inf", "v_both", "v_nan", "k_nan"])
+def test_later_tokens_never_reach_earlier_rows(monkeypatch, d, page, splits, special):
+    """Infinities and NaN in the keys' rows: rows that see their token get them, as the
+    softmax's products do; rows before it are what they are without it."""
+    monkeypatch.setattr(PF, "_splits", lambda *a: splits)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    n, hq, prefix = 150, 4, 70 if page else 0
+    m = n + prefix
+    q, k, v = rows(gen, n, hq, d), rows(gen, m, 2, d), rows(gen, m, 2, d)
+    inf = float("inf")
+    for at, sign in ((prefix + 2, 1), (prefix + 97, -1), (m - 1, 1)):
+        if special == "k_nan":
+            k[at, 1, 3] = float("nan")
+        else:
+            v[at, 0, d - 7] = float("nan") if special == "v_nan" else sign * inf
+            if special == "v_both":
+                v[at, 0, 5], v[at, 1, 33] = inf, sign * inf
+    keys, vals, tables = k, v, None
+    if page:
+        used = -(-m // page)
+        order = np.random.default_rng(d).permutation(used + 1)[:used]
+        keys, vals = (torch.full((used + 1, page, 2, d), float("nan"), device="cuda").bfloat16() for _ in "kv")
+        for i, b in enumerate(order):
+            part = slice(page * i, min(page * (i + 1), m))
+            keys[b, :part.stop - part.start], vals[b, :part.stop - part.start] = k[part], v[part]
+        tables = torch.tensor(order[None], dtype=torch.int32, device="cuda")
+    cu = lambda x: torch.tensor([0, x], dtype=torch.int32, device="cuda")  # noqa: E731
+    assert PF._packed_ok(q, keys, vals, torch.empty_like(q), cu(n), cu(m), 0.1, tables)
+    out = PF.packed_prefill(q, keys, vals, cu(n), cu(m), 0.1, tables=tables).double().cpu()
+    q, k, v = (t.double().cpu() for t in (q, k, v))
+    for t in range(n):
+        seen = prefix + t + 1
+        for h in range(hq):
+            p = (k[:seen, h // 2] @ q[t, h] * 0.1).softmax(-1)
+            # a product and a sum a key, as a matrix product's zero terms are none of them
+            want = (p[:, None] * v[:seen, h // 2]).sum(0)
+            got = out[t, h]
+            assert torch.equal(got.isnan(), want.isnan()), (t, h)
+            assert torch.equal(got[want.isinf()], want[want.isinf()]), (t, h)
+            ok = want.isfinite()
+            assert not ok.any() or (got[ok] - want[ok]).abs().max() < 2.0 ** -6, (t, h)
