@@ -1,7 +1,10 @@
 """GPU parity of the one-token layer kernels with the same formulas in 64 bits.
 
-A product's inputs are rounded to bf16 after the norm or gate (2^-9 relative, at random
-over its terms: bounded by 2^-8 of the products' 2-norm times 4), its result once more.
+A product's inputs are rounded to bf16 after the norm or gate, its float32 sums once more
+at the end.  The reference rounds the inputs alike; where float32 may round one the other
+way (within 2^-19 of a tie), the difference is allowed.  A sum is a chain of at most K / 8
++ 24 float32 additions (its terms shared by four wavefronts or more with two sums each,
+then the wavefronts' partial sums and the residual).
 """
 import pytest
 import torch
@@ -24,14 +27,34 @@ def normed(x, w):
     return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * (1 + w.double())
 
 
-def check(got, h, w, ref=None, slack=1.0):
-    """got ~ ref, a product of h [rows, K] and w [features, K] by default."""
-    plain = h @ w.double().T
-    ref = plain if ref is None else ref
-    spread = (h.square() @ w.double().square().T).sqrt()
-    bound = 2.0 ** -6 * slack * spread + 2.0 ** -8 * ref.abs() + 1e-30
+def rounded(h):
+    """(h in bf16, how far the other rounding of values near a tie is)."""
+    low, high = ((h * (1 + s * 2.0 ** -19)).to(torch.bfloat16).double() for s in (-1, 1))
+    return h.to(torch.bfloat16).double(), (high - low).abs()
+
+
+def product(h, w):
+    """(h w^T, bound of a float32 sum of it), h [rows, K] before its rounding to bf16."""
+    h, tie = rounded(h.double())
+    w = w.double()
+    chain = (h.shape[1] / 8 + 24) * 2.0 ** -24
+    return h @ w.T, chain * (h.abs() @ w.abs().T) + tie @ w.abs().T
+
+
+def within(got, ref, bound):
+    """got (bf16) is ref, known to `bound`, rounded."""
+    bound = bound + 2.0 ** -8 * (ref.abs() + bound) + 1e-30
     worst = ((got.double() - ref).abs() / bound).max()
     assert worst <= 1, float(worst)
+
+
+def check(got, h, w):
+    within(got, *product(h, w))
+
+
+def check_sum(got, held, h, w):
+    ref, bound = product(h, w)
+    within(got, held.double() + ref, bound)
 
 
 @pytest.mark.parametrize("rows", [1, 2, 4, 5, 8, 9, 16])
@@ -66,18 +89,24 @@ def test_gate_up_and_residual(rows, dim):
     gate, up = bf16(gen, mid, dim, scale=dim ** -0.5), bf16(gen, mid, dim, scale=dim ** -0.5)
     out = torch.empty(rows, mid, device="cuda", dtype=torch.bfloat16)
     _native.norm_gate_up(x, norm, 1e-6, gate, up, out)
-    h = normed(x, norm)
-    ref = F.silu(h @ gate.double().T) * (h @ up.double().T)
-    check(out, h, gate, ref, slack=4.0)
+    (a, da), (b, db) = product(normed(x, norm), gate), product(normed(x, norm), up)
+    # silu's slope is at most 1.1, its float32 value good to 2^-19
+    within(out, F.silu(a) * b, 1.1 * da * (b.abs() + db) + F.silu(a).abs() * (db + 2.0 ** -19 * b.abs()))
     h, w, held = bf16(gen, rows, dim), bf16(gen, 72, dim, scale=0.05), bf16(gen, rows, 72)
     y = held.clone()
     _native.linear_add(h, w, y)
-    check(y, h.double(), w, held.double() + h.double() @ w.double().T)
-    d = 64
+    check_sum(y, held, h, w)
+
+
+@pytest.mark.parametrize("rows", [1, 4, 8, 9, 16])
+@pytest.mark.parametrize("dim,d", [(64, 64), (256, 64), (256, 128), (256, 256), (768, 256),
+                                   (2048, 128), (2048, 256)])
+def test_gated_residual(rows, dim, d):
+    gen = torch.Generator(device="cuda").manual_seed(rows + dim + d)
+    h, w, held = bf16(gen, rows, dim), bf16(gen, 72, dim, scale=0.05), bf16(gen, rows, 72)
     q, y = bf16(gen, rows, dim // d, 2 * d, scale=2), held.clone()
     _native.linear_add(h, w, y, q[..., d:], d)
-    g = h.double() * torch.sigmoid(q[..., d:].double()).reshape(rows, dim)
-    check(y, g, w, held.double() + g @ w.double().T)
+    check_sum(y, held, h.double() * torch.sigmoid(q[..., d:].double()).reshape(rows, dim), w)
 
 
 @pytest.mark.parametrize("dim", [6144, 1088])
@@ -87,7 +116,7 @@ def test_long_inputs_take_several_rounds(dim):
         h, w, held = bf16(gen, rows, dim), bf16(gen, 40, dim, scale=0.05), bf16(gen, rows, 40)
         y = held.clone()
         _native.linear_add(h, w, y)
-        check(y, h.double(), w, held.double() + h.double() @ w.double().T)
+        check_sum(y, held, h, w)
 
 
 @pytest.mark.parametrize("rows,held", [(1, True), (3, False), (8, True), (11, True)])
