@@ -3,6 +3,8 @@
 float32 results are held to a few float32 ulps of the largest terms of their sums, bf16
 results to half a bf16 ulp (2^-8 of the value) more.
 """
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -289,3 +291,81 @@ def test_layers_read_the_general_prefill_form(length):
     assert DL.decoder_weights(model, runner.cache.pool.block.device) is not None
     got = runner.prefill(prompt).float()
     assert (got - want).norm() <= 0.01 * want.norm()
+
+
+def generation(model, batch, length, modules, steps=3, mode="eager"):
+    """Logits of a prompt and of decode steps, then states and pages; phase 0 is the prompt,
+    phase i decode step i, and `modules` the phases that run on transformers' modules."""
+    vocab = model.config.vocab_size
+    runner = H.HybridRunner(model=model, backend="hip_matched", batch=batch, mode=mode,
+                            max_context=length + steps + 1)
+    runner.cache.pool.block.zero_()
+    prompt = [[(7 * i + 31 * j + 3) % vocab for i in range(length)] for j in range(batch)]
+    fed = [torch.tensor([(5 + 13 * s + 7 * j) % vocab for j in range(batch)], device="cuda")
+           for s in range(steps)]
+    logits = []
+    for phase in range(steps + 1):
+        handle = (model.model.layers[1].mlp.register_forward_hook(lambda *a: None)
+                  if phase in modules else None)
+        assert (DL.decoder_weights(model, runner.cache.pool.block.device) is None) == bool(handle)
+        logits.append((runner.prefill(prompt) if phase == 0 else
+                       runner.decode_step(fed[phase - 1], length + phase - 1)).float().clone())
+        if handle:
+            handle.remove()
+    return logits + [t.float() for t in runner.cache.state_tensors()] + [runner.cache.pool.block.float()]
+
+
+def agree(got, want, rel):
+    assert len(got) == len(want)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).norm() <= rel * b.norm(), (i, float((a - b).norm() / b.norm()))
+
+
+ALL = (0, 1, 2, 3)
+
+
+@pytest.mark.parametrize("batch", [1, 3, 8, 16, 17, 20])
+@pytest.mark.parametrize("length", [1, 5])
+def test_batches_agree_with_the_modules(batch, length):
+    """Few-row, one-token and row forms of the prompt and of the steps: up to 16 rows the
+    one-token products, more the row form, whose steps continue held states."""
+    model = small_model()
+    # bf16 roundings at different places, through four layers
+    agree(generation(model, batch, length, ()), generation(model, batch, length, ALL), 0.03)
+
+
+@pytest.mark.parametrize("modules", [(1, 2, 3), (0,), (2,), (0, 2)])
+@pytest.mark.parametrize("batch", [2, 18])
+def test_kernels_and_modules_take_turns(batch, modules):
+    """States, pages and lengths are the same to either, in mid-generation too."""
+    model = small_model()
+    agree(generation(model, batch, 9, modules), generation(model, batch, 9, ()), 0.03)
+
+
+@pytest.mark.parametrize("batch", [4, 18])
+def test_captured_steps_of_batches(batch):
+    model = small_model()
+    runs = [generation(model, batch, 6, (), mode=mode) for mode in ("graph", "eager")]
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("batch,length", [(1, 300), (2, 130), (1, 40), (3, 4), (20, 3)])
+def test_full_width_is_as_exact_as_the_modules(batch, length):
+    """The decoder's own widths (hidden 2048, 16 linear heads of 128, vocabulary 151936): the
+    logits are no further from those of the same weights in float64 than transformers' bf16
+    modules leave them, but for a fifth, as both are draws of the same roundings."""
+    model = H.random_init_model(H.decoder_config(num_hidden_layers=4), "cuda", seed=1)
+    exact = copy.deepcopy(model).double()
+    exact.config._attn_implementation = exact.model.config._attn_implementation = "eager"
+    vocab, steps = model.config.vocab_size, 2
+    kernels = generation(model, batch, length, (), steps)
+    modules = generation(model, batch, length, ALL, steps)
+    tokens = torch.tensor([[(7 * i + 31 * j + 3) % vocab for i in range(length)]
+                           + [(5 + 13 * s + 7 * j) % vocab for s in range(steps)]
+                           for j in range(batch)], device="cuda")
+    with torch.inference_mode():
+        want = exact(tokens, use_cache=False, logits_to_keep=steps + 1).logits
+    for s in range(steps + 1):
+        off = [float((x[s] - want[:, s]).norm() / want[:, s].norm()) for x in (kernels, modules)]
+        assert off[0] <= 1.2 * off[1] and off[1] < 0.05, (s, off)
