@@ -16,10 +16,10 @@
 // products a chunk, whose columns of dv are independent: chunk_scan_kernel
 // runs 16 of them a workgroup.
 //
-// Measured on MI355X, 16 heads of 128 x 128, against the recurrence: 20 and 15
-// us for 64 tokens, 23 and 26 for 128, 44 and 88 for 512 (prepare 18, scan
-// 26), 153 and 336 for 2049; eight sequences of 64 37 and 42, of 384 139 and
-// 213.
+// Measured on MI355X, 16 heads of 128 x 128, against the recurrence: 20 and 14
+// us for 64 tokens, 23 and 24 for 128, 44 and 88 for 512 (prepare 18, scan
+// 26), 153 and 336 for 2049; eight sequences of 64 37 and 42, of 96 51 and 60,
+// of 384 139 and 213.
 //
 // Everything is float32, products included (16x16x4 MFMAs, 64 flops a clock
 // and SIMD: what bounds both kernels).  Ratios of decays are exponentials of

@@ -28,7 +28,12 @@ from .prefill import batched_prefill, device_cus
 
 MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
 TOKEN_ROWS = 16         # rows of one MFMA operand
-CHUNK_STEPS = 96        # tokens from which the delta rule is faster in chunks (one sequence)
+# Tokens of a sequence from which the delta rule runs in chunks.  The recurrence and the
+# chunks take 14 and 20 us at 64 tokens of one sequence, 19 and 23 at 96, 24 and 23 at 128 (16
+# heads of 128 x 128); of two sequences 24 and 24 at 96, of four 28 and 33 at 96 and 35 and 34
+# at 128, of eight 42 and 37 at 64 and 60 and 51 at 96.  The lines of one and of eight
+# sequences are as far from 96; neither costs 6 us.
+CHUNK_STEPS = 96
 
 KINDS = (nn.Embedding, nn.Linear, nn.Conv1d, SiLUActivation, Qwen3_5Attention, Qwen3_5DecoderLayer,
          Qwen3_5GatedDeltaNet, Qwen3_5MLP, Qwen3_5RMSNorm, Qwen3_5RMSNormGated,

@@ -62,11 +62,12 @@ def device_cus(device):
 def _splits(workgroups, max_keys, dim, device):
     """Key spans per row tile, of 256 keys or more each: as many as fill the device's slots
     (two workgroups a CU), and at head_dim 256, where a workgroup's rows are few and its
-    spans uneven, twice that.  Measured, one span against the rule's: 104 and 78 us (2049
-    rows, Hq 8 / Hkv 2, D 256, 260 workgroups, 4 spans; 2 spans 89), 155 and 37 us (100 rows
-    after 3072, Hq 16 / Hkv 4, D 256, 16 spans), 73 and 24 us (128 after 2048, Hq 8 / Hkv 2,
-    D 128, 8 spans); two spans where the workgroups fill the slots alone: 101 instead of 84
-    us (2048 rows, Hq 32 / Hkv 8, D 128)."""
+    spans uneven, twice that.  Measured, one span against the rule's: 108 and 79 us (2049
+    rows, Hq 8 / Hkv 2, D 256, 258 workgroups, 4 spans; 2 spans 91), 176 and 42 us (100 rows
+    after 3072, Hq 16 / Hkv 4, D 256, 12 spans; 8 spans 40), 80 and 26 us (128 after 2048, Hq
+    8 / Hkv 2, D 128, 8 spans), 30 and 25 us (512 rows, Hq 8 / Hkv 2, D 256, 2 spans; 4 spans
+    22); two spans where the workgroups fill the slots alone: 103 instead of 87 us (2048
+    rows, Hq 32 / Hkv 8, D 128)."""
     if not isinstance(max_keys, numbers.Integral):
         return 1
     cus = device_cus(device)
