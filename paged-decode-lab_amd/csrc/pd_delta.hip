@@ -42,10 +42,14 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
+using pd::aligned16;
+using pd::as_stream;
+using pd::launch_status;
 
 constexpr int kChunk = 64;
 static_assert(kChunk == 64, "four 16-token tiles");
@@ -376,8 +380,6 @@ __global__ void __launch_bounds__(256, 1) chunk_scan_kernel(const ChunkArgs p) {
       if (i / KW == wave) state[(16 * i + e) * DV] = s[i][e];
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 // Floats of workspace per (sequence, value head, chunk), G_C padded to 16 bytes.
 int64_t chunk_floats(int dk, int dv) { return int64_t(kChunk) * (3 * dk + dv + kChunk) + 4; }
 
@@ -420,7 +422,7 @@ extern "C" int pd_delta_chunks(const float* act, const float* gates, float* stat
   // XCD (with a multiple of eight heads) and share its L2.
   const dim3 prepare{unsigned(hv), unsigned(chunks), unsigned(batch)};
   const dim3 scan{unsigned(hv), unsigned(dv / 16), unsigned(batch)};
-  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const hipStream_t st = as_stream(stream);
   const auto go = [&](auto first, auto second) {
     hipLaunchKernelGGL(first, prepare, dim3(kPrepareThreads), 0, st, p);
     hipLaunchKernelGGL(second, scan, dim3(256), 0, st, p);
@@ -431,8 +433,5 @@ extern "C" int pd_delta_chunks(const float* act, const float* gates, float* stat
   else
     dv == 64 ? go(chunk_prepare_kernel<128, 64>, chunk_scan_kernel<128, 64>)
              : go(chunk_prepare_kernel<128, 128>, chunk_scan_kernel<128, 128>);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "pd_delta_chunks launch failed: %s", hipGetErrorString(err));
-  return PD_OK;
+  return launch_status("pd_delta_chunks");
 }

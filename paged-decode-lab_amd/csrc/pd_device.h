@@ -14,6 +14,7 @@ namespace pdk {
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef float floatx16_t __attribute__((ext_vector_type(16)));
 typedef float floatx2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
@@ -39,6 +40,8 @@ __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_ex
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 __device__ __forceinline__ float ln_fast(float x) { return __builtin_amdgcn_logf(x) * kLn2; }
 __device__ __forceinline__ float rcp_fast(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + exp_fast(-x)); }
+__device__ __forceinline__ float silu(float x) { return x / (1.f + exp_fast(-x)); }
 
 // x of lane L ^ M, for M = 1, 2, 4, 8, 16 or 32, with VALU lane moves (no LDS
 // round trip, unlike ds_bpermute).  Lane layouts checked on gfx950 with an
@@ -796,6 +799,28 @@ __device__ __forceinline__ void mfma_result_barrier(floatx4_t (&x)[N]) {
 // bf16 bits of (a, b), round to nearest even (v_cvt_pk_bf16_f32).
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2_t{a, b}, bf16x2_t));
+}
+
+// Eight bf16 of a 16-byte piece as floats, and back (rounded to nearest even).
+__device__ __forceinline__ void unpack8(u32x4_t t, float (&x)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[2 * i] = bf16_lo(t[i]), x[2 * i + 1] = bf16_hi(t[i]);
+}
+__device__ __forceinline__ u32x4_t pack8(const float (&x)[8]) {
+  u32x4_t t;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
+  return t;
+}
+
+// D += A B of one bf16 tile, 8 elements of the contraction a lane.
+__device__ __forceinline__ floatx4_t mfma16(u32x4_t a, u32x4_t b, floatx4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx16_t mfma32(u32x4_t a, u32x4_t b, floatx16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
 // Block-table window of one sequence: lane `lane` holds in e[r] the entry of

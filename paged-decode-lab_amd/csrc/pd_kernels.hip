@@ -41,10 +41,13 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
+using pd::aligned16;
+using pd::launch_status;
 
 template <int D, int GP>
 struct MatchedShared {
@@ -1620,15 +1623,6 @@ ml_online_merge_loop_kernel(const float* __restrict__ maxima, const float* __res
 }
 
 // --------------------------------------------------------------- launchers
-
-int launch_status(const char* what) {
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "%s launch failed: %s", what, hipGetErrorString(err));
-  return PD_OK;
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 int check_qkv(const void* q, int64_t qsb, int64_t qsh, const void* k, const void* v,
               const int32_t* table, int32_t width, const int32_t* lengths, int32_t batch,

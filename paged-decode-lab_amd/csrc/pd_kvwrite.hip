@@ -13,8 +13,12 @@
 #include <cstdint>
 
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
+
+using pd::aligned16;
+using pd::launch_status;
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -73,15 +77,6 @@ store_pages_kernel(const uint16_t* __restrict__ key, int64_t ksb, int64_t ksh, i
       *reinterpret_cast<const u32x4_t*>(value + b * vsb + h * vsh + s * vss + 8 * c);
   *reinterpret_cast<u32x4_t*>(k_pages + dst) = kx;
   *reinterpret_cast<u32x4_t*>(v_pages + dst) = vx;
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-int launch_status(const char* what) {
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "%s launch failed: %s", what, hipGetErrorString(err));
-  return PD_OK;
 }
 
 }  // namespace

@@ -16,24 +16,15 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
-
-__device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + exp_fast(-x)); }
-__device__ __forceinline__ float silu(float x) { return x / (1.f + exp_fast(-x)); }
-
-__device__ __forceinline__ void unpack8(u32x4_t t, float (&x)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) x[2 * i] = bf16_lo(t[i]), x[2 * i + 1] = bf16_hi(t[i]);
-}
-__device__ __forceinline__ u32x4_t pack8(const float (&x)[8]) {
-  u32x4_t t;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) t[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
-  return t;
-}
+using pd::all_aligned16;
+using pd::as_stream;
+using pd::launch_status;
+using pd::u16;
 
 // E consecutive bf16 (E = 1, 2 or 4) at element p.
 template <int E>
@@ -346,18 +337,14 @@ gates_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ wa,
   const int f0 = blockIdx.y * 16;
   const int64_t feature = int64_t(min(f0 + op, hv - 1)) * K + 8 * quad;
   const uint16_t* x = h + min(r0 + op, rows - 1) * K + 8 * quad;
-  const auto mfma = [](u32x4_t a, u32x4_t b, floatx4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  };
   floatx4_t acc[2] = {};
 #pragma unroll 4
   for (int k = 64 * w; k < K; k += 64 * kGateWaves) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const u32x4_t xv = load16(x + k + 32 * s);
-      acc[0] = mfma(load16(wa + feature + k + 32 * s), xv, acc[0]);
-      acc[1] = mfma(load16(wb + feature + k + 32 * s), xv, acc[1]);
+      acc[0] = mfma16(load16(wa + feature + k + 32 * s), xv, acc[0]);
+      acc[1] = mfma16(load16(wb + feature + k + 32 * s), xv, acc[1]);
     }
   }
   mfma_result_barrier(acc);
@@ -588,21 +575,6 @@ __global__ void __launch_bounds__(256) qk_rope_kernel(const QkArgs p) {
     if (kp) store_bf16<E>(kp + hk * D + E * lane, x);
   }
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-template <typename... Ts>
-bool all_aligned16(Ts... p) { return (aligned16(p) && ...); }
-
-int launch_status(const char* what) {
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "%s launch failed: %s", what, hipGetErrorString(err));
-  return PD_OK;
-}
-
-hipStream_t as_stream(pd_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
-const uint16_t* u16(const void* p) { return static_cast<const uint16_t*>(p); }
-uint16_t* u16(void* p) { return static_cast<uint16_t*>(p); }
 
 bool valid_linear_dims(int dk, int dv) {
   return (dk == 64 || dk == 128) && (dv == 64 || dv == 128);

@@ -34,12 +34,14 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
-
-typedef float floatx16_t __attribute__((ext_vector_type(16)));
+using pd::aligned16;
+using pd::as_stream;
+using pd::launch_status;
 
 constexpr int kMaxSegments = 4;
 constexpr int BN = 128;
@@ -53,11 +55,6 @@ struct LinearArgs {
   int m[kMaxSegments];
   int segments, rows, K, row_tiles, feature_tiles;
 };
-
-__device__ __forceinline__ floatx16_t mfma32(u32x4_t a, u32x4_t b, floatx16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 // Waits until at most `n` of this wavefront's copies are under way.
 template <int n>
@@ -227,8 +224,6 @@ __global__ void __launch_bounds__(256, 1) linear_kernel(const LinearArgs a) {
   }
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 template <int kEpi, int BM>
 int launch(LinearArgs& a, pd_stream_t stream) {
   constexpr int per = kEpi == kSiluMul ? BM / 2 : BM;
@@ -239,11 +234,8 @@ int launch(LinearArgs& a, pd_stream_t stream) {
   if (grid > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
   a.feature_tiles = int(tiles);
   hipLaunchKernelGGL((linear_kernel<kEpi, BM>), dim3(unsigned(grid)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), a);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "pd_linears launch failed: %s", hipGetErrorString(err));
-  return PD_OK;
+                     as_stream(stream), a);
+  return launch_status("pd_linears");
 }
 
 }  // namespace

@@ -58,13 +58,14 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
-
-typedef float floatx16_t __attribute__((ext_vector_type(16)));
-
+using pd::aligned16;
+using pd::as_stream;
+using pd::launch_status;
 
 struct PrefillArgs {
   const uint16_t *q, *k, *v;
@@ -121,11 +122,6 @@ __device__ __forceinline__ uint32_t odd_halves(uint32_t x) {
 // The upper halves of (a, b) as one dword, a in the low half.
 __device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_perm(b, a, 0x07060302u);
-}
-
-__device__ __forceinline__ floatx16_t mfma32(u32x4_t a, u32x4_t b, floatx16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
 // The sequence and row tile of grid tile `t` (counted from the last), for
@@ -595,8 +591,6 @@ __global__ void __launch_bounds__(256) check_packed_kernel(const PackedCheck a) 
   if (outside) a.flags[1] = 1;
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 template <int D>
 void launch(const PrefillArgs& a, unsigned grid, hipStream_t stream) {
   const dim3 g(grid, unsigned(a.splits));
@@ -692,17 +686,14 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
                              : int64_t(num_seqs) * ((int64_t(seq_len) * G + kRows - 1) / kRows);
   const int64_t grid = tiles * num_kv_heads;
   if (grid > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
-  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const hipStream_t st = as_stream(stream);
   if (head_dim == 64)
     launch<64>(a, unsigned(grid), st);
   else if (head_dim == 128)
     launch<128>(a, unsigned(grid), st);
   else
     launch<256>(a, unsigned(grid), st);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "pd_prefill launch failed: %s", hipGetErrorString(err));
-  return PD_OK;
+  return launch_status("pd_prefill");
 }
 
 extern "C" int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs,
@@ -718,9 +709,6 @@ extern "C" int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t
                       num_seqs, table_width, page_size, flags};
   const int64_t blocks = (int64_t(num_seqs) * (table ? table_width : 1) + 255) / 256;
   hipLaunchKernelGGL(check_packed_kernel, dim3(unsigned(blocks < 256 ? blocks : 256)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), a);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "pd_check_packed launch failed: %s", hipGetErrorString(err));
-  return PD_OK;
+                     as_stream(stream), a);
+  return launch_status("pd_check_packed");
 }

@@ -39,24 +39,15 @@
 
 #include "pd_device.h"
 #include "pd_internal.h"
+#include "pd_launch.h"
 
 namespace {
 
 using namespace pdk;
-
-__device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + exp_fast(-x)); }
-__device__ __forceinline__ float silu(float x) { return x / (1.f + exp_fast(-x)); }
-
-__device__ __forceinline__ void unpack8(u32x4_t t, float (&x)[8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) x[2 * i] = bf16_lo(t[i]), x[2 * i + 1] = bf16_hi(t[i]);
-}
-__device__ __forceinline__ u32x4_t pack8(const float (&x)[8]) {
-  u32x4_t t;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) t[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
-  return t;
-}
+using pd::all_aligned16;
+using pd::as_stream;
+using pd::launch_status;
+using pd::u16;
 
 constexpr int kMaxRows = 16;     // activation rows of a product
 constexpr int kMaxSegments = 4;  // weight matrices sharing one input
@@ -81,11 +72,6 @@ struct TokenArgs {
 enum { kPlain, kNorm, kGated };               // prologues
 enum { kStore, kConv, kResidual, kSiluMul };  // epilogues
 enum { kWide, kHalves, kPairs };              // forms
-
-__device__ __forceinline__ floatx4_t mfma16(u32x4_t a, u32x4_t b, floatx4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
 
 // Input rows normed to bf16 in LDS, rows K + 8 elements apart.  kItems rows of
 // up to 8 elements a thread (K <= 2048) are held in registers between the sum
@@ -436,21 +422,6 @@ __global__ void __launch_bounds__(kStepThreads) delta_step_kernel(const StepArgs
     p.out[at] = uint16_t(bf16_bits(o * rsqrtf(ss / DV + p.eps) * weight * silu(z)));
   }
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-template <typename... Ts>
-bool all_aligned16(Ts... p) { return (aligned16(p) && ...); }
-
-int launch_status(const char* what) {
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess)
-    return pd::fail(PD_ELAUNCH, "%s launch failed: %s", what, hipGetErrorString(err));
-  return PD_OK;
-}
-
-hipStream_t as_stream(pd_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
-const uint16_t* u16(const void* p) { return static_cast<const uint16_t*>(p); }
-uint16_t* u16(void* p) { return static_cast<uint16_t*>(p); }
 
 constexpr int kMaxLds = 160 * 1024;
 
