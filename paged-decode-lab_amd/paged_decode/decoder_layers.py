@@ -28,6 +28,7 @@ from .prefill import batched_prefill, device_cus
 
 MAX_HIDDEN = 8192       # add_rms_norm keeps a row in the registers of one workgroup
 TOKEN_ROWS = 16         # rows of one MFMA operand
+MAX_BATCH, MAX_STEPS = 65535, 65535 * 16    # what the convolution's grid holds
 # Tokens of a sequence from which the delta rule runs in chunks.  The recurrence and the
 # chunks take 14 and 20 us at 64 tokens of one sequence, 19 and 23 at 96, 24 and 23 at 128 (16
 # heads of 128 x 128); of two sequences 24 and 24 at 96, of four 28 and 33 at 96 and 35 and 34
@@ -255,10 +256,11 @@ def _linear_states(cache, index, batch, weights, device):
 
 def decoder_states(runner, weights, tokens):
     """The linear-attention states of every layer, or None where the kernels cannot run:
-    another batch than the runner's, several steps on top of earlier tokens, or states of
-    another form."""
+    another batch than the runner's, more tokens than a grid holds, several steps on top of
+    earlier tokens, or states of another form."""
     cache, found = runner.cache, {}
-    if tokens.dim() != 2 or tokens.shape[0] != runner.batch or tokens.shape[1] < 1:
+    if (tokens.dim() != 2 or tokens.shape[0] != runner.batch or tokens.shape[0] > MAX_BATCH
+            or not 1 <= tokens.shape[1] <= MAX_STEPS):
         return None
     steps = tokens.shape[1]
     for index in cache.linear:

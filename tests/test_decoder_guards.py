@@ -2,6 +2,7 @@
 import os
 import subprocess
 import sys
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -110,3 +111,13 @@ def test_changed_instances_keep_the_modules(change):
     else:
         layer.mlp.float()
     assert not served(model)
+
+
+@pytest.mark.parametrize("batch,steps,runs", [(1, 65535 * 16, True), (1, 65535 * 16 + 1, False),
+                                              (65536, 1, False), (2, 0, False)])
+def test_token_counts_past_the_grids_keep_the_modules(batch, steps, runs):
+    runner = SimpleNamespace(batch=batch, device=CPU, cache=SimpleNamespace(linear={}))
+    tokens = torch.zeros(1, 1, dtype=torch.long).expand(batch, steps)
+    assert (DL.decoder_states(runner, None, tokens) is not None) == runs
+    other_batch = SimpleNamespace(**{**vars(runner), "batch": batch + 1})
+    assert DL.decoder_states(other_batch, None, tokens) is None

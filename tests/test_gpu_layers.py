@@ -350,7 +350,7 @@ def test_captured_steps_of_batches(batch):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("batch,length", [(1, 300), (2, 130), (1, 40), (3, 4), (20, 3)])
+@pytest.mark.parametrize("batch,length", [(1, 300), (2, 130), (1, 40), (3, 4), (16, 1), (20, 3)])
 def test_full_width_is_as_exact_as_the_modules(batch, length):
     """The decoder's own widths (hidden 2048, 16 linear heads of 128, vocabulary 151936): the
     logits are no further from those of the same weights in float64 than transformers' bf16
