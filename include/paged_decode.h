@@ -306,15 +306,26 @@ int pd_prefill(const void* q, const int64_t* q_strides, const void* k, const int
                int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
                float* part_o, float* part_ml, pd_stream_t stream);
 
-/* Checks the metadata of a packed or paged pd_prefill on the device.  Sets
- * flags[0] (int32 [2], zeroed by the caller, device or pinned host memory)
- * where sequences are not rows of the tensors in order, or a sequence of new
- * tokens has no keys or a page in [-num_pages, -1]; flags[1] where one has
- * more keys than its table's entries hold or any other page outside the pool. */
-int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs, int64_t total_q,
-                    int64_t total_k, const int32_t* table, int64_t table_stride_b,
-                    int32_t table_width, int32_t page_size, int64_t num_pages, int32_t* flags,
-                    pd_stream_t stream);
+/* pd_prefill of packed or paged sequences whose metadata are checked on the
+ * device.  verdicts: int32 [PD_CHECK_WORDS] of pinned host memory, zeroed by the
+ * caller and kept until pd_check_wait returns, which waits for the check, not
+ * for the attention, and gives what was found:
+ *   PD_CHECK_ODD      sequences are not rows of the tensors in order, or one of
+ *                     new tokens has no keys or a page in [-num_pages, -1];
+ *   PD_CHECK_OUTSIDE  a sequence has more keys than its table's entries hold,
+ *                     or any other page outside the pool. */
+#define PD_CHECK_WORDS 64
+#define PD_CHECK_ODD 1
+#define PD_CHECK_OUTSIDE 2
+int pd_prefill_checked(const void* q, const int64_t* q_strides, const void* k,
+                       const int64_t* k_strides, const void* v, const int64_t* v_strides, void* out,
+                       const int64_t* out_strides, const int32_t* cu_q, const int32_t* cu_k,
+                       int32_t num_seqs, int32_t seq_len, int64_t total_q, int64_t total_k,
+                       const int32_t* table, int64_t table_stride_b, int32_t table_width,
+                       int32_t page_size, int64_t num_pages, int32_t num_heads,
+                       int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
+                       float* part_o, float* part_ml, int32_t* verdicts, pd_stream_t stream);
+int pd_check_wait(const int32_t* verdicts, pd_stream_t stream, int32_t* found);
 
 /* The decoder layer between its matrix products.  bf16 tensors are contiguous
  * and 16-byte aligned unless strides are given; arithmetic is float32. */

@@ -44,15 +44,16 @@
 // Measured on MI355X, K/V write included: four prompts of 17 to 2048 tokens, Hq
 // 32 / Hkv 8 / D 128, 3964 -> 204 us (float32 products of the materialized
 // scores before; 210 with a split of 7 operations and masks in line); 1000
-// tokens after 3072 cached, Hq 16 / Hkv 4 / D 256, 1144 -> 168 us; 3 us more in
-// both with the check of the metadata; 512 tokens, Hq 8 / Hkv 2 / D 256, 31 us
-// in one span (45 with 32 whole rows a wavefront).
+// tokens after 3072 cached, Hq 16 / Hkv 4 / D 256, 1144 -> 168 us; 512 tokens,
+// Hq 8 / Hkv 2 / D 256, 31 us in one span (45 with 32 whole rows a wavefront).
 //
 // Few rows leave CUs idle (128 rows of each kv head a workgroup): grid.y > 1
 // cuts each row tile's keys into equal spans whose float32 (m, l, O) partials
 // prefill_merge_kernel combines.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 
@@ -76,6 +77,7 @@ struct PrefillArgs {
   int64_t total_q, total_k, num_pages;
   int num_seqs, seq_len, table_width, page_size, num_kv_heads, G, splits;
   float scale;
+  int32_t* verdicts;        // of the packed metadata, or null
 };
 
 template <int D>
@@ -156,6 +158,45 @@ __device__ __forceinline__ bool find_tile(const PrefillArgs& a, int t, int lane,
   return false;
 }
 
+// What the caller must know of packed metadata, which only the device holds.
+// The first workgroups look at a share of them before their tile, and each
+// wavefront writes kChecked and the bits it found to its word of pinned memory,
+// which the host polls while the attention runs.  A call of 5 rows takes 15 us
+// unchecked and 20 so; 27 with a kernel and an event of the check's own, which
+// also cost the stream 3 to 5 us a call, 22 with a kernel and the poll.
+constexpr int kChecked = 4, kCheckGroups = PD_CHECK_WORDS / 4;
+
+template <bool kPaged>
+__device__ __forceinline__ void check_packed(const PrefillArgs& a, int tid) {
+  const int width = kPaged ? a.table_width : 1;
+  const int64_t total = int64_t(a.num_seqs) * width;
+  const int step = min(int(gridDim.x), kCheckGroups) * 256;
+  bool odd = false, outside = false;
+  for (int64_t at = blockIdx.x * 256 + tid; at < total; at += step) {
+    const int64_t i = at / width;
+    const int entry = int(at - i * width);
+    const int64_t k0 = a.cu_k[i], k1 = a.cu_k[i + 1], nk = k1 - k0;
+    if (entry == 0) {
+      const int64_t q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
+      odd |= q0 < 0 || q1 < q0 || q1 > a.total_q || nk < 0 || (nk == 0 && q1 > q0);
+      if (kPaged)
+        outside |= nk > int64_t(width) * a.page_size;
+      else
+        odd |= k0 < 0 || k1 > a.total_k;
+    }
+    if (kPaged && int64_t(entry) * a.page_size < nk) {
+      const int64_t page = a.table[i * a.tsb + entry];
+      odd |= page < 0;
+      outside |= page >= a.num_pages || page < -a.num_pages;
+    }
+  }
+  const int found =
+      kChecked | (__any(odd) ? PD_CHECK_ODD : 0) | (__any(outside) ? PD_CHECK_OUTSIDE : 0);
+  if ((tid & 63) == 0)
+    __hip_atomic_store(a.verdicts + 4 * blockIdx.x + (tid >> 6), found, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // kPaged: K and V are pages read through the table, page_size a multiple of
 // the tile; else rows of the call's own tensors.
 template <int D, bool kPaged>
@@ -168,6 +209,8 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = wave % (kRows / 32), part = wave / (kRows / 32);  // rows 32 w, columns of `part`
   const int half = lane >> 5, col = lane & 31;
+
+  if (a.verdicts && blockIdx.x < kCheckGroups && blockIdx.y == 0) check_packed<kPaged>(a, tid);
 
   // Longest first: tiles are counted from the last, whose rows see most keys.
   const int id = blockIdx.x;
@@ -554,43 +597,6 @@ prefill_merge_kernel(const PrefillArgs a, int64_t all) {
   for (int e = 0; e < E; ++e) out[e] = uint16_t(bf16_bits(o[e] * inv));
 }
 
-// What the caller must know of packed metadata, which only the device holds:
-// flags[0] where sequences are not rows of the tensors in order, or a sequence
-// of new tokens has no keys or a page counted from the pool's end; flags[1]
-// where a sequence reaches past its table or to a page that does not exist.
-// Other flags are left alone.  One thread a table entry, and a sequence.
-struct PackedCheck {
-  const int32_t *cu_q, *cu_k, *table;
-  int64_t total_q, total_k, num_pages, tsb;
-  int num_seqs, table_width, page_size;
-  int32_t* flags;
-};
-
-__global__ void __launch_bounds__(256) check_packed_kernel(const PackedCheck a) {
-  const int width = a.table ? a.table_width : 1;
-  const int64_t total = int64_t(a.num_seqs) * width, step = int64_t(gridDim.x) * 256;
-  bool odd = false, outside = false;
-  for (int64_t at = int64_t(blockIdx.x) * 256 + threadIdx.x; at < total; at += step) {
-    const int i = int(at / width), entry = int(at % width);
-    const int64_t k0 = a.cu_k[i], k1 = a.cu_k[i + 1], nk = k1 - k0;
-    if (entry == 0) {
-      const int64_t q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
-      odd |= q0 < 0 || q1 < q0 || q1 > a.total_q || nk < 0 || (nk == 0 && q1 > q0);
-      if (a.table)
-        outside |= nk > int64_t(width) * a.page_size;
-      else
-        odd |= k0 < 0 || k1 > a.total_k;
-    }
-    if (a.table && int64_t(entry) * a.page_size < nk) {
-      const int64_t page = a.table[i * a.tsb + entry];
-      odd |= page < 0;
-      outside |= page >= a.num_pages || page < -a.num_pages;
-    }
-  }
-  if (odd) a.flags[0] = 1;
-  if (outside) a.flags[1] = 1;
-}
-
 template <int D>
 void launch(const PrefillArgs& a, unsigned grid, hipStream_t stream) {
   const dim3 g(grid, unsigned(a.splits));
@@ -605,16 +611,13 @@ void launch(const PrefillArgs& a, unsigned grid, hipStream_t stream) {
   }
 }
 
-}  // namespace
-
-extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k,
-                          const int64_t* k_strides, const void* v, const int64_t* v_strides,
-                          void* out, const int64_t* out_strides, const int32_t* cu_q,
-                          const int32_t* cu_k, int32_t num_seqs, int32_t seq_len, int64_t total_q,
-                          int64_t total_k, const int32_t* table, int64_t table_stride_b,
-                          int32_t table_width, int32_t page_size, int64_t num_pages,
-                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, double scale,
-                          int32_t splits, float* part_o, float* part_ml, pd_stream_t stream) {
+int run_prefill(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                const void* v, const int64_t* v_strides, void* out, const int64_t* out_strides,
+                const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs, int32_t seq_len,
+                int64_t total_q, int64_t total_k, const int32_t* table, int64_t table_stride_b,
+                int32_t table_width, int32_t page_size, int64_t num_pages, int32_t num_heads,
+                int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
+                float* part_o, float* part_ml, int32_t* verdicts, pd_stream_t stream) {
   pd::clear_error();
   if (num_seqs < 1 || num_heads < 1 || num_kv_heads < 1 || num_heads % num_kv_heads)
     return pd::fail(PD_EINVAL, "sequences and heads must be positive, heads divisible by kv heads");
@@ -622,7 +625,11 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
     return pd::fail(PD_EINVAL, "prefill supports head_dim 64, 128, or 256");
   if (total_q < 0 || total_q > 0x7fffffff || total_k < 0 || total_k > 0x7fffffff)
     return pd::fail(PD_EINVAL, "token counts must lie in [0, 2^31)");
-  if (total_q == 0) return PD_OK;
+  if (verdicts && !cu_q) return pd::fail(PD_EINVAL, "only packed metadata are checked");
+  if (total_q == 0) {
+    for (int word = 0; verdicts && word < PD_CHECK_WORDS; ++word) verdicts[word] = kChecked;
+    return PD_OK;
+  }
   if (!q || !k || !v || !out || !q_strides || !k_strides || !v_strides || !out_strides)
     return pd::fail(PD_EINVAL, "null tensor pointer");
   if ((cu_q == nullptr) != (cu_k == nullptr) || (table && !cu_q))
@@ -686,6 +693,9 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
                              : int64_t(num_seqs) * ((int64_t(seq_len) * G + kRows - 1) / kRows);
   const int64_t grid = tiles * num_kv_heads;
   if (grid > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
+  a.verdicts = verdicts;
+  for (int word = 4 * int(std::min<int64_t>(grid, kCheckGroups)); verdicts && word < PD_CHECK_WORDS; ++word)
+    verdicts[word] = kChecked;  // workgroups that there are not
   const hipStream_t st = as_stream(stream);
   if (head_dim == 64)
     launch<64>(a, unsigned(grid), st);
@@ -696,19 +706,60 @@ extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k
   return launch_status("pd_prefill");
 }
 
-extern "C" int pd_check_packed(const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs,
-                               int64_t total_q, int64_t total_k, const int32_t* table,
-                               int64_t table_stride_b, int32_t table_width, int32_t page_size,
-                               int64_t num_pages, int32_t* flags, pd_stream_t stream) {
+}  // namespace
+
+extern "C" int pd_prefill(const void* q, const int64_t* q_strides, const void* k,
+                          const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          void* out, const int64_t* out_strides, const int32_t* cu_q,
+                          const int32_t* cu_k, int32_t num_seqs, int32_t seq_len, int64_t total_q,
+                          int64_t total_k, const int32_t* table, int64_t table_stride_b,
+                          int32_t table_width, int32_t page_size, int64_t num_pages,
+                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, double scale,
+                          int32_t splits, float* part_o, float* part_ml, pd_stream_t stream) {
+  return run_prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu_k, num_seqs,
+                     seq_len, total_q, total_k, table, table_stride_b, table_width, page_size,
+                     num_pages, num_heads, num_kv_heads, head_dim, scale, splits, part_o, part_ml,
+                     nullptr, stream);
+}
+
+extern "C" int pd_prefill_checked(const void* q, const int64_t* q_strides, const void* k,
+                       const int64_t* k_strides, const void* v, const int64_t* v_strides, void* out,
+                       const int64_t* out_strides, const int32_t* cu_q, const int32_t* cu_k,
+                       int32_t num_seqs, int32_t seq_len, int64_t total_q, int64_t total_k,
+                       const int32_t* table, int64_t table_stride_b, int32_t table_width,
+                       int32_t page_size, int64_t num_pages, int32_t num_heads,
+                       int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
+                       float* part_o, float* part_ml, int32_t* verdicts, pd_stream_t stream) {
+  return run_prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu_k, num_seqs,
+                     seq_len, total_q, total_k, table, table_stride_b, table_width, page_size,
+                     num_pages, num_heads, num_kv_heads, head_dim, scale, splits, part_o, part_ml,
+                     verdicts, stream);
+}
+
+extern "C" int pd_check_wait(const int32_t* verdicts, pd_stream_t stream, int32_t* found) {
   pd::clear_error();
-  if (num_seqs < 1) return pd::fail(PD_EINVAL, "sequences must be positive");
-  if (!cu_q || !cu_k || !flags) return pd::fail(PD_EINVAL, "null tensor pointer");
-  if (table && (table_width < 1 || page_size < 1))
-    return pd::fail(PD_EINVAL, "empty table or pages");
-  const PackedCheck a{cu_q, cu_k, table, total_q, total_k, num_pages, table_stride_b,
-                      num_seqs, table_width, page_size, flags};
-  const int64_t blocks = (int64_t(num_seqs) * (table ? table_width : 1) + 255) / 256;
-  hipLaunchKernelGGL(check_packed_kernel, dim3(unsigned(blocks < 256 ? blocks : 256)), dim3(256), 0,
-                     as_stream(stream), a);
-  return launch_status("pd_check_packed");
+  if (!verdicts || !found) return pd::fail(PD_EINVAL, "null pointer");
+  *found = 0;
+  // The stream is asked once a millisecond, which costs it a packet: when it has
+  // ended, every write has been made.
+  using Clock = std::chrono::steady_clock;
+  auto ask = Clock::now() + std::chrono::milliseconds(1);
+  bool done = false;
+  for (int word = 0; word < PD_CHECK_WORDS; ++word) {
+    int32_t v = 0;
+    for (unsigned spin = 1;; ++spin) {
+      v = __atomic_load_n(verdicts + word, __ATOMIC_ACQUIRE);
+      if (v || done) break;
+      if (spin % 64 == 0 && Clock::now() >= ask) {
+        const hipError_t state = hipStreamQuery(as_stream(stream));
+        if (state != hipSuccess && state != hipErrorNotReady)
+          return pd::fail(PD_ELAUNCH, "pd_check_wait: %s", hipGetErrorString(state));
+        done = state == hipSuccess;
+        ask = Clock::now() + std::chrono::milliseconds(1);
+      }
+    }
+    if (!v) return pd::fail(PD_ELAUNCH, "pd_check_wait: the check did not run");
+    *found |= v & (PD_CHECK_ODD | PD_CHECK_OUTSIDE);
+  }
+  return PD_OK;
 }

@@ -52,7 +52,10 @@ SIGNATURES = {
                           _i32, _vp, _i32, _i32, _i32, _i32, _vp],
     "pd_prefill": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _vp,
                    _i64, _i32, _i32, _i64, _i32, _i32, _i32, _dbl, _i32, _vp, _vp, _vp],
-    "pd_check_packed": [_vp, _vp, _i32, _i64, _i64, _vp, _i64, _i32, _i32, _i64, _vp, _vp],
+    "pd_prefill_checked": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64,
+                           _vp, _i64, _i32, _i32, _i64, _i32, _i32, _i32, _dbl, _i32, _vp, _vp, _vp,
+                           _vp],
+    "pd_check_wait": [_vp, _vp, ctypes.POINTER(_i32)],
     "pd_add_rms_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
     "pd_gated_norm": [_vp, _vp, _vp, _vp, _i64, _i32, _dbl, _vp],
     "pd_silu_mul": [_vp, _vp, _vp, _i64, _vp],
@@ -267,26 +270,31 @@ _Strides = _i64 * 3
 
 def prefill(q, q_strides, k, k_strides, v, v_strides, out, out_strides, cu_q, cu_k, num_seqs,
             seq_len, total_q, total_k, tables, page_size, num_pages, heads, kv_heads, head_dim,
-            scale, splits, part_o, part_ml):
-    """pd_prefill; strides are (batch, token, head) in elements."""
-    check(lib().pd_prefill(
-        q.data_ptr(), _Strides(*q_strides), k.data_ptr(), _Strides(*k_strides), v.data_ptr(),
-        _Strides(*v_strides), out.data_ptr(), _Strides(*out_strides),
-        None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
-        num_seqs, seq_len, total_q, total_k, None if tables is None else tables.data_ptr(),
-        0 if tables is None else tables.stride(0), 0 if tables is None else tables.shape[1],
-        page_size, num_pages, heads, kv_heads, head_dim, scale, splits,
-        None if part_o is None else part_o.data_ptr(),
-        None if part_ml is None else part_ml.data_ptr(), stream_handle(q.device)))
+            scale, splits, part_o, part_ml, verdicts=None):
+    """pd_prefill, or with verdicts (int32 [CHECK_WORDS] pinned, zero) pd_prefill_checked;
+    strides are (batch, token, head) in elements."""
+    args = (q.data_ptr(), _Strides(*q_strides), k.data_ptr(), _Strides(*k_strides), v.data_ptr(),
+            _Strides(*v_strides), out.data_ptr(), _Strides(*out_strides),
+            None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
+            num_seqs, seq_len, total_q, total_k, None if tables is None else tables.data_ptr(),
+            0 if tables is None else tables.stride(0), 0 if tables is None else tables.shape[1],
+            page_size, num_pages, heads, kv_heads, head_dim, scale, splits,
+            None if part_o is None else part_o.data_ptr(),
+            None if part_ml is None else part_ml.data_ptr())
+    if verdicts is None:
+        check(lib().pd_prefill(*args, stream_handle(q.device)))
+    else:
+        check(lib().pd_prefill_checked(*args, verdicts.data_ptr(), stream_handle(q.device)))
 
 
-def check_packed(cu_q, cu_k, num_seqs, total_q, total_k, tables, page_size, num_pages, flags):
-    """pd_check_packed; flags int32 [2] pinned, zero."""
-    check(lib().pd_check_packed(
-        cu_q.data_ptr(), cu_k.data_ptr(), num_seqs, total_q, total_k,
-        None if tables is None else tables.data_ptr(), 0 if tables is None else tables.stride(0),
-        0 if tables is None else tables.shape[1], page_size, num_pages, flags.data_ptr(),
-        stream_handle(cu_q.device)))
+CHECK_WORDS, CHECK_ODD, CHECK_OUTSIDE = 64, 1, 2
+
+
+def check_wait(verdicts, device):
+    """The bits that a checked prefill found, launched on the current stream of ``device``."""
+    found = _i32(0)
+    check(lib().pd_check_wait(verdicts.data_ptr(), stream_handle(device), ctypes.byref(found)))
+    return found.value
 
 
 def add_rms_norm(x, y, weight, out, eps):

@@ -92,10 +92,10 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group
     ``group``: query heads per kv head of the layer (None: what the tensors have); tensors
     with other head counts fail in the PyTorch form.
 
-    The metadata are checked on the device ahead of the attention, which reads nothing outside
-    its tensors whatever they hold, and the host waits for that check alone: what does not fit
-    the tensors is left to the PyTorch form, which fails on it, and pages outside the cache
-    raise.  A captured call has no such check: there such rows read as zeros.
+    The metadata are checked on the device as the attention starts, which reads nothing
+    outside its tensors whatever they hold, and the host waits for that check alone: what does
+    not fit the tensors is left to the PyTorch form, which fails on it, and pages outside the
+    cache raise.  A captured call has no such check: there such rows read as zeros.
     """
     out = torch.empty_like(q)
     if group is None:
@@ -111,24 +111,19 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group
         return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     page_size, num_pages = (k.shape[1], k.shape[0]) if tables is not None else (0, 0)
     total_k = 0 if tables is not None else k.shape[0]
-    if not capturing:
-        flags = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-        _native.check_packed(cu_q, cu_k, seqs, n, total_k, tables, page_size, num_pages, flags)
-        checked = torch.cuda.Event()
-        checked.record(torch.cuda.current_stream(q.device))
     splits = _splits((n * (hq // hkv) // _rows(d) + seqs) * hkv, max_keys, d, q.device)
     part_o, part_ml = _workspace(splits, n, hq, d, q.device)
     rows = lambda t: (t.stride(0) if t.dim() == 4 else 0, t.stride(-3), t.stride(-2))  # noqa: E731
+    verdicts = None if capturing else torch.zeros(_native.CHECK_WORDS, dtype=torch.int32,
+                                                  pin_memory=True)
     _native.prefill(q, rows(q), k, rows(k), v, rows(v), out, rows(out), cu_q, cu_k, seqs, 0, n,
                     total_k, tables, page_size, num_pages, hq, hkv, d, float(scale), splits, part_o,
-                    part_ml)
-    if not capturing:
-        checked.synchronize()
-        odd, outside = flags.tolist()
-        if outside:
-            raise IndexError("a sequence reaches past its block table or to a page outside the cache")
-        if odd:
-            return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
+                    part_ml, verdicts)
+    found = 0 if capturing else _native.check_wait(verdicts, q.device)
+    if found & _native.CHECK_OUTSIDE:
+        raise IndexError("a sequence reaches past its block table or to a page outside the cache")
+    if found & _native.CHECK_ODD:
+        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
     return out
 
 
