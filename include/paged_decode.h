@@ -307,9 +307,10 @@ int pd_prefill(const void* q, const int64_t* q_strides, const void* k, const int
                float* part_o, float* part_ml, pd_stream_t stream);
 
 /* pd_prefill of packed or paged sequences whose metadata are checked on the
- * device.  verdicts: int32 [PD_CHECK_WORDS] of pinned host memory, zeroed by the
- * caller and kept until pd_check_wait returns, which waits for the check, not
- * for the attention, and gives what was found:
+ * device, and pd_store_kv (above) that checks them for the pd_prefill behind it.
+ * verdicts: int32 [PD_CHECK_WORDS] of pinned host memory, zeroed by the caller
+ * and kept until pd_check_wait returns, which waits for the check, not for the
+ * kernel, and gives what was found:
  *   PD_CHECK_ODD      sequences are not rows of the tensors in order, or one of
  *                     new tokens has no keys or a page in [-num_pages, -1];
  *   PD_CHECK_OUTSIDE  a sequence has more keys than its table's entries hold,
@@ -325,6 +326,13 @@ int pd_prefill_checked(const void* q, const int64_t* q_strides, const void* k,
                        int32_t page_size, int64_t num_pages, int32_t num_heads,
                        int32_t num_kv_heads, int32_t head_dim, double scale, int32_t splits,
                        float* part_o, float* part_ml, int32_t* verdicts, pd_stream_t stream);
+int pd_store_kv_checked(const void* key, int64_t key_stride, const void* value,
+                        int64_t value_stride, void* k_cache, void* v_cache,
+                        const int32_t* slot_mapping, int64_t num_tokens, int32_t row_elems,
+                        const int32_t* cu_q, const int32_t* cu_k, int32_t num_seqs, int64_t total_q,
+                        int64_t total_k, const int32_t* table, int64_t table_stride_b,
+                        int32_t table_width, int32_t page_size, int64_t num_pages,
+                        int32_t* verdicts, pd_stream_t stream);
 int pd_check_wait(const int32_t* verdicts, pd_stream_t stream, int32_t* found);
 
 /* The decoder layer between its matrix products.  bf16 tensors are contiguous

@@ -12,6 +12,7 @@
 
 #include <cstdint>
 
+#include "pd_check.h"
 #include "pd_internal.h"
 #include "pd_launch.h"
 
@@ -26,13 +27,24 @@ constexpr int kThreads = 256;
 
 // One 16-byte piece per thread: row = piece / kPieces, chunk = piece % kPieces.
 // src rows are `src_stride` elements apart; dst row r goes to slot slots[r]
-// (row_elems elements per slot).  A negative slot skips the row.
+// (row_elems elements per slot).  A negative slot skips the row.  kCheck: the
+// metadata of the prefill behind it are checked on the way, so that the host,
+// which prepares that launch meanwhile, does not wait for them.
+template <bool kCheck>
 __global__ void __launch_bounds__(kThreads)
 store_slots_kernel(const uint16_t* __restrict__ key, int64_t key_stride,
                    const uint16_t* __restrict__ value, int64_t value_stride,
                    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
                    const int32_t* __restrict__ slots, int64_t rows, int pieces_per_row,
-                   int64_t row_elems) {
+                   int64_t row_elems, const pdk::PackedCheck check) {
+  if constexpr (kCheck) {
+    if (pdk::has_share(check.verdicts)) {
+      if (check.table)
+        pdk::check_packed<true>(check, threadIdx.x);
+      else
+        pdk::check_packed<false>(check, threadIdx.x);
+    }
+  }
   const int64_t piece = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   if (piece >= rows * pieces_per_row) return;
   const int64_t r = piece / pieces_per_row;
@@ -81,13 +93,17 @@ store_pages_kernel(const uint16_t* __restrict__ key, int64_t ksb, int64_t ksh, i
 
 }  // namespace
 
-extern "C" int pd_store_kv(const void* key, int64_t key_stride, const void* value,
-                           int64_t value_stride, void* k_cache, void* v_cache,
-                           const int32_t* slot_mapping, int64_t num_tokens, int32_t row_elems,
-                           pd_stream_t stream) {
+namespace {
+
+int store_slots(const void* key, int64_t key_stride, const void* value, int64_t value_stride,
+                void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_tokens,
+                int32_t row_elems, const pdk::PackedCheck& check, pd_stream_t stream) {
   pd::clear_error();
   if (num_tokens < 0) return pd::fail(PD_EINVAL, "num_tokens must be non-negative");
-  if (num_tokens == 0) return PD_OK;
+  if (num_tokens == 0) {
+    pdk::mark_absent(check.verdicts, 0);
+    return PD_OK;
+  }
   if (!key || !value || !k_cache || !v_cache || !slot_mapping)
     return pd::fail(PD_EINVAL, "null tensor pointer");
   if (row_elems <= 0 || row_elems % 8)
@@ -101,12 +117,41 @@ extern "C" int pd_store_kv(const void* key, int64_t key_stride, const void* valu
   const int64_t total = num_tokens * pieces;
   const int64_t blocks = (total + kThreads - 1) / kThreads;
   if (blocks > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
-  hipLaunchKernelGGL(store_slots_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0,
-                     reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(key),
-                     key_stride, static_cast<const uint16_t*>(value), value_stride,
+  pdk::mark_absent(check.verdicts, blocks);
+  hipLaunchKernelGGL(check.verdicts ? store_slots_kernel<true> : store_slots_kernel<false>,
+                     dim3(unsigned(blocks)), dim3(kThreads), 0, pd::as_stream(stream),
+                     static_cast<const uint16_t*>(key), key_stride,
+                     static_cast<const uint16_t*>(value), value_stride,
                      static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache),
-                     slot_mapping, num_tokens, pieces, int64_t(row_elems));
+                     slot_mapping, num_tokens, pieces, int64_t(row_elems), check);
   return launch_status("pd_store_kv");
+}
+
+}  // namespace
+
+extern "C" int pd_store_kv(const void* key, int64_t key_stride, const void* value,
+                           int64_t value_stride, void* k_cache, void* v_cache,
+                           const int32_t* slot_mapping, int64_t num_tokens, int32_t row_elems,
+                           pd_stream_t stream) {
+  return store_slots(key, key_stride, value, value_stride, k_cache, v_cache, slot_mapping,
+                     num_tokens, row_elems, pdk::PackedCheck{}, stream);
+}
+
+extern "C" int pd_store_kv_checked(const void* key, int64_t key_stride, const void* value,
+                                   int64_t value_stride, void* k_cache, void* v_cache,
+                                   const int32_t* slot_mapping, int64_t num_tokens,
+                                   int32_t row_elems, const int32_t* cu_q, const int32_t* cu_k,
+                                   int32_t num_seqs, int64_t total_q, int64_t total_k,
+                                   const int32_t* table, int64_t table_stride_b,
+                                   int32_t table_width, int32_t page_size, int64_t num_pages,
+                                   int32_t* verdicts, pd_stream_t stream) {
+  pd::clear_error();
+  if (num_seqs < 1 || !cu_q || !cu_k || !verdicts || (table && (table_width < 1 || page_size < 1)))
+    return pd::fail(PD_EINVAL, "a check needs sequences, their lengths, pages and verdicts");
+  const pdk::PackedCheck check{cu_q, cu_k, table, total_q, total_k, num_pages, table_stride_b,
+                               num_seqs, table_width, page_size, verdicts};
+  return store_slots(key, key_stride, value, value_stride, k_cache, v_cache, slot_mapping,
+                     num_tokens, row_elems, check, stream);
 }
 
 extern "C" int pd_store_kv_pages(const void* key, int64_t key_stride_b, int64_t key_stride_h,

@@ -52,11 +52,11 @@
 // prefill_merge_kernel combines.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
 
+#include "pd_check.h"
 #include "pd_device.h"
 #include "pd_internal.h"
 #include "pd_launch.h"
@@ -77,7 +77,7 @@ struct PrefillArgs {
   int64_t total_q, total_k, num_pages;
   int num_seqs, seq_len, table_width, page_size, num_kv_heads, G, splits;
   float scale;
-  int32_t* verdicts;        // of the packed metadata, or null
+  int32_t* verdicts;  // of the packed metadata, or null
 };
 
 template <int D>
@@ -158,45 +158,6 @@ __device__ __forceinline__ bool find_tile(const PrefillArgs& a, int t, int lane,
   return false;
 }
 
-// What the caller must know of packed metadata, which only the device holds.
-// The first workgroups look at a share of them before their tile, and each
-// wavefront writes kChecked and the bits it found to its word of pinned memory,
-// which the host polls while the attention runs.  A call of 5 rows takes 15 us
-// unchecked and 20 so; 27 with a kernel and an event of the check's own, which
-// also cost the stream 3 to 5 us a call, 22 with a kernel and the poll.
-constexpr int kChecked = 4, kCheckGroups = PD_CHECK_WORDS / 4;
-
-template <bool kPaged>
-__device__ __forceinline__ void check_packed(const PrefillArgs& a, int tid) {
-  const int width = kPaged ? a.table_width : 1;
-  const int64_t total = int64_t(a.num_seqs) * width;
-  const int step = min(int(gridDim.x), kCheckGroups) * 256;
-  bool odd = false, outside = false;
-  for (int64_t at = blockIdx.x * 256 + tid; at < total; at += step) {
-    const int64_t i = at / width;
-    const int entry = int(at - i * width);
-    const int64_t k0 = a.cu_k[i], k1 = a.cu_k[i + 1], nk = k1 - k0;
-    if (entry == 0) {
-      const int64_t q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
-      odd |= q0 < 0 || q1 < q0 || q1 > a.total_q || nk < 0 || (nk == 0 && q1 > q0);
-      if (kPaged)
-        outside |= nk > int64_t(width) * a.page_size;
-      else
-        odd |= k0 < 0 || k1 > a.total_k;
-    }
-    if (kPaged && int64_t(entry) * a.page_size < nk) {
-      const int64_t page = a.table[i * a.tsb + entry];
-      odd |= page < 0;
-      outside |= page >= a.num_pages || page < -a.num_pages;
-    }
-  }
-  const int found =
-      kChecked | (__any(odd) ? PD_CHECK_ODD : 0) | (__any(outside) ? PD_CHECK_OUTSIDE : 0);
-  if ((tid & 63) == 0)
-    __hip_atomic_store(a.verdicts + 4 * blockIdx.x + (tid >> 6), found, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // kPaged: K and V are pages read through the table, page_size a multiple of
 // the tile; else rows of the call's own tensors.
 template <int D, bool kPaged>
@@ -210,7 +171,7 @@ __global__ void __launch_bounds__(256, 2) prefill_kernel(const PrefillArgs a) {
   const int w = wave % (kRows / 32), part = wave / (kRows / 32);  // rows 32 w, columns of `part`
   const int half = lane >> 5, col = lane & 31;
 
-  if (a.verdicts && blockIdx.x < kCheckGroups && blockIdx.y == 0) check_packed<kPaged>(a, tid);
+  if (has_share(a.verdicts)) check_packed<kPaged>(a, tid);
 
   // Longest first: tiles are counted from the last, whose rows see most keys.
   const int id = blockIdx.x;
@@ -627,7 +588,7 @@ int run_prefill(const void* q, const int64_t* q_strides, const void* k, const in
     return pd::fail(PD_EINVAL, "token counts must lie in [0, 2^31)");
   if (verdicts && !cu_q) return pd::fail(PD_EINVAL, "only packed metadata are checked");
   if (total_q == 0) {
-    for (int word = 0; verdicts && word < PD_CHECK_WORDS; ++word) verdicts[word] = kChecked;
+    mark_absent(verdicts, 0);
     return PD_OK;
   }
   if (!q || !k || !v || !out || !q_strides || !k_strides || !v_strides || !out_strides)
@@ -694,8 +655,7 @@ int run_prefill(const void* q, const int64_t* q_strides, const void* k, const in
   const int64_t grid = tiles * num_kv_heads;
   if (grid > 0x7fffffff) return pd::fail(PD_EINVAL, "grid dimension exceeds device limits");
   a.verdicts = verdicts;
-  for (int word = 4 * int(std::min<int64_t>(grid, kCheckGroups)); verdicts && word < PD_CHECK_WORDS; ++word)
-    verdicts[word] = kChecked;  // workgroups that there are not
+  mark_absent(verdicts, grid);
   const hipStream_t st = as_stream(stream);
   if (head_dim == 64)
     launch<64>(a, unsigned(grid), st);

@@ -10,7 +10,7 @@ ModelRunner.prepare_prefill / prepare_decode set, engine/model_runner.py:136-195
 * a decode step calls ``paged_decode`` on the layer's cache with the engine's block
   tables (-1 padded in eager mode) and context lengths, using the ``decode_backend`` and
   ``decode_resources`` that ``integration.configure_model`` attached;
-* prefill runs causal attention over the packed sequences (``packed_prefill``, a HIP
+* prefill runs causal attention over the packed sequences (``PackedPrefill``, a HIP
   kernel in the place of the overlay's flash-attn varlen call), reading the cache through
   the block tables when a prefix is cached.
 
@@ -22,8 +22,8 @@ from dataclasses import dataclass
 import torch
 from torch import nn
 
-from .kv_write import store_kvcache
-from .prefill import packed_prefill
+from .kv_write import _store, store_kvcache
+from .prefill import PackedPrefill
 from .runtime import paged_decode
 
 
@@ -136,10 +136,11 @@ class Attention(nn.Module):
         """q [N, Hq, D], k/v [N, Hkv, D] of this step's tokens; returns [N, Hq, D] for a
         prefill and [B, 1, Hq, D] for a decode step (the overlay's shapes)."""
         context = get_context()
-        if self.k_cache.numel() and self.v_cache.numel():
-            store_kvcache(k, v, self.k_cache, self.v_cache, context.slot_mapping)
+        cached = self.k_cache.numel() and self.v_cache.numel()
         if context.is_prefill:
-            return self._prefill(q, k, v, context)
+            return self._prefill(q, k, v, context, cached)
+        if cached:
+            store_kvcache(k, v, self.k_cache, self.v_cache, context.slot_mapping)
         if self.decode_backend == "flash_attn":
             raise NotImplementedError("flash-attn decode is not available on this GPU; "
                                       "configure_model with a custom decode_backend")
@@ -147,9 +148,14 @@ class Attention(nn.Module):
                             context.context_lens, resources=self.decode_resources,
                             backend=self.decode_backend, scale=self.scale).unsqueeze(1)
 
-    def _prefill(self, q, k, v, context):
-        if context.block_tables is not None:  # prefix cache: the whole context is paged
-            k, v = self.k_cache, self.v_cache
-        return packed_prefill(q, k, v, context.cu_seqlens_q, context.cu_seqlens_k, self.scale,
-                              tables=context.block_tables, max_keys=context.max_seqlen_k,
-                              group=self.num_heads // self.num_kv_heads)
+    def _prefill(self, q, k, v, context, cached):
+        # prefix cache: the whole context is paged
+        keys, values = (k, v) if context.block_tables is None else (self.k_cache, self.v_cache)
+        call = PackedPrefill(q, keys, values, context.cu_seqlens_q, context.cu_seqlens_k, self.scale,
+                             context.block_tables, context.max_seqlen_k,
+                             self.num_heads // self.num_kv_heads)
+        if not cached:
+            return call.run()
+        check = call.check if k.shape[0] else None      # a write of no rows is not launched
+        _store(k, v, self.k_cache, self.v_cache, context.slot_mapping, check)
+        return call.run(checking=check is not None)

@@ -24,6 +24,11 @@ def store_kvcache(key, value, k_cache, v_cache, slot_mapping):
     caches: [blocks, block_size, Hkv, D] bf16 with stride(1) == Hkv*D;
     slot_mapping: int32 [N] on the same device.
     """
+    _store(key, value, k_cache, v_cache, slot_mapping)
+
+
+def _store(key, value, k_cache, v_cache, slot_mapping, metadata=None):
+    """store_kvcache, with the metadata that _native.store_kv checks on the way."""
     _require(key.dim() == 3 and value.shape == key.shape, "key/value must be [N, kv_heads, head_dim]")
     n, hkv, d = key.shape
     _require(key.stride(-1) == 1 and value.stride(-1) == 1, "key/value last dim must be contiguous")
@@ -38,7 +43,7 @@ def store_kvcache(key, value, k_cache, v_cache, slot_mapping):
     _require(key.is_cuda and all(t.device == key.device
                                  for t in (value, k_cache, v_cache, slot_mapping)),
              "all tensors must be on one CUDA device")
-    _native.store_kv(key, value, k_cache, v_cache, slot_mapping)
+    _native.store_kv(key, value, k_cache, v_cache, slot_mapping, metadata)
 
 
 def write_pages(key, value, k_pages, v_pages, tables, positions):

@@ -97,34 +97,60 @@ def packed_prefill(q, k, v, cu_q, cu_k, scale, *, tables=None, max_keys=0, group
     not fit the tensors is left to the PyTorch form, which fails on it, and pages outside the
     cache raise.  A captured call has no such check: there such rows read as zeros.
     """
-    out = torch.empty_like(q)
-    if group is None:
-        group = q.shape[1] // k.shape[-2]
-    if not _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables) or q.shape[1] != group * k.shape[-2]:
-        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
-    n, hq, d = q.shape
-    hkv, seqs = k.shape[-2], cu_q.shape[0] - 1
-    capturing = torch.cuda.is_current_stream_capturing()
-    if seqs < 1 or (n == 0 and capturing):
-        return out
-    if n == 0:
-        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
-    page_size, num_pages = (k.shape[1], k.shape[0]) if tables is not None else (0, 0)
-    total_k = 0 if tables is not None else k.shape[0]
-    splits = _splits((n * (hq // hkv) // _rows(d) + seqs) * hkv, max_keys, d, q.device)
-    part_o, part_ml = _workspace(splits, n, hq, d, q.device)
-    rows = lambda t: (t.stride(0) if t.dim() == 4 else 0, t.stride(-3), t.stride(-2))  # noqa: E731
-    verdicts = None if capturing else torch.zeros(_native.CHECK_WORDS, dtype=torch.int32,
-                                                  pin_memory=True)
-    _native.prefill(q, rows(q), k, rows(k), v, rows(v), out, rows(out), cu_q, cu_k, seqs, 0, n,
-                    total_k, tables, page_size, num_pages, hq, hkv, d, float(scale), splits, part_o,
-                    part_ml, verdicts)
-    found = 0 if capturing else _native.check_wait(verdicts, q.device)
-    if found & _native.CHECK_OUTSIDE:
-        raise IndexError("a sequence reaches past its block table or to a page outside the cache")
-    if found & _native.CHECK_ODD:
-        return _packed_torch(q, k, v, cu_q, cu_k, scale, tables, out, group)
-    return out
+    return PackedPrefill(q, k, v, cu_q, cu_k, scale, tables, max_keys, group).run()
+
+
+class PackedPrefill:
+    """One packed_prefill call, so that the K/V write ahead of it can check its metadata:
+    ``check`` is what that launch takes (None: nothing for it to check), then ``run``."""
+
+    def __init__(self, q, k, v, cu_q, cu_k, scale, tables=None, max_keys=0, group=None):
+        self.call = q, k, v, cu_q, cu_k, scale, tables
+        self.max_keys = max_keys
+        self.out = torch.empty_like(q)
+        self.group = q.shape[1] // k.shape[-2] if group is None else group
+        self.kernel = (_packed_ok(q, k, v, self.out, cu_q, cu_k, scale, tables)
+                       and q.shape[1] == self.group * k.shape[-2])
+        self.check = None
+        if (self.kernel and q.shape[0] and cu_q.shape[0] > 1
+                and not torch.cuda.is_current_stream_capturing()):
+            page_size, num_pages = (k.shape[1], k.shape[0]) if tables is not None else (0, 0)
+            self.check = (cu_q, cu_k, cu_q.shape[0] - 1, q.shape[0],
+                          0 if tables is not None else k.shape[0], tables, page_size, num_pages,
+                          torch.zeros(_native.CHECK_WORDS, dtype=torch.int32, pin_memory=True))
+
+    def run(self, checking=False):
+        """The attention; ``checking``: a launch with ``check`` is under way."""
+        q, k, v, cu_q, cu_k, scale, tables = self.call
+        if not self.kernel:
+            return self._general()
+        n, hq, d = q.shape
+        hkv, seqs = k.shape[-2], cu_q.shape[0] - 1
+        if self.check is None:
+            if seqs < 1 or n == 0:
+                empty = seqs < 1 or torch.cuda.is_current_stream_capturing()
+                return self.out if empty else self._general()
+            verdicts = None
+        else:
+            verdicts = self.check[-1]
+        try:
+            splits = _splits((n * (hq // hkv) // _rows(d) + seqs) * hkv, self.max_keys, d, q.device)
+            part_o, part_ml = _workspace(splits, n, hq, d, q.device)
+            rows = lambda t: (t.stride(0) if t.dim() == 4 else 0, t.stride(-3), t.stride(-2))  # noqa: E731
+            paged = tables is not None
+            _native.prefill(q, rows(q), k, rows(k), v, rows(v), self.out, rows(self.out), cu_q, cu_k,
+                            seqs, 0, n, 0 if paged else k.shape[0], tables,
+                            k.shape[1] if paged else 0, k.shape[0] if paged else 0, hq, hkv, d,
+                            float(scale), splits, part_o, part_ml, None if checking else verdicts)
+            checking = verdicts is not None
+        finally:        # until it has been waited for, a check writes to ``verdicts``
+            found = _native.check_wait(verdicts, q.device) if checking else 0
+        if found & _native.CHECK_OUTSIDE:
+            raise IndexError("a sequence reaches past its block table or to a page outside the cache")
+        return self._general() if found & _native.CHECK_ODD else self.out
+
+    def _general(self):
+        return _packed_torch(*self.call, self.out, self.group)
 
 
 def _packed_ok(q, k, v, out, cu_q, cu_k, scale, tables):

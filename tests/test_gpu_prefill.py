@@ -11,6 +11,7 @@ if not torch.cuda.is_available():
     pytest.skip("needs an MI355X GPU", allow_module_level=True)
 
 from paged_decode import prefill as PF
+from paged_decode.engine_attention import Attention, reset_context, set_context
 
 pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -24
@@ -292,3 +293,53 @@ def test_later_tokens_never_reach_earlier_rows(monkeypatch, d, page, splits, spe
             assert torch.equal(got[want.isinf()], want[want.isinf()]), (t, h)
             ok = want.isfinite()
             assert not ok.any() or (got[ok] - want[ok]).abs().max() < 2.0 ** -6, (t, h)
+
+
+@pytest.mark.parametrize("prefix", [0, 96])
+@pytest.mark.parametrize("fault", [None, "q_end", "k_order", "page", "width", "wrapped"])
+def test_layers_check_the_metadata_with_the_write(prefix, fault):
+    """The engine's layer: what does not fit fails as in packed_prefill, the rows are written
+    first, and the next call is a plain one."""
+    page, d, lens = 32, 256, (40, 1, 300)
+    q, k, v, cu_q, cu_k, table = metadata(d, page, lens, prefix)
+    if not prefix and fault in ("page", "width", "wrapped"):
+        pytest.skip("no pages to read")
+    layer = Attention(4, d, 0.1, 2)
+    layer.k_cache, layer.v_cache = k, v
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    key, value = rows(gen, sum(lens), 2, d), rows(gen, sum(lens), 2, d)
+    slots = torch.cat([torch.tensor([table[i][t // page] * page + t % page
+                                     for t in range(prefix, prefix + n)]) for i, n in enumerate(lens)])
+    if not prefix:
+        cu_k = list(cu_q)
+    good = list(cu_q), list(cu_k), [list(t) for t in table]
+    if fault == "q_end":
+        cu_q[-1] += 1
+    elif fault == "k_order":
+        cu_k[2:] = [n - (cu_k[2] - cu_k[1] + 2) for n in cu_k[2:]]
+    elif fault == "page":
+        table[2][0] = k.shape[0]
+    elif fault == "width":
+        cu_k[-1] += page
+    elif fault == "wrapped":
+        table[2][0] -= k.shape[0]
+    device = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+
+    def run(cu_q, cu_k, table):
+        set_context(True, device(cu_q), device(cu_k), 300, 500, slots.int().cuda(),
+                    block_tables=device(table) if prefix else None)
+        try:
+            return layer(q, key, value)
+        finally:
+            reset_context()
+
+    want = run(*good)
+    flat = k.view(-1, 2, d)
+    flat[slots.cuda()] = 0
+    if fault in (None, "wrapped"):
+        assert (run(cu_q, cu_k, table) - want).abs().max() < 2.0 ** -6
+    else:
+        with pytest.raises(IndexError if fault in ("page", "width") else RuntimeError):
+            run(cu_q, cu_k, table)
+    assert torch.equal(flat[slots.cuda()], key)
+    assert torch.equal(run(*good), want)
