@@ -82,9 +82,8 @@ def _as_installed():
 
 def _plain_module(module, kind):
     """`module` runs the forward its class defines and nothing else."""
-    own = module.__dict__
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
-            and "forward" not in own and "_norm" not in own and module._compiled_call_impl is None
+            and "forward" not in module.__dict__ and module._compiled_call_impl is None
             and not module.training)
 
 
@@ -124,6 +123,7 @@ class _Reader:
         if not self.ok:
             return None, 0.0
         if kind is Qwen3_5RMSNorm:
+            self.ok = "_norm" not in module.__dict__
             return self.weight(module, (dim,)), float(module.eps)
         self.ok = module.__dict__.get("activation", "silu") == "silu"
         return self.weight(module, (dim,)), float(module.variance_epsilon)
