@@ -247,22 +247,25 @@ def chunk_rows(max_batch, num_heads, num_kv_heads, head_dim, sm_count):
     return rows.value
 
 
-def store_kv(key, value, k_cache, v_cache, slot_mapping, metadata=None):
-    """key/value [N, Hkv, D] (rows 16-byte aligned); caches [..., Hkv, D] flat over slots.
-    ``metadata``: (cu_q, cu_k, sequences, total_q, total_k, tables or None, page_size,
-    num_pages, verdicts) of the packed prefill behind the write, checked with it."""
+def store_kv(key, value, k_cache, v_cache, slot_mapping):
+    """key/value [N, Hkv, D] (rows 16-byte aligned); caches [..., Hkv, D] flat over slots."""
     n, hkv, d = key.shape
-    args = (key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), k_cache.data_ptr(),
-            v_cache.data_ptr(), slot_mapping.data_ptr(), n, hkv * d)
-    if metadata is None:
-        check(lib().pd_store_kv(*args, stream_handle(key.device)))
-        return
+    check(lib().pd_store_kv(key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0),
+                            k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(), n,
+                            hkv * d, stream_handle(key.device)))
+
+
+def store_kv_checked(key, value, k_cache, v_cache, slot_mapping, metadata):
+    """store_kv that checks the packed prefill behind it: ``metadata`` is its (cu_q, cu_k,
+    sequences, total_q, total_k, tables or None, page_size, num_pages, verdicts)."""
+    n, hkv, d = key.shape
     cu_q, cu_k, seqs, total_q, total_k, tables, page_size, num_pages, verdicts = metadata
     check(lib().pd_store_kv_checked(
-        *args, cu_q.data_ptr(), cu_k.data_ptr(), seqs, total_q, total_k,
-        None if tables is None else tables.data_ptr(), 0 if tables is None else tables.stride(0),
-        0 if tables is None else tables.shape[1], page_size, num_pages, verdicts.data_ptr(),
-        stream_handle(key.device)))
+        key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0), k_cache.data_ptr(),
+        v_cache.data_ptr(), slot_mapping.data_ptr(), n, hkv * d, cu_q.data_ptr(), cu_k.data_ptr(),
+        seqs, total_q, total_k, None if tables is None else tables.data_ptr(),
+        0 if tables is None else tables.stride(0), 0 if tables is None else tables.shape[1],
+        page_size, num_pages, verdicts.data_ptr(), stream_handle(key.device)))
 
 
 def store_kv_pages(key, value, k_pages, v_pages, tables, positions):

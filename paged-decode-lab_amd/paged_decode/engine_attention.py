@@ -22,7 +22,7 @@ from dataclasses import dataclass
 import torch
 from torch import nn
 
-from .kv_write import _store, store_kvcache
+from .kv_write import store_kvcache
 from .prefill import PackedPrefill
 from .runtime import paged_decode
 
@@ -157,5 +157,5 @@ class Attention(nn.Module):
         if not cached:
             return call.run()
         check = call.check if k.shape[0] else None      # a write of no rows is not launched
-        _store(k, v, self.k_cache, self.v_cache, context.slot_mapping, check)
+        store_kvcache(k, v, self.k_cache, self.v_cache, context.slot_mapping, _metadata=check)
         return call.run(checking=check is not None)

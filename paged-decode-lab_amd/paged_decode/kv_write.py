@@ -17,18 +17,14 @@ def _require(condition, message):
         raise ValueError(message)
 
 
-def store_kvcache(key, value, k_cache, v_cache, slot_mapping):
+def store_kvcache(key, value, k_cache, v_cache, slot_mapping, *, _metadata=None):
     """k_cache.view(-1, Hkv*D)[slot_mapping[i]] = key[i] (and V); slot -1 skips.
 
     key/value: [N, Hkv, D] bf16 with stride(-1) == 1 and stride(1) == D;
     caches: [blocks, block_size, Hkv, D] bf16 with stride(1) == Hkv*D;
     slot_mapping: int32 [N] on the same device.
+    _metadata: what _native.store_kv_checked checks on the way, for the engine's layer.
     """
-    _store(key, value, k_cache, v_cache, slot_mapping)
-
-
-def _store(key, value, k_cache, v_cache, slot_mapping, metadata=None):
-    """store_kvcache, with the metadata that _native.store_kv checks on the way."""
     _require(key.dim() == 3 and value.shape == key.shape, "key/value must be [N, kv_heads, head_dim]")
     n, hkv, d = key.shape
     _require(key.stride(-1) == 1 and value.stride(-1) == 1, "key/value last dim must be contiguous")
@@ -43,7 +39,10 @@ def _store(key, value, k_cache, v_cache, slot_mapping, metadata=None):
     _require(key.is_cuda and all(t.device == key.device
                                  for t in (value, k_cache, v_cache, slot_mapping)),
              "all tensors must be on one CUDA device")
-    _native.store_kv(key, value, k_cache, v_cache, slot_mapping, metadata)
+    if _metadata is not None:
+        _native.store_kv_checked(key, value, k_cache, v_cache, slot_mapping, _metadata)
+        return
+    _native.store_kv(key, value, k_cache, v_cache, slot_mapping)
 
 
 def write_pages(key, value, k_pages, v_pages, tables, positions):
